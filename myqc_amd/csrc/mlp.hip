@@ -42,12 +42,13 @@ struct MlpState {
     float *d_X = nullptr, *d_T = nullptr, *d_M = nullptr, *d_Z[3] = {nullptr, nullptr, nullptr},
           *d_H[3] = {nullptr, nullptr, nullptr}, *d_Y = nullptr, *d_dA = nullptr, *d_dB = nullptr,
           *d_loss = nullptr;
+    float *d_gpart = nullptr;   // weight gradients of each range of rows (mlp_backward)
     // per-atom environment features (kElem x kEnv each) of up to env_cap atoms
     float *d_env = nullptr;
     int env_cap = 0;
     void release() {
         float **ps[] = {&d_par, &d_grad, &d_m, &d_v, &d_X, &d_T, &d_M, &d_Z[0], &d_Z[1], &d_Z[2],
-                        &d_H[0], &d_H[1], &d_H[2], &d_Y, &d_dA, &d_dB, &d_loss, &d_env};
+                        &d_H[0], &d_H[1], &d_H[2], &d_Y, &d_dA, &d_dB, &d_loss, &d_env, &d_gpart};
         for (auto p : ps) dfree((void **)p);
         cap = 0;
         env_cap = 0;
@@ -67,76 +68,184 @@ void free_mlp(myqc_ctx *ctx) {
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + __expf(-z)); }
 
-// C[M x N] = op(A) op(B) (+ bias[j]); row-major.  op(A)(i,k) = TA ? A[k lda + i]
-// : A[i lda + k]; op(B)(k,j) = TB ? B[j ldb + k] : B[k ldb + j].  EPI 0: plain,
-// 1: Z = C + bias, H = silu(Z), 2: C + bias (linear output).  64 x 64 tiles,
-// each of 256 threads owning 4 x 4 outputs; K in steps of 16 through LDS.
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, const float *__restrict__ A, int lda,
-                                               const float *__restrict__ B, int ldb, const float *__restrict__ bias,
-                                               float *__restrict__ Z, float *__restrict__ C) {
-    __shared__ float As[16][68], Bs[16][68];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-    float acc[4][4];
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+// C[M x N] = op(A) op(B) in FP32 on the matrix cores; row-major.
+//   op(A)(i,k) = AK ? A[i lda + k] : A[k lda + i];   op(B)(k,j) = BK ? B[j ldb + k] : B[k ldb + j].
+// EPI 1: Z = C + bias, C = silu(Z); 2: C + bias (linear output); 3: C silu'(Z)
+// (the gradient through the layer below); 4: one k range per blockIdx.z, its
+// sums to C + blockIdx.z zstride and, from the first column of workgroups,
+// the column sums of A (M of them) to bsum + blockIdx.z zstride.
+//
+// What bounds it: the layers are 200 x 128 .. 128 x 16, so a product is a few
+// microseconds of matrix-core time and the cost is how many workgroups share
+// it.  Tiles of BT x BT by four wavefronts (2 x 2, v_mfma_f32_16x16x4f32,
+// twice the FP32 FMA rate without packed instructions); BT = 64 when that
+// gives every CU a workgroup, else 32.  The weight gradients contract over
+// the rows, so their k range is cut into ranges of at least 64 rows for
+// up to 64 workgroups per tile; k_fold_parts adds the ranges in a fixed
+// order.  One gradient of the 200-128-128-128-16 network at 8192 rows:
+// weight gradients 4.8 ms (8 workgroups, each over all rows) and bias column
+// sums 6.0 ms (one thread per column) before, 47 us together now.
+//
+// LDS: an operand with k contiguous in memory is kept [row][k] (36 floats a
+// row: the 16 rows a wavefront reads with 16-byte loads fall in distinct
+// banks), one with rows contiguous [k][row] (BT + 4 floats, likewise).  Both
+// are read so that lane group g supplies k = 4 g + j to the j-th product of
+// a 16-wide step.
+constexpr int MK = 32;
+template <int BT>
+constexpr int lds_floats(bool kmajor) { return kmajor ? BT * (MK + 4) : MK * (BT + 4); }
+
+// the thread's 16-byte pieces of one BT x MK slice of an operand: rows r0 ..,
+// k from k0 up to k1
+template <int BT, bool KM>
+__device__ __forceinline__ void mlp_fetch(const float *__restrict__ A, long long lda, int rows, int r0, int k0, int k1,
+                                          int vec, f4_t (&v)[BT / 32]) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int q = 0; q < BT / 32; ++q) {
+        const int c = threadIdx.x + 256 * q;
+        v[q] = (f4_t){0.f, 0.f, 0.f, 0.f};
+        if constexpr (KM) {
+            const int r = r0 + (c >> 3), k = k0 + (c & 7) * 4;
+            if (r >= rows) continue;
+            const float *src = A + r * lda + k;
+            if (vec && k + 4 <= k1) v[q] = *reinterpret_cast<const f4_t *>(src);
+            else
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.f;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-            const int kk = e & 15, r = e >> 4;
-            const int gi = i0 + r, gk = k0 + kk, gj = j0 + r;
-            As[kk][r] = (gi < M && gk < K) ? (TA ? A[(size_t)gk * lda + gi] : A[(size_t)gi * lda + gk]) : 0.f;
-            Bs[kk][r] = (gj < N && gk < K) ? (TB ? B[(size_t)gj * ldb + gk] : B[(size_t)gk * ldb + gj]) : 0.f;
+                for (int e = 0; e < 4; ++e)
+                    if (k + e < k1) v[q][e] = src[e];
+        } else {
+            const int k = k0 + c / (BT / 4), r = r0 + (c % (BT / 4)) * 4;
+            if (k >= k1) continue;
+            const float *src = A + k * lda + r;
+            if (vec && r + 4 <= rows) v[q] = *reinterpret_cast<const f4_t *>(src);
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (r + e < rows) v[q][e] = src[e];
+        }
+    }
+}
+
+template <int BT, bool KM>
+__device__ __forceinline__ void mlp_stage(float *sm, const f4_t (&v)[BT / 32]) {
+#pragma unroll
+    for (int q = 0; q < BT / 32; ++q) {
+        const int c = threadIdx.x + 256 * q;
+        float *dst = KM ? sm + (c >> 3) * (MK + 4) + (c & 7) * 4 : sm + c / (BT / 4) * (BT + 4) + (c % (BT / 4)) * 4;
+        *reinterpret_cast<f4_t *>(dst) = v[q];
+    }
+}
+
+// row r of the slice at k = kk + 4 g .. + 3
+template <int BT, bool KM>
+__device__ __forceinline__ f4_t mlp_frag(const float *sm, int r, int k) {
+    if constexpr (KM) return *reinterpret_cast<const f4_t *>(sm + r * (MK + 4) + k);
+    f4_t v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = sm[(k + j) * (BT + 4) + r];
+    return v;
+}
+
+template <int BT, bool AK, bool BK, int EPI>
+__global__ __launch_bounds__(256) void k_mlp_gemm(int M, int N, int K, int kchunk, const float *__restrict__ A, int lda,
+                                                  const float *__restrict__ B, int ldb, int vec,
+                                                  const float *__restrict__ bias, float *__restrict__ Z,
+                                                  float *__restrict__ C, float *__restrict__ bsum, long long zstride) {
+    constexpr int NT = BT / 32, WT = BT / 2;
+    __shared__ __attribute__((aligned(16))) float sA[2][lds_floats<BT>(AK)], sB[2][lds_floats<BT>(BK)];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r = lane & 15, g = lane >> 4;
+    const int wr = (w & 1) * WT, wc = (w >> 1) * WT;
+    const int i0 = blockIdx.y * BT, j0 = blockIdx.x * BT;
+    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
+    f4_t acc[NT][NT];
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+#pragma unroll
+        for (int y = 0; y < NT; ++y) acc[x][y] = (f4_t){0.f, 0.f, 0.f, 0.f};
+    f4_t va[NT], vb[NT], cs = (f4_t){0.f, 0.f, 0.f, 0.f};
+    mlp_fetch<BT, AK>(A, lda, M, i0, kb, ke, vec & 1, va);
+    mlp_fetch<BT, BK>(B, ldb, N, j0, kb, ke, vec & 2, vb);
+    int buf = 0;
+    for (int k0 = kb; k0 < ke; k0 += MK, buf ^= 1) {
+        mlp_stage<BT, AK>(sA[buf], va);
+        mlp_stage<BT, BK>(sB[buf], vb);
+        if constexpr (EPI == 4) {
+#pragma unroll
+            for (int q = 0; q < NT; ++q) cs += va[q];
         }
         __syncthreads();
+        if (k0 + MK < ke) {
+            mlp_fetch<BT, AK>(A, lda, M, i0, k0 + MK, ke, vec & 1, va);
+            mlp_fetch<BT, BK>(B, ldb, N, j0, k0 + MK, ke, vec & 2, vb);
+        }
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
+        for (int kk = 0; kk < MK; kk += 16) {
+            f4_t fa[NT], fb[NT];
+#pragma unroll
+            for (int x = 0; x < NT; ++x) fa[x] = mlp_frag<BT, AK>(sA[buf], wr + 16 * x + r, kk + 4 * g);
+#pragma unroll
+            for (int y = 0; y < NT; ++y) fb[y] = mlp_frag<BT, BK>(sB[buf], wc + 16 * y + r, kk + 4 * g);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int x = 0; x < NT; ++x)
+#pragma unroll
+                    for (int y = 0; y < NT; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[x][j], fb[y][j], acc[x][y], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+#pragma unroll
+        for (int y = 0; y < NT; ++y)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                a[q] = As[kk][ty * 4 + q];
-                b[q] = Bs[kk][tx * 4 + q];
+                const int gi = i0 + wr + 16 * x + 4 * g + q, gj = j0 + wc + 16 * y + r;
+                if (gi >= M || gj >= N) continue;
+                const size_t e = (size_t)gi * N + gj;
+                float v = acc[x][y][q];
+                if constexpr (EPI == 1 || EPI == 2) v += bias[gj];
+                if constexpr (EPI == 1) {
+                    Z[e] = v;
+                    v = v * sigm(v);
+                }
+                if constexpr (EPI == 3) {
+                    const float z = Z[e], s = sigm(z);
+                    v *= s * (1.0f + z * (1.0f - s));
+                }
+                if constexpr (EPI == 4) C[blockIdx.z * zstride + e] = v;
+                else C[e] = v;
             }
-#pragma unroll
-            for (int x = 0; x < 4; ++x)
-#pragma unroll
-                for (int y = 0; y < 4; ++y) acc[x][y] = fmaf(a[x], b[y], acc[x][y]);
-        }
+    if constexpr (EPI == 4) {
+        // column sums of A over this k range: thread t holds those of its
+        // four rows of op(A) over its share of the k's
+        if (blockIdx.x != 0) return;
+        constexpr int PER = BT / 4;
         __syncthreads();
-    }
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            const int gi = i0 + ty * 4 + x, gj = j0 + tx * 4 + y;
-            if (gi >= M || gj >= N) continue;
-            float v = acc[x][y];
-            if (EPI >= 1) v += bias[gj];
-            if (EPI == 1) {
-                Z[(size_t)gi * N + gj] = v;
-                v = v * sigm(v);
-            }
-            C[(size_t)gi * N + gj] = v;
+        f4_t *red = reinterpret_cast<f4_t *>(&sA[0][0]);
+        red[t] = cs;
+        __syncthreads();
+        if (t < BT && i0 + t < M) {
+            float v = 0.f;
+            for (int q = 0; q < 256 / PER; ++q) v += red[q * PER + (t >> 2)][t & 3];
+            bsum[blockIdx.z * zstride + i0 + t] = v;
         }
-}
-
-// dZ = dH * silu'(Z)
-__global__ void k_silu_grad(const float *__restrict__ Z, float *__restrict__ dH, long long cnt) {
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < cnt; e += (long long)gridDim.x * blockDim.x) {
-        const float z = Z[e], s = sigm(z);
-        dH[e] *= s * (1.0f + z * (1.0f - s));
     }
 }
 
-// db[j] = sum_i dZ[i][j]   (one thread per column; fixed order)
-__global__ void k_colsum(const float *__restrict__ dZ, int rows, int cols, float *__restrict__ db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) return;
-    float s = 0.f;
-    for (int i = 0; i < rows; ++i) s += dZ[(size_t)i * cols + j];
-    db[j] = s;
+// g[e] = sum over the np ranges of part[range cnt + e], in a fixed order
+__global__ void k_fold_parts(const float *__restrict__ part, int np, long long cnt, float *__restrict__ g) {
+    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= cnt) return;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    int p = 0;
+    for (; p + 4 <= np; p += 4)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] += part[(p + q) * cnt + e];
+    for (; p < np; ++p) s[0] += part[p * cnt + e];
+    g[e] = (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 // masked MSE: dY = 2 M (Y - T) / sum(M); per-block partial losses into part
@@ -196,11 +305,32 @@ static int mlp_ensure(myqc_ctx *ctx, MlpState &s, int rows) {
     return 0;
 }
 
-template <bool TA, bool TB, int EPI>
-static void sgemm(myqc_ctx *ctx, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
-                  const float *bias, float *Z, float *C) {
-    const dim3 grid((N + 63) / 64, (M + 63) / 64);
-    k_sgemm<TA, TB, EPI><<<grid, 256, 0, ctx->stream>>>(M, N, K, A, lda, B, ldb, bias, Z, C);
+// Rows per range of the weight gradients: at least 64, in at most kMlpRanges
+// ranges, whose partial sums (n_par each) together take at most 64 MiB (a
+// network that large has tiles enough without ranges)
+constexpr int kMlpRanges = 64;
+constexpr long long kMlpPartFloats = 16LL << 20;
+static int mlp_kchunk(int rows, long long n_par) {
+    const int most = (int)std::max(1LL, std::min<long long>(kMlpRanges, kMlpPartFloats / n_par));
+    const int c = std::max(64, (rows + most - 1) / most);
+    return ((c + MK - 1) / MK) * MK;
+}
+
+template <bool AK, bool BK, int EPI>
+static void mlp_gemm(myqc_ctx *ctx, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
+                     const float *bias, float *Z, float *C, float *bsum = nullptr, long long zstride = 0) {
+    const int kchunk = EPI == 4 ? mlp_kchunk(K, zstride) : K;
+    const unsigned nz = (unsigned)((K + kchunk - 1) / kchunk);
+    // 16-byte loads where rows start on 16-byte boundaries
+    auto ok = [](const float *p, int ld) { return (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const int vec = (ok(A, lda) ? 1 : 0) | (ok(B, ldb) ? 2 : 0);
+    const long long big = (long long)((N + 63) / 64) * ((M + 63) / 64) * nz;
+    if (big >= 256)
+        k_mlp_gemm<64, AK, BK, EPI><<<dim3((N + 63) / 64, (M + 63) / 64, nz), 256, 0, ctx->stream>>>(
+            M, N, K, kchunk, A, lda, B, ldb, vec, bias, Z, C, bsum, zstride);
+    else
+        k_mlp_gemm<32, AK, BK, EPI><<<dim3((N + 31) / 32, (M + 31) / 32, nz), 256, 0, ctx->stream>>>(
+            M, N, K, kchunk, A, lda, B, ldb, vec, bias, Z, C, bsum, zstride);
 }
 
 // Y = net(X) for `rows` rows in s.d_X (keeps Z, H for the backward pass)
@@ -209,13 +339,13 @@ static void mlp_forward(myqc_ctx *ctx, MlpState &s, int rows) {
     const float *in = s.d_X;
     int k = s.n_in;
     for (int l = 0; l < 3; ++l) {
-        sgemm<false, true, 1>(ctx, rows, s.width, k, in, k, P + s.off[2 * l], k, P + s.off[2 * l + 1], s.d_Z[l],
-                              s.d_H[l]);
+        mlp_gemm<true, true, 1>(ctx, rows, s.width, k, in, k, P + s.off[2 * l], k, P + s.off[2 * l + 1], s.d_Z[l],
+                                s.d_H[l]);
         in = s.d_H[l];
         k = s.width;
     }
-    sgemm<false, true, 2>(ctx, rows, s.n_out, s.width, in, s.width, P + s.off[6], s.width, P + s.off[7], nullptr,
-                          s.d_Y);
+    mlp_gemm<true, true, 2>(ctx, rows, s.n_out, s.width, in, s.width, P + s.off[6], s.width, P + s.off[7], nullptr,
+                            s.d_Y);
 }
 
 // gradient of the masked MSE into s.d_grad; loss partials in s.d_loss
@@ -223,25 +353,27 @@ static int mlp_backward(myqc_ctx *ctx, MlpState &s, int rows, float inv_w, int *
     const long long cnt = (long long)rows * s.n_out;
     const int blocks = (int)std::min<long long>(1024, (cnt + 255) / 256);
     *nblk = blocks;
+    const int kchunk = mlp_kchunk(rows, s.n_par), np = (rows + kchunk - 1) / kchunk;
+    MYQC_CHECK(dalloc(ctx, (void **)&s.d_gpart, sizeof(float) * (size_t)np * s.n_par));
     k_mse<<<blocks, 256, 0, ctx->stream>>>(s.d_Y, s.d_T, s.d_M, cnt, inv_w, s.d_dA, s.d_loss);
-    float *G = s.d_grad;
+    float *G = s.d_gpart;   // per k range, laid out as the parameters
     const float *P = s.d_par;
-    // output layer: dW4 = dY^T H3, db4 = colsum dY, dH3 = dY W4
+    // output layer: dW4 = dY^T H3, db4 = column sums of dY, dH3 = dY W4
     float *dcur = s.d_dA, *dnext = s.d_dB;
     int width_out = s.n_out;
     for (int l = 3; l >= 0; --l) {
         const float *in = l == 0 ? s.d_X : s.d_H[l - 1];
         const int k = l == 0 ? s.n_in : s.width;
-        sgemm<true, false, 0>(ctx, width_out, k, rows, dcur, width_out, in, k, nullptr, nullptr, G + s.off[2 * l]);
-        k_colsum<<<(width_out + 127) / 128, 128, 0, ctx->stream>>>(dcur, rows, width_out, G + s.off[2 * l + 1]);
+        mlp_gemm<false, false, 4>(ctx, width_out, k, rows, dcur, width_out, in, k, nullptr, nullptr,
+                                  G + s.off[2 * l], G + s.off[2 * l + 1], s.n_par);
         if (l > 0) {
-            sgemm<false, false, 0>(ctx, rows, k, width_out, dcur, width_out, P + s.off[2 * l], k, nullptr, nullptr,
-                                   dnext);
-            k_silu_grad<<<1024, 256, 0, ctx->stream>>>(s.d_Z[l - 1], dnext, (long long)rows * s.width);
+            mlp_gemm<true, false, 3>(ctx, rows, k, width_out, dcur, width_out, P + s.off[2 * l], k, nullptr,
+                                     s.d_Z[l - 1], dnext);
             std::swap(dcur, dnext);
             width_out = s.width;
         }
     }
+    k_fold_parts<<<(unsigned)((s.n_par + 255) / 256), 256, 0, ctx->stream>>>(G, np, s.n_par, s.d_grad);
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
