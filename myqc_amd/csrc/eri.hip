@@ -551,17 +551,27 @@ static int build_schedule(myqc_ctx *ctx) {
         sao[X] = ctx->shells[X].ao;
         sL[X] = ctx->shells[X].L;
     }
-    // LDS rows: the G rows (FP64) and the D rows (FP64 for the plain pass)
-    const int max_rows = std::min(64, (int)(kDigestLds / (2 * sizeof(double) * (size_t)n)));
+    // Rows and values per workgroup.  LDS holds the G rows (FP64) and the D
+    // rows (FP64 for the plain pass), which bounds the rows; a system small
+    // enough to leave the chip short of workgroups takes fewer rows (down to
+    // one pair of p shells), and its values are cut into about 600 runs of at
+    // least 8k values, where a pass is bounded by its longest wavefronts'
+    // chains of row loads: measured (FP64 kernel, waters, with rows / values):
+    // 8: 131 us (58 rows, 64k) -> 24 us (6, 8k); 13: 104 -> 30; 24: 94 -> 69.
+    // A large one is bounded by traffic: fewer rows mean more partial rows to
+    // write and gather (40 waters: 171 us with 11 rows, 174 with 8, 189 with
+    // 6; 183 with 128k values each, 185 with 32k).  In between, 28 waters: 95
+    // us with 8 rows, 102 with 6, 105 with 11 of 64k.
+    const long long stored = ctx->n_stored;
+    const int lds_rows = (int)(kDigestLds / (2 * sizeof(double) * (size_t)n));
+    const int max_rows = std::min(lds_rows, stored < 12000000 ? 6 : stored < 32000000 ? 8 : 64);
+    const long long target = std::min(1LL << 16, std::max(1LL << 13, stored / 600));
     if (max_rows < 6)
         return set_error(ctx, MYQC_E_ARG, "digestion: n=%d leaves fewer than 6 rows of G and D in %zu bytes of LDS", n,
                          kDigestLds);
-    // workgroups of about 64k stored values: measured on the 40-water
-    // cluster, 2^15 and 2^17 were 8 % and 10 % slower per pass (fewer chunks
-    // per workgroup to balance its wavefronts, or too few workgroups)
     DigestPlan &pl = ctx->plan;
     const std::string e =
-        build_digest_schedule(pl, sao, sL, ctx->pairs, ctx->pair_ids, ctx->schwarz, max_rows, 1LL << 16);
+        build_digest_schedule(pl, sao, sL, ctx->pairs, ctx->pair_ids, ctx->schwarz, max_rows, target);
     if (!e.empty()) return set_error(ctx, MYQC_E_ARG, "%s", e.c_str());
     ctx->n_wg = (int)(pl.wg.size() / kWgInts);
     MYQC_CHECK(upload(ctx, &ctx->d_wg, pl.wg));
