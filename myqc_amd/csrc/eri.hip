@@ -268,21 +268,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(C
                 }
 }
 
-// Schwarz factor of each pair of one class: sqrt(max_ab |(ab|ab)|)
+// Schwarz factors sqrt(max_ab |(ab|ab)|) of the pairs of all three classes,
+// kSchwarzLanes lanes per pair sharing its up to 81 primitive quartets.  With
+// a lane per pair and a launch per class this was bounded by one lane's
+// serial chain (66 + 71 + 94 us for 40 waters, 55 + 55 + 86 for one water);
+// eight lanes each and one launch take 34 and 17 us.
+constexpr int kSchwarzLanes = 8, kSchwarzPairs = 256 / kSchwarzLanes;
+
 template <int C>
-__global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
-                                                 const double *__restrict__ ftT, const int *__restrict__ ids, int np,
-                                                 double *__restrict__ q) {
-    __shared__ double s_ft[FT_TOTAL];
-    load_ft(ftT, s_ft);
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= np) return;
+__device__ __forceinline__ void schwarz_pair(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
+                                             const double *s_ft, int p, bool on, int sub, double *__restrict__ q) {
     constexpr int LA = PairL<C>::a, LB = PairL<C>::b;
     constexpr int na = ncart(LA), nb = ncart(LB);
-    const int p = ids[t];
     const ShellPair sp = pairs[p];
-    QuartetAcc<LA, LB, LA, LB> acc;
-    quartet_prims<LA, LB, LA, LB, false>(sp, sp, prims, prims, s_ft, acc);
+    using AQ = QuartetAcc<LA, LB, LA, LB>;
+    AQ acc;
+    quartet_prims_split<LA, LB, LA, LB, kSchwarzLanes, false>(sp, sp, prims, [&](int j) { return prims[sp.pp0 + j]; },
+                                                              s_ft, acc, sub);
+#pragma unroll
+    for (int e = 0; e < AQ::NE; ++e)
+#pragma unroll
+        for (int f = 0; f < AQ::NF; ++f) acc.v[e][f] = group_sum<kSchwarzLanes>(acc.v[e][f]);
     double out[na * nb * na * nb];
     quartet_hrr<LA, LB, LA, LB>(acc, sp.AB, sp.AB, out);
     double m = 0.0;
@@ -290,7 +296,27 @@ __global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ p
     for (int ia = 0; ia < na; ++ia)
 #pragma unroll
         for (int ib = 0; ib < nb; ++ib) m = fmax(m, fabs(out[((ia * nb + ib) * na + ia) * nb + ib]));
-    q[p] = sqrt(m);
+    if (on && sub == 0) q[p] = sqrt(m);
+}
+
+struct SchwarzArgs {
+    const int *ids[3];   // pairs of each class
+    int np[3];
+    int blk[3];          // first workgroup of each class: blk[c] .. (pp pairs, the longest, come first)
+};
+
+__global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
+                                                 const double *__restrict__ ftT, SchwarzArgs a, double *__restrict__ q) {
+    __shared__ double s_ft[FT_TOTAL];
+    load_ft(ftT, s_ft);
+    const int b = blockIdx.x, c = b >= a.blk[0] ? 0 : b >= a.blk[1] ? 1 : 2;
+    // lanes past the last pair repeat it (the group sums need every lane)
+    const int t = (b - a.blk[c]) * kSchwarzPairs + threadIdx.x / kSchwarzLanes, sub = threadIdx.x % kSchwarzLanes;
+    const bool on = t < a.np[c];
+    const int p = a.ids[c][on ? t : a.np[c] - 1];
+    if (c == 0) schwarz_pair<0>(pairs, prims, s_ft, p, on, sub, q);
+    else if (c == 1) schwarz_pair<1>(pairs, prims, s_ft, p, on, sub, q);
+    else schwarz_pair<2>(pairs, prims, s_ft, p, on, sub, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -330,24 +356,21 @@ int eri_schwarz(myqc_ctx *ctx) {
     if (ctx->have_schwarz) return 0;
     const int np = (int)ctx->pairs.size();
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_schwarz, sizeof(double) * np));
-    for (int c = 0; c < 3; ++c) {
+    SchwarzArgs sa{};
+    int nblk = 0;
+    for (int c = 2; c >= 0; --c) {
         const auto &ids = ctx->pair_ids[c];
+        sa.blk[c] = nblk;
+        sa.np[c] = (int)ids.size();
         if (ids.empty()) continue;
         MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_sorted[c], sizeof(int) * ids.size()));
         MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_sorted[c], ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice,
                                      ctx->stream));
-        const int nblk = ((int)ids.size() + 255) / 256;
-        if (c == 0)
-            k_schwarz<0><<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, ctx->d_sorted[c],
-                                                         (int)ids.size(), ctx->d_schwarz);
-        else if (c == 1)
-            k_schwarz<1><<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, ctx->d_sorted[c],
-                                                         (int)ids.size(), ctx->d_schwarz);
-        else
-            k_schwarz<2><<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, ctx->d_sorted[c],
-                                                         (int)ids.size(), ctx->d_schwarz);
-        MYQC_HIP(ctx, hipGetLastError());
+        sa.ids[c] = ctx->d_sorted[c];
+        nblk += ((int)ids.size() + kSchwarzPairs - 1) / kSchwarzPairs;
     }
+    k_schwarz<<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, sa, ctx->d_schwarz);
+    MYQC_HIP(ctx, hipGetLastError());
     ctx->schwarz.resize(np);
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->schwarz.data(), ctx->d_schwarz, sizeof(double) * np, hipMemcpyDeviceToHost,
                                  ctx->stream));
@@ -415,22 +438,45 @@ static void class_counts(myqc_ctx *ctx, int cb, int ck, double tol, std::vector<
 }
 
 // Launch shape of each quartet class in the stored build: lanes per shell
-// quartet (1, 2, 4, 8) and threads per workgroup (64, 128, 256).  The
-// defaults hold until myqc_eri_tune measures the candidates on a system and
-// keeps the fastest of each class for the process.
+// quartet (1, 2, 4, 8) and threads per workgroup (64, 128, 256).  Until
+// myqc_eri_tune measures the candidates on a system and keeps the fastest of
+// each class for the process (or myqc_eri_set_shapes gives one), the lanes
+// follow the class's size.
 struct EriShape {
-    int split = 1, tpb = 256;
+    int split = 0, tpb = 256;   // split 0: by the rule
 };
 static std::mutex g_shape_mu;
 static EriShape g_shape[6];
 
-static EriShape class_shape(int c) {
-    std::lock_guard<std::mutex> g(g_shape_mu);
-    return g_shape[c];
+// A class with few quartets is bounded by one lane's chain of up to 81
+// primitive quartets, not by throughput, so its quartets are spread over as
+// many lanes as keep it under 2^18 lanes (a full chip of four wavefronts per
+// SIMD): one water's build took 387 us with a lane per quartet, 102 us with
+// eight; eight waters 393 -> 157.  The best of 1, 2, 4, 8 lanes as measured:
+// ss|ss 16k quartets 8, 72k 4, 140k 2, 358k 1; ps|ps 33k 8, 77k 2, 222k 1;
+// pp|ss 19k 8, 47k 4, 125k 2, 340k 1; pp|ps 22k 8, 62k 4, 154k 1.  pp|pp, whose
+// lane holds the most registers, gains from eight lanes only below 8k
+// quartets (4.6k 8, 10k 4), and one lane of it never pays (20k quartets: 213
+// us with one lane, 81 with four).
+static int rule_split(int c, long long nq) {
+    if (c == 5) return nq <= (1 << 13) ? 8 : 4;
+    int s = 8;
+    while (s > 1 && nq * s > (1 << 18)) s >>= 1;
+    return s;
+}
+
+static EriShape class_shape(int c, long long nq) {
+    EriShape sh;
+    {
+        std::lock_guard<std::mutex> g(g_shape_mu);
+        sh = g_shape[c];
+    }
+    if (sh.split == 0) sh.split = rule_split(c, nq);
+    return sh;
 }
 
 template <int CB, int CK, int MODE>
-static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, double *XX, hipStream_t s, EriShape sh = EriShape{}) {
+static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, double *XX, hipStream_t s, EriShape sh) {
     EriArgs a;
     a.pairs = ctx->d_pairs;
     a.prims = ctx->d_prims;
@@ -448,8 +494,7 @@ static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, double *XX, hipStr
     a.x32 = ctx->d_x32;
     a.XX = XX;
     a.n = ctx->n;
-    if (MODE == 1) sh = EriShape{};   // the dense fill (small systems) keeps one lane per quartet
-    const long long nblk = (qc.nq * sh.split + sh.tpb - 1) / sh.tpb;
+        const long long nblk = (qc.nq * sh.split + sh.tpb - 1) / sh.tpb;
     switch (sh.split) {
         case 2: k_eri<CB, CK, MODE, 2><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
         case 4: k_eri<CB, CK, MODE, 4><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
@@ -654,7 +699,7 @@ int eri_store(myqc_ctx *ctx, double tol, bool want32) {
     for (int c : kOrder) {
         if (ctx->cls[c].nq == 0) continue;
         launch_class<0>(ctx, c, nullptr, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream,
-                        class_shape(c));
+                        class_shape(c, ctx->cls[c].nq));
         MYQC_HIP(ctx, hipGetLastError());
     }
     for (int k = 0; k < 2; ++k) {
@@ -691,7 +736,7 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
     EriShape best[6];
     double best_ms[6];
     for (int c = 0; c < 6 && rc == 0; ++c) {
-        best[c] = class_shape(c);
+        best[c] = class_shape(c, ctx->cls[c].nq);
         best_ms[c] = 0.0;
         if (ctx->cls[c].nq == 0) continue;
         best_ms[c] = 1e300;
@@ -762,7 +807,7 @@ int eri_fill_dense(myqc_ctx *ctx, double tol, double *d_XX) {
         hipEvent_t ev;
         rc = timer_begin(ctx, T_ERI, &ev);
         for (int c = 0; c < 6 && rc == 0; ++c) {
-            launch_class<1>(ctx, c, d_XX, ctx->stream, EriShape{});
+            launch_class<1>(ctx, c, d_XX, ctx->stream, class_shape(c, ctx->cls[c].nq));
             if (hipGetLastError() != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "ERI dense-fill launch failed");
         }
         if (rc == 0) rc = timer_end(ctx, T_ERI, ev, ctx->eri_flops);

@@ -375,7 +375,7 @@ MYQC_HD void quartet_prims_f(const ShellPair &bra, const ShellPair &ket, const P
 // The same sum split over SPLIT lanes: lane `sub` of the quartet's group
 // takes the primitive quartets t = j npp_bra + i with t = sub (mod SPLIT);
 // the group's partial sums are added afterwards (split_reduce on the device).
-template <int LA, int LB, int LC, int LD, int SPLIT, typename KF>
+template <int LA, int LB, int LC, int LD, int SPLIT, bool SCREEN = true, typename KF>
 MYQC_HD void quartet_prims_split(const ShellPair &bra, const ShellPair &ket, const PrimPair *__restrict__ ppb,
                                  KF &&kprim, const double *__restrict__ ftT, QuartetAcc<LA, LB, LC, LD> &acc,
                                  int sub) {
@@ -395,7 +395,8 @@ MYQC_HD void quartet_prims_split(const ShellPair &bra, const ShellPair &ket, con
     for (int t = sub; t < total; t += SPLIT) {
         const PrimPair k = kprim(j);
         const PrimPair b = ppb[bra.pp0 + i];
-        if (!(b.EIJ * k.EIJ < 1.0e-14)) prim_quartet<LA, LB, LC, LD>(b, k, Q, c0, ftT, acc);   // int2e.f90:257
+        if (!(SCREEN && b.EIJ * k.EIJ < 1.0e-14))
+            prim_quartet<LA, LB, LC, LD>(b, k, Q, c0, ftT, acc);   // int2e.f90:257
         i += SPLIT;
         while (i >= nbp) {
             i -= nbp;
