@@ -11,17 +11,18 @@
 #include <cmath>
 #include <vector>
 
-#include "context.h"
+#include "dense.h"
 
 namespace myqc {
-int gemm_bf16x3(myqc_ctx *ctx, bool transA, int m, int n, int k, const double *A, int lda, long long strideA,
-                const double *B, int ldb, long long strideB, double *C, int ldc, long long strideC, int batch);
-int ao2mo12_bf16x3(myqc_ctx *ctx, int np, const double *Cp, int nq, const double *Cq, int n, const double *XX,
-                   double *M);
-int ao2mo12_f64(myqc_ctx *ctx, int np, const double *Cp, int nq, const double *Cq, int n, const double *XX,
-                double *M);
+// (mfma_gemm.hip, mfma_f64.hip)
+int bf16x3_planes(myqc_ctx *ctx, const TransformJob *jobs, int njobs, int n);
+int ao2mo12_bf16x3(myqc_ctx *ctx, const TransformJob *jobs, int njobs, int job, int n, const double *XX, int nblk,
+                   const int *tri);
+int ao2mo12_f64(myqc_ctx *ctx, const TransformJob &job, int n, const double *XX, int nblk, const int *tri);
+int gemm_bf16x3(myqc_ctx *ctx, int m, int n, int k, const double *A, int lda, long long strideA, const double *B,
+                int ldb, double *C, int ldc, long long strideC, int batch, bool tri);
 int gemm_f64(myqc_ctx *ctx, int m, int nb, int k, const double *A, long long lda, long long sA, const double *B,
-             long long ldb, double *C, long long ldc, long long sC, int batch);
+             long long ldb, double *C, long long ldc, long long sC, int batch, bool tri);
 }
 
 namespace myqc {
@@ -169,110 +170,119 @@ __global__ __launch_bounds__(256) void k_mp2_fold(const double *__restrict__ par
     }
 }
 
-// Quarter steps 1 and 2 (idx1_trans, idx2_trans) over two column blocks of
-// orbitals, Cp (n x np) and Cq (n x nq), leading dimension n, fused per (l,d)
-// block so that L(p,v,l,d) = sum_u Cp(u,p) XX(u,v,l,d) stays on chip:
-//   M(p,q,l,d) = sum_v [sum_u Cp(u,p) XX(u,v,l,d)] Cq(v,q)      (np x nq x n x n)
-// With release_xx, *dXX is freed once nothing reads it any more.
-static int quarter12(myqc_ctx *ctx, double **dXX, bool release_xx, const double *Cp, int np, const double *Cq, int nq,
-                     int precision, double **dM) {
+// Quarter steps 1 and 2 (idx1_trans, idx2_trans) of the listed jobs over
+// pairs of column blocks of orbitals, Cp (n x np) and Cq (n x nq), leading
+// dimension n, fused per (l,d) block so that L(p,v,l,d) = sum_u Cp(u,p)
+// XX(u,v,l,d) stays on chip:
+//   M(p,q,l,d) = sum_v [sum_u Cp(u,p) XX(u,v,l,d)] Cq(v,q)
+// XX, and so M, is symmetric in (l,d): only l >= d is formed, M's block at
+// l (l + 1) / 2 + d (np x nq x n (n + 1) / 2 in all).  The blocks of XX are
+// expanded from the stored integrals a buffer's worth at a time.  24 waters,
+// FP64: 6.4 ms for the expansion and both steps (all n^2 blocks of a
+// dense XX of 6.4 GB: 5.6 ms, and 20.9 to fill it).
+static int transform12(myqc_ctx *ctx, DenseSource &src, const TransformJob *jobs, int njobs, int precision) {
     const int n = ctx->n;
-    const size_t N = n, msize = sizeof(double) * (size_t)np * nq * N * N;
-    MYQC_CHECK(dalloc(ctx, (void **)dM, msize));   // (a kept buffer of that size is reused)
-    if (precision == MYQC_BF16X3) MYQC_CHECK(ao2mo12_bf16x3(ctx, np, Cp, nq, Cq, n, *dXX, *dM));
-    else MYQC_CHECK(ao2mo12_f64(ctx, np, Cp, nq, Cq, n, *dXX, *dM));
-    if (release_xx) dfree((void **)dXX);   // (hipFree waits for the kernel)
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_xwork, src.chunk_bytes()));
+    if (precision == MYQC_BF16X3) MYQC_CHECK(bf16x3_planes(ctx, jobs, njobs, n));
+    for (const ExpandChunk &c : src.chunks) {
+        MYQC_CHECK(src.expand(c, ctx->d_xwork));
+        for (int j = 0; j < njobs; ++j)
+            if (precision == MYQC_BF16X3)
+                MYQC_CHECK(ao2mo12_bf16x3(ctx, jobs, njobs, j, n, ctx->d_xwork, c.nblk, src.d_tri + c.blk0));
+            else
+                MYQC_CHECK(ao2mo12_f64(ctx, jobs[j], n, ctx->d_xwork, c.nblk, src.d_tri + c.blk0));
+    }
     return 0;
 }
 
 // C = A B with A (m x k, lda, stride sA per problem) and the shared B (k x nb,
-// leading dimension k) for `batch` problems, in the transform's precision
+// leading dimension k) for `batch` problems, in the transform's precision.
+// tri: column kk of problem d's A is block (kk, d) of a triangular array
 static int quarter_gemm(myqc_ctx *ctx, int m, int nb, int k, const double *A, long long lda, long long sA,
-                        const double *B, double *C, long long ldc, long long sC, int batch, int precision) {
+                        const double *B, double *C, long long ldc, long long sC, int batch, int precision,
+                        bool tri = false) {
     if (precision == MYQC_BF16X3)
-        return gemm_bf16x3(ctx, false, m, nb, k, A, (int)lda, sA, B, k, 0, C, (int)ldc, sC, batch);
-    return gemm_f64(ctx, m, nb, k, A, lda, sA, B, k, C, ldc, sC, batch);
+        return gemm_bf16x3(ctx, m, nb, k, A, (int)lda, sA, B, k, C, (int)ldc, sC, batch, tri);
+    return gemm_f64(ctx, m, nb, k, A, lda, sA, B, k, C, ldc, sC, batch, tri);
 }
 
 // Quarter steps 3 and 4 (idx3_trans, idx4_trans) with the second pair's
 // orbital blocks Cr (n x nr) and Cs (n x ns):
 //   O(pq,r,s) = sum_d [sum_l M(pq,l,d) Cr(l,r)] Cs(d,s)     (m1 x nr x ns, pq fastest)
 static int quarter34(myqc_ctx *ctx, const double *dM, int m1, const double *Cr, int nr, const double *Cs, int ns,
-                     int precision, double *dO, double **keep = nullptr) {
+                     int precision, double *dO) {
     const int n = ctx->n;
-    const size_t N = n;
-    double *dN = keep ? *keep : nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&dN, sizeof(double) * (size_t)m1 * nr * N));
-    if (keep) *keep = dN;
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_q3, sizeof(double) * std::max<size_t>((size_t)m1 * nr * n, 1)));
     // 3: N(pq,r,d) = sum_l M(pq,l,d) Cr(l,r)
-    int rc = quarter_gemm(ctx, m1, nr, n, dM, m1, (long long)m1 * n, Cr, dN, m1, (long long)m1 * nr, n, precision);
+    int rc = quarter_gemm(ctx, m1, nr, n, dM, m1, 0, Cr, ctx->d_q3, m1, (long long)m1 * nr, n, precision, true);
     // 4: O(pq,r,s) = sum_d N(pq,r,d) Cs(d,s)
     if (rc == 0)
-        rc = quarter_gemm(ctx, m1 * nr, ns, n, dN, (long long)m1 * nr, 0, Cs, dO, (long long)m1 * nr, 0, 1, precision);
-    if (!keep) dfree((void **)&dN);
+        rc = quarter_gemm(ctx, m1 * nr, ns, n, ctx->d_q3, (long long)m1 * nr, 0, Cs, dO, (long long)m1 * nr, 0, 1,
+                          precision);
     return rc;
 }
 
-static double transform_flops(int o1, int nv1, int o2, int nv2, int n) {
+// operations of steps 3-4, and of steps 1-2 over the pairs l >= d
+static double flops34(int o1, int nv1, int o2, int nv2, int n) {
     const double N = n;
-    return 2.0 * ((double)o1 * N * N * N * N + (double)o1 * nv1 * N * N * N + (double)o1 * nv1 * o2 * N * N +
-                  (double)o1 * nv1 * o2 * nv2 * N);
+    return 2.0 * ((double)o1 * nv1 * o2 * N * N + (double)o1 * nv1 * o2 * nv2 * N);
+}
+static double flops12(int np, int nq, int n) {
+    const double N = n;
+    return ((double)np * N * N + (double)np * nq * N) * N * (N + 1);
 }
 
-static int upload_square(myqc_ctx *ctx, const double *host, double **dev) {
+// a scratch array of the transforms above this is given back after the call
+static void give_back(double **p, size_t keep = (size_t)4 << 30) {
+    if (dcapacity(*p) > keep) dfree((void **)p);
+}
+
+static int upload_square(myqc_ctx *ctx, const double *host, int slot, double **dev) {
     const size_t nn = (size_t)ctx->n * ctx->n;
-    MYQC_CHECK(dalloc(ctx, (void **)dev, sizeof(double) * nn));
+    MYQC_CHECK(dtmp(ctx, slot, dev, sizeof(double) * nn));
     if (hipMemcpyAsync(*dev, host, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
         return set_error(ctx, MYQC_E_HIP, "ao2mo: upload failed");
     return 0;
 }
 
-// dense AO integrals at the stored build's screening threshold
-static int dense_integrals(myqc_ctx *ctx, double **dXX) {
-    const size_t N = ctx->n;
-    MYQC_CHECK(dalloc(ctx, (void **)dXX, sizeof(double) * N * N * N * N));
-    return eri_fill_dense(ctx, ctx->have_eri ? ctx->eri_tol : 0.0, *dXX);
+// the transforms' integrals: at the stored build's screening threshold
+static double transform_tol(myqc_ctx *ctx) { return ctx->have_eri ? ctx->eri_tol : 0.0; }
+
+// the context's d_q12 for M of `vals` values
+static int m_buffer(myqc_ctx *ctx, double **p, size_t vals) {
+    return dalloc(ctx, (void **)p, sizeof(double) * std::max<size_t>(vals, 1));
 }
 
 // RHF: (ia|jb) for the one set of orbitals (slow_ao2mo_MP2_RHF,
 // src/ao2mo/ao2mo.f90:465-602) into ctx->d_iajb
 static int ao2mo(myqc_ctx *ctx, const double *C_host, int o, int precision) {
     const int n = ctx->n, nv = n - o;
-    double *dXX = nullptr, *dC = nullptr;
-    int rc = 0;
-    auto cleanup = [&]() {
-        dfree((void **)&dXX);
-        dfree((void **)&dC);
-    };
-#define TRY(x)          \
-    do {                \
-        rc = (x);       \
-        if (rc) {       \
-            cleanup();  \
-            return rc;  \
-        }               \
-    } while (0)
-    TRY(upload_square(ctx, C_host, &dC));
-    TRY(dense_integrals(ctx, &dXX));
+    const size_t N = n, tri = N * (N + 1) / 2, oe = (size_t)o * nv * o * nv;
+    double *dC = nullptr;
+    DenseSource src(ctx);
+    MYQC_CHECK(upload_square(ctx, C_host, TMP_CA, &dC));
+    MYQC_CHECK(src.open(transform_tol(ctx)));
+    MYQC_CHECK(src.plan_chunks());
     // the output and the quarter-step intermediates (kept by the context, so
     // a repeated transform of one size allocates nothing) before the timed
     // region
-    const size_t oe = (size_t)o * nv * o * nv, N = n;
     if (ctx->iajb_elems != oe) {
-        TRY(dalloc(ctx, (void **)&ctx->d_iajb, sizeof(double) * (oe ? oe : 1)));
+        ctx->iajb_elems = 0;
+        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_iajb, sizeof(double) * (oe ? oe : 1)));
         ctx->iajb_elems = oe;
     }
-    TRY(dalloc(ctx, (void **)&ctx->d_q12, sizeof(double) * std::max<size_t>((size_t)o * nv * N * N, 1)));
-    TRY(dalloc(ctx, (void **)&ctx->d_q3, sizeof(double) * std::max<size_t>((size_t)o * nv * o * N, 1)));
+    MYQC_CHECK(m_buffer(ctx, &ctx->d_q12, (size_t)o * nv * tri));
+    const TransformJob job{dC, o, dC + N * o, nv, ctx->d_q12};
     hipEvent_t ev;
-    TRY(timer_begin(ctx, T_AO2MO, &ev));
-    TRY(quarter12(ctx, &dXX, false, dC, o, dC + (size_t)n * o, nv, precision, &ctx->d_q12));
-    TRY(quarter34(ctx, ctx->d_q12, o * nv, dC, o, dC + (size_t)n * o, nv, precision, ctx->d_iajb, &ctx->d_q3));
-    TRY(timer_end(ctx, T_AO2MO, ev, transform_flops(o, nv, o, nv, n)));
+    MYQC_CHECK(timer_begin(ctx, T_AO2MO, &ev));
+    MYQC_CHECK(transform12(ctx, src, &job, 1, precision));
+    MYQC_CHECK(quarter34(ctx, ctx->d_q12, o * nv, dC, o, dC + N * o, nv, precision, ctx->d_iajb));
+    MYQC_CHECK(timer_end(ctx, T_AO2MO, ev, flops12(o, nv, n) + flops34(o, nv, o, nv, n)));
     ctx->iajb_nocc = o;
     ctx->iajb_nv = nv;
-    cleanup();
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    give_back(&ctx->d_q12);
+    give_back(&ctx->d_q3);
     return 0;
 }
 
@@ -282,74 +292,78 @@ static int ao2mo(myqc_ctx *ctx, const double *C_host, int o, int precision) {
 // into ctx->d_vvoo[0..1] (alpha, beta), [a][b][i][j] with a fastest, from the
 // same dense integrals.
 // The reference recomputes the first two quarter steps for each set; here
-// M_A = steps 1-2 with Ca serves both AA and AB, so the dense integrals are
-// contracted twice (Ca, Cb) instead of three times.  A set with no occupied
-// or no virtual orbital is empty.
+// M_A = steps 1-2 with Ca serves both AA and AB, and every block of the AO
+// integrals is contracted for all of M_A, M_B and the (ab|..) of each spin
+// while it is at hand.  A set with no occupied or no virtual orbital is empty.
 int ao2mo_uhf(myqc_ctx *ctx, const double *Ca_host, const double *Cb_host, int oa, int ob, int precision, bool vvoo) {
     const int n = ctx->n, va = n - oa, vb = n - ob;
-    double *dXX = nullptr, *dCa = nullptr, *dCb = nullptr, *dMa = nullptr, *dMb = nullptr;
-    int rc = 0;
-    auto cleanup = [&]() {
-        dfree((void **)&dXX);
-        dfree((void **)&dCa);
-        dfree((void **)&dCb);
-        dfree((void **)&dMa);
-        dfree((void **)&dMb);
-    };
+    const size_t N = n, tri = N * (N + 1) / 2;
     ctx->have_uhf = ctx->have_vvoo = false;
     const int dims[3][4] = {{oa, va, oa, va}, {ob, vb, ob, vb}, {oa, va, ob, vb}};
     for (int s = 0; s < 3; ++s) {
         const size_t e = (size_t)dims[s][0] * dims[s][1] * dims[s][2] * dims[s][3];
-        TRY(dalloc(ctx, (void **)&ctx->d_uhf[s], sizeof(double) * (e ? e : 1)));
+        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_uhf[s], sizeof(double) * (e ? e : 1)));
         for (int k = 0; k < 4; ++k) ctx->uhf_dims[s][k] = dims[s][k];
     }
     const bool want_a = (size_t)oa * va > 0, want_b = (size_t)ob * vb > 0;
-    TRY(upload_square(ctx, Ca_host, &dCa));
-    TRY(upload_square(ctx, Cb_host, &dCb));
-    if (want_a || want_b) TRY(dense_integrals(ctx, &dXX));
-    hipEvent_t ev;
-    TRY(timer_begin(ctx, T_AO2MO, &ev));
+    double *dC[2] = {nullptr, nullptr};
+    MYQC_CHECK(upload_square(ctx, Ca_host, TMP_CA, &dC[0]));
+    MYQC_CHECK(upload_square(ctx, Cb_host, TMP_CB, &dC[1]));
+    DenseSource src(ctx);
+    // the M of each job, one after another in d_q12: both spins' (occ, virt),
+    // then both spins' (virt, virt)
+    const int os[2] = {oa, ob}, vs[2] = {va, vb};
+    TransformJob jobs[4];
+    size_t at[4], vals = 0;
+    int njobs = 0, jov[2] = {-1, -1}, jvv[2] = {-1, -1};
     double flops = 0.0;
-    if (want_a) TRY(quarter12(ctx, &dXX, !want_b && !vvoo, dCa, oa, dCa + (size_t)n * oa, va, precision, &dMa));
-    if (want_b) TRY(quarter12(ctx, &dXX, !vvoo, dCb, ob, dCb + (size_t)n * ob, vb, precision, &dMb));
-    if (vvoo) {
-        const double *Cs[2] = {dCa, dCb};
-        const int os[2] = {oa, ob}, vs[2] = {va, vb};
-        for (int s = 0; s < 2; ++s) {
-            const size_t e = (size_t)vs[s] * vs[s] * os[s] * os[s];
-            TRY(dalloc(ctx, (void **)&ctx->d_vvoo[s], sizeof(double) * (e ? e : 1)));
-            ctx->vvoo_dims[s][0] = vs[s];
-            ctx->vvoo_dims[s][1] = os[s];
-            if (e == 0) continue;
-            double *dV = nullptr;
-            const double *Cv = Cs[s] + (size_t)n * os[s];
-            rc = quarter12(ctx, &dXX, false, Cv, vs[s], Cv, vs[s], precision, &dV);
-            if (rc == 0) rc = quarter34(ctx, dV, vs[s] * vs[s], Cs[s], os[s], Cs[s], os[s], precision, ctx->d_vvoo[s]);
-            dfree((void **)&dV);
-            TRY(rc);
-            flops += transform_flops(vs[s], vs[s], os[s], os[s], n);
+    auto add = [&](int s, int p0, int np, int q0, int nq) {
+        jobs[njobs] = TransformJob{dC[s] + N * p0, np, dC[s] + N * q0, nq, nullptr};
+        at[njobs] = vals;
+        vals += (size_t)np * nq * tri;
+        flops += flops12(np, nq, n);
+        return njobs++;
+    };
+    for (int s = 0; s < 2; ++s)
+        if (os[s] > 0 && vs[s] > 0) jov[s] = add(s, 0, os[s], os[s], vs[s]);
+    for (int s = 0; s < 2 && vvoo; ++s) {
+        const size_t e = (size_t)vs[s] * vs[s] * os[s] * os[s];
+        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_vvoo[s], sizeof(double) * (e ? e : 1)));
+        ctx->vvoo_dims[s][0] = vs[s];
+        ctx->vvoo_dims[s][1] = os[s];
+        if (e) jvv[s] = add(s, os[s], vs[s], os[s], vs[s]);
+    }
+    if (njobs > 0) {
+        MYQC_CHECK(src.open(transform_tol(ctx)));
+        MYQC_CHECK(src.plan_chunks());
+        MYQC_CHECK(m_buffer(ctx, &ctx->d_q12, vals));
+        for (int j = 0; j < njobs; ++j) jobs[j].M = ctx->d_q12 + at[j];
+    }
+    hipEvent_t ev;
+    MYQC_CHECK(timer_begin(ctx, T_AO2MO, &ev));
+    if (njobs > 0) MYQC_CHECK(transform12(ctx, src, jobs, njobs, precision));
+    for (int s = 0; s < 2; ++s)
+        if (jvv[s] >= 0) {
+            MYQC_CHECK(quarter34(ctx, jobs[jvv[s]].M, vs[s] * vs[s], dC[s], os[s], dC[s], os[s], precision,
+                                 ctx->d_vvoo[s]));
+            flops += flops34(vs[s], vs[s], os[s], os[s], n);
         }
-    }
-    dfree((void **)&dXX);
-    if (want_a) {
-        TRY(quarter34(ctx, dMa, oa * va, dCa, oa, dCa + (size_t)n * oa, va, precision, ctx->d_uhf[0]));
-        flops += transform_flops(oa, va, oa, va, n);
-    }
-    if (want_b) {
-        TRY(quarter34(ctx, dMb, ob * vb, dCb, ob, dCb + (size_t)n * ob, vb, precision, ctx->d_uhf[1]));
-        flops += transform_flops(ob, vb, ob, vb, n);
-    }
+    for (int s = 0; s < 2; ++s)
+        if (jov[s] >= 0) {
+            MYQC_CHECK(quarter34(ctx, jobs[jov[s]].M, os[s] * vs[s], dC[s], os[s], dC[s] + N * os[s], vs[s], precision,
+                                 ctx->d_uhf[s]));
+            flops += flops34(os[s], vs[s], os[s], vs[s], n);
+        }
     if (want_a && want_b) {
-        TRY(quarter34(ctx, dMa, oa * va, dCb, ob, dCb + (size_t)n * ob, vb, precision, ctx->d_uhf[2]));
-        // steps 3-4 only: steps 1-2 are shared with the AA set
-        flops += 2.0 * ((double)oa * va * ob * n * n + (double)oa * va * ob * vb * n);
+        MYQC_CHECK(quarter34(ctx, jobs[jov[0]].M, oa * va, dC[1], ob, dC[1] + N * ob, vb, precision, ctx->d_uhf[2]));
+        flops += flops34(oa, va, ob, vb, n);   // (steps 1-2 are shared with the AA set)
     }
-    TRY(timer_end(ctx, T_AO2MO, ev, flops));
-    cleanup();
+    MYQC_CHECK(timer_end(ctx, T_AO2MO, ev, flops));
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    give_back(&ctx->d_q12);
+    give_back(&ctx->d_q3);
     ctx->have_uhf = true;
     ctx->have_vvoo = vvoo;
-#undef TRY
     return 0;
 }
 
@@ -358,13 +372,13 @@ static int download_records(myqc_ctx *ctx, const double *dO, const int *d, int t
     const size_t nrec = tri ? (size_t)d[0] * (d[0] > 0 ? d[0] - 1 : 0) / 2 : (size_t)d[0] * d[2];
     const size_t cnt = nrec * d[1] * d[3];
     if (cnt == 0) return 0;
-    double *d_rec = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&d_rec, sizeof(double) * cnt));
-    k_records<<<1024, 256, 0, ctx->stream>>>(dO, d_rec, d[0], d[1], d[2], d[3], tri);
+    // the transform's intermediate N is done with: the records go there
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_q3, sizeof(double) * cnt));
+    k_records<<<1024, 256, 0, ctx->stream>>>(dO, ctx->d_q3, d[0], d[1], d[2], d[3], tri);
     int rc = 0;
-    if (d2h(ctx, host, d_rec, sizeof(double) * cnt) != hipSuccess)
+    if (d2h(ctx, host, ctx->d_q3, sizeof(double) * cnt) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "ao2mo: download failed");
-    dfree((void **)&d_rec);
+    give_back(&ctx->d_q3);
     return rc;
 }
 

@@ -124,6 +124,10 @@ struct myqc_ctx {
     // ao2mo output kept on the device for mp2
     double *d_iajb = nullptr;             // [i][a][j][b] with i fastest (o*v*o*v)
     double *d_q12 = nullptr, *d_q3 = nullptr;   // the RHF transform's quarter-step intermediates (kept)
+    // dense blocks of the AO integrals being contracted (or the dense array of
+    // a small int2e call) and the tables they are expanded by (dense.hip)
+    double *d_xwork = nullptr;
+    void *d_dtab = nullptr;
     uint16_t *d_planes = nullptr;         // split-bf16 GEMM: hi/lo planes of the small operand
     size_t iajb_elems = 0;
     int iajb_nocc = 0, iajb_nv = 0;
@@ -152,7 +156,7 @@ struct myqc_ctx {
     // guess), kept across calls with their capacity: a repeated call makes no
     // hipMalloc/hipFree (hipFree waits for the whole device, which would
     // serialise contexts that run side by side on other streams)
-    void *d_tmp[8] = {};
+    void *d_tmp[16] = {};
 
     // pinned host staging for small device-to-host reads (d2h)
     void *h_pin = nullptr;
@@ -202,6 +206,8 @@ int set_error(myqc_ctx *ctx, int code, const char *fmt, ...);
 
 // bytes of the pinned staging buffer (ctx->h_pin)
 constexpr size_t kPinBytes = 4096;
+// a work array up to this size stays with the context for the next call
+constexpr size_t kKeepWork = (size_t)320 << 20;
 // records (i,j) the no-allocation MP2 entry point takes at most (nocc <= 256)
 constexpr size_t kNoAllocRecords = 65536;
 
@@ -242,8 +248,8 @@ int blas_reserve(myqc_ctx *ctx, F calls) {
 }
 
 // slots of ctx->d_tmp
-enum TmpSlot { TMP_S = 0, TMP_H, TMP_ATOMS, TMP_GPAIRS, TMP_GATOMS, TMP_GDENS, TMP_GMOL, TMP_NSLOT };
-static_assert(TMP_NSLOT <= 8, "d_tmp slots");
+enum TmpSlot { TMP_S = 0, TMP_H, TMP_ATOMS, TMP_GPAIRS, TMP_GATOMS, TMP_GDENS, TMP_GMOL, TMP_CA, TMP_CB, TMP_NSLOT };
+static_assert(TMP_NSLOT <= 16, "d_tmp slots");
 // a temporary of at least `bytes` in slot `slot`, kept by the context
 template <typename T>
 int dtmp(myqc_ctx *ctx, int slot, T **p, size_t bytes) {
@@ -278,7 +284,7 @@ struct HostClock {
 // internals shared between translation units
 int eri_schwarz(myqc_ctx *ctx);
 int eri_store(myqc_ctx *ctx, double tol, bool want32);
-int eri_fill_dense(myqc_ctx *ctx, double tol, double *d_XX);
+int eri_values(myqc_ctx *ctx, double tol, bool want32);
 // G(D) into d_G (precision FP64), or d_G += G32(D - Dprev) (precision FP32;
 // Dprev may be NULL for D itself)
 int digest_G(myqc_ctx *ctx, const double *d_D, double *d_G, int precision, const double *d_Dprev = nullptr);

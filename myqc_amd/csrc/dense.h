@@ -1,0 +1,82 @@
+// dense.h -- square blocks of the AO integrals, (uv|ld) over all u, v for one
+// function pair (l, d), expanded from the stored (element-major, pre-weighted)
+// integrals of digest_plan.h.
+#pragma once
+
+#include "context.h"
+
+namespace myqc {
+
+// Function pairs (l, d) expanded by one workgroup: the same element of up to
+// kExpPairs shell pairs of consecutive Schwarz rank.
+constexpr int kExpPairs = 16;
+struct ExpandRec {
+    int pos0, cls, ep, pad;      // first pair (class-sorted position), its class, the element
+    int ld[kExpPairs];           // l + n d of each pair's element, -1: none
+    int blk[kExpPairs];          // its block
+};
+
+// A run of records whose blocks fit the work buffer
+struct ExpandChunk {
+    int rec0, nrec;              // records
+    int blk0, nblk;              // blocks, as a range of the triangular indices below
+};
+
+// The unscreened-or-screened value store at threshold `tol`, opened for
+// expansion: the context's stored integrals when they were built at that
+// threshold, else a build of its own, which leaves the context's stored
+// integrals as they are.  close() (or the destructor) gives back what the
+// open made.
+class DenseSource {
+  public:
+    explicit DenseSource(myqc_ctx *c) : ctx(c) {}
+    ~DenseSource() { close(); }
+    int open(double tol);
+    void close();
+
+    // Blocks of the pairs l >= d in chunks: records and tables go to the
+    // device; chunk c's blocks are written by expand() to X, block b of the
+    // chunk at X + b n^2, and d_tri + chunk.blk0 + b holds its l (l + 1) / 2 + d.
+    int plan_chunks();
+    std::vector<ExpandChunk> chunks;
+    const int *d_tri = nullptr;
+    int expand(const ExpandChunk &c, double *X);
+    size_t chunk_bytes() const;
+    // all blocks at their places in the dense n^4 array
+    int expand_full(double *XX);
+
+  private:
+    int tables(bool full);
+    myqc_ctx *ctx;
+    bool opened = false, swapped = false;
+    // the context's own store, put aside while another is open
+    struct Saved {
+        QuartetClass cls[6];
+        DigestPlan plan;
+        long long *d_segoff;
+        int *d_rank;
+        double *d_x64;
+        float *d_x32;
+        long long n_stored, n_quartets;
+        double eri_flops;
+        int ns;
+    } saved;
+    // device tables (ctx->d_dtab)
+    const int *d_T = nullptr;
+    const long long *d_off = nullptr;
+    const int2 *d_range = nullptr;
+    const ExpandRec *d_rec = nullptr;
+    int nrec = 0, pos1 = 0, pos2 = 0;
+};
+
+// One product of quarter steps 1 and 2: M(p, q, l d) from the orbital blocks
+// Cp (n x np) and Cq (n x nq), both with leading dimension n.
+struct TransformJob {
+    const double *Cp;
+    int np;
+    const double *Cq;
+    int nq;
+    double *M;
+};
+
+}  // namespace myqc

@@ -22,6 +22,7 @@
 #include <unordered_map>
 
 #include "context.h"
+#include "dense.h"
 #include "wave.h"
 #include "ket_soa.h"
 #include "system.h"
@@ -139,13 +140,10 @@ struct EriArgs {
     int nbra;
     long long nq;
     int same_class;
-    // MODE 0: the stored (pre-weighted) block of each quartet
+    // the stored (pre-weighted) block of each quartet
     const long long *segoff;   // [bra pair*3 + ket class]: element e of ket rank r at segoff + r + e*len
     double *x64;
     float *x32;
-    // MODE 1: dense XX
-    double *XX;
-    int n;
 };
 
 __device__ __forceinline__ void find_quartet(const long long *__restrict__ cum, int nbra, long long t, int same,
@@ -166,14 +164,13 @@ __device__ __forceinline__ void load_ft(const double *__restrict__ ftT, double *
     __syncthreads();
 }
 
-// MODE 0: store the block's copies for digestion;  MODE 1: scatter into dense XX (8-fold).
 // SPLIT lanes per shell quartet: they share its primitive quartets, add their
 // sums (group_sum), and each stores every SPLIT-th element of the block.
 // Waves per SIMD asked of the register allocator per class (the staged
 // table's 23 KB of LDS allows seven 256-thread workgroups per CU): ss|ss 6,
 // ps|ss 5, ps|ps and pp|ss 4, the rest unconstrained.
 constexpr int eri_waves(int cb, int ck) { return cb + ck == 0 ? 6 : cb + ck == 1 ? 5 : cb + ck == 2 ? 4 : 1; }
-template <int CB, int CK, int MODE, int SPLIT>
+template <int CB, int CK, int SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(CB, CK)))) void k_eri(EriArgs a) {
     __shared__ double s_ft[FT_TOTAL];
     load_ft(a.ftT, s_ft);
@@ -216,30 +213,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(C
     double out[BLK];
     quartet_hrr<LA, LB, LC, LD>(acc, bra.AB, CD, out);
     const int same_pair = (pb == pk);
-    if (MODE == 0) {
-        // one copy under the bra pair, each element times its degeneracy
-        // weight (the digestion then applies the same six updates to all);
-        // element-major over the bra's kets of this class (len of them)
-        const long long base = a.segoff[(long long)pb * 3 + CK] + rk;
-        const long long len = a.cum[rb + 1] - a.cum[rb];
-#pragma unroll
-        for (int ia = 0; ia < na; ++ia)
-#pragma unroll
-            for (int ib = 0; ib < nb; ++ib)
-#pragma unroll
-                for (int ic = 0; ic < nc; ++ic)
-#pragma unroll
-                    for (int id = 0; id < nd; ++id) {
-                        const int e = ((ia * nb + ib) * nc + ic) * nd + id;
-                        if (SPLIT > 1 && e % SPLIT != sub) continue;
-                        const double w = block_weight(ia, ib, ic, id, bra.same, ket.same, same_pair, nb, nd,
-                                                      bra.ao_a + ia, bra.ao_b + ib, ket.ao_a + ic, ket.ao_b + id);
-                        const double v = out[e] * w;
-                        a.x64[base + e * len] = v;
-                        if (a.x32) a.x32[base + e * len] = (float)v;
-                    }
-        return;
-    }
+    // one copy under the bra pair, each element times its degeneracy
+    // weight (the digestion then applies the same six updates to all);
+    // element-major over the bra's kets of this class (len of them)
+    const long long base = a.segoff[(long long)pb * 3 + CK] + rk;
+    const long long len = a.cum[rb + 1] - a.cum[rb];
 #pragma unroll
     for (int ia = 0; ia < na; ++ia)
 #pragma unroll
@@ -250,21 +228,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(C
                 for (int id = 0; id < nd; ++id) {
                     const int e = ((ia * nb + ib) * nc + ic) * nd + id;
                     if (SPLIT > 1 && e % SPLIT != sub) continue;
-                    const int i = bra.ao_a + ia, j = bra.ao_b + ib, k = ket.ao_a + ic, l = ket.ao_b + id;
-                    const double w = block_weight(ia, ib, ic, id, bra.same, ket.same, same_pair, nb, nd, i, j, k, l);
-                    if (w != 0.0) {
-                        const size_t n = a.n;
-                        const double v = out[e];
-                        const size_t I = i, J = j, K = k, L = l;
-                        a.XX[I + n * (J + n * (K + n * L))] = v;
-                        a.XX[J + n * (I + n * (K + n * L))] = v;
-                        a.XX[I + n * (J + n * (L + n * K))] = v;
-                        a.XX[J + n * (I + n * (L + n * K))] = v;
-                        a.XX[K + n * (L + n * (I + n * J))] = v;
-                        a.XX[L + n * (K + n * (I + n * J))] = v;
-                        a.XX[K + n * (L + n * (J + n * I))] = v;
-                        a.XX[L + n * (K + n * (J + n * I))] = v;
-                    }
+                    const double w = block_weight(ia, ib, ic, id, bra.same, ket.same, same_pair, nb, nd,
+                                                  bra.ao_a + ia, bra.ao_b + ib, ket.ao_a + ic, ket.ao_b + id);
+                    const double v = out[e] * w;
+                    a.x64[base + e * len] = v;
+                    if (a.x32) a.x32[base + e * len] = (float)v;
                 }
 }
 
@@ -475,8 +443,8 @@ static EriShape class_shape(int c, long long nq) {
     return sh;
 }
 
-template <int CB, int CK, int MODE>
-static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, double *XX, hipStream_t s, EriShape sh) {
+template <int CB, int CK>
+static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, hipStream_t s, EriShape sh) {
     EriArgs a;
     a.pairs = ctx->d_pairs;
     a.prims = ctx->d_prims;
@@ -492,28 +460,25 @@ static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, double *XX, hipStr
     a.segoff = ctx->d_segoff;
     a.x64 = ctx->d_x64;
     a.x32 = ctx->d_x32;
-    a.XX = XX;
-    a.n = ctx->n;
         const long long nblk = (qc.nq * sh.split + sh.tpb - 1) / sh.tpb;
     switch (sh.split) {
-        case 2: k_eri<CB, CK, MODE, 2><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
-        case 4: k_eri<CB, CK, MODE, 4><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
-        case 8: k_eri<CB, CK, MODE, 8><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
-        default: k_eri<CB, CK, MODE, 1><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
+        case 2: k_eri<CB, CK, 2><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
+        case 4: k_eri<CB, CK, 4><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
+        case 8: k_eri<CB, CK, 8><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
+        default: k_eri<CB, CK, 1><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
     }
 }
 
-template <int MODE>
-static void launch_class(myqc_ctx *ctx, int c, double *XX, hipStream_t s, EriShape sh) {
+static void launch_class(myqc_ctx *ctx, int c, hipStream_t s, EriShape sh) {
     const QuartetClass &qc = ctx->cls[c];
     if (qc.nq == 0) return;
     switch (c) {
-        case 0: launch_eri<0, 0, MODE>(ctx, qc, XX, s, sh); break;
-        case 1: launch_eri<1, 0, MODE>(ctx, qc, XX, s, sh); break;
-        case 2: launch_eri<1, 1, MODE>(ctx, qc, XX, s, sh); break;
-        case 3: launch_eri<2, 0, MODE>(ctx, qc, XX, s, sh); break;
-        case 4: launch_eri<2, 1, MODE>(ctx, qc, XX, s, sh); break;
-        case 5: launch_eri<2, 2, MODE>(ctx, qc, XX, s, sh); break;
+        case 0: launch_eri<0, 0>(ctx, qc, s, sh); break;
+        case 1: launch_eri<1, 0>(ctx, qc, s, sh); break;
+        case 2: launch_eri<1, 1>(ctx, qc, s, sh); break;
+        case 3: launch_eri<2, 0>(ctx, qc, s, sh); break;
+        case 4: launch_eri<2, 1>(ctx, qc, s, sh); break;
+        case 5: launch_eri<2, 2>(ctx, qc, s, sh); break;
     }
 }
 
@@ -671,11 +636,13 @@ static int ensure_side_streams(myqc_ctx *ctx) {
     return 0;
 }
 
-int eri_store(myqc_ctx *ctx, double tol, bool want32) {
+// The values of every screened quartet at threshold tol, and their layout:
+// all of the stored build but the digestion schedule.  Leaves the kernels
+// in flight on the context stream.
+int eri_values(myqc_ctx *ctx, double tol, bool want32) {
     HostClock hc(ctx);
     MYQC_CHECK(eri_schwarz(ctx));
     hc.mark("eri_store: Schwarz factors");
-    free_eri(ctx, true);
     MYQC_CHECK(build_classes(ctx, tol));
     hc.mark("eri_store: quartet classes");
     MYQC_CHECK(build_layout(ctx, tol));
@@ -684,8 +651,6 @@ int eri_store(myqc_ctx *ctx, double tol, bool want32) {
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_x64, sizeof(double) * nx));
     if (want32) MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_x32, sizeof(float) * nx));
     else dfree((void **)&ctx->d_x32);   // a kept buffer may be smaller than this build
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair, sizeof(double) * 9 * ctx->pairs.size()));
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair32, sizeof(float) * 9 * ctx->pairs.size()));
     MYQC_CHECK(ensure_side_streams(ctx));
     hipEvent_t ev;
     MYQC_CHECK(timer_begin(ctx, T_ERI, &ev));
@@ -698,8 +663,8 @@ int eri_store(myqc_ctx *ctx, double tol, bool want32) {
     static const int kOrder[6] = {5, 4, 3, 2, 0, 1};
     for (int c : kOrder) {
         if (ctx->cls[c].nq == 0) continue;
-        launch_class<0>(ctx, c, nullptr, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream,
-                        class_shape(c, ctx->cls[c].nq));
+        launch_class(ctx, c, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream,
+                     class_shape(c, ctx->cls[c].nq));
         MYQC_HIP(ctx, hipGetLastError());
     }
     for (int k = 0; k < 2; ++k) {
@@ -708,6 +673,16 @@ int eri_store(myqc_ctx *ctx, double tol, bool want32) {
     }
     MYQC_CHECK(timer_end(ctx, T_ERI, ev, ctx->eri_flops));
     hc.mark("eri_store: allocations and launches");
+    return 0;
+}
+
+int eri_store(myqc_ctx *ctx, double tol, bool want32) {
+    HostClock hc(ctx);
+    free_eri(ctx, true);
+    MYQC_CHECK(eri_values(ctx, tol, want32));
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair, sizeof(double) * 9 * ctx->pairs.size()));
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair32, sizeof(float) * 9 * ctx->pairs.size()));
+    hc.mark("eri_store: values");
     // the digestion schedule is built while the kernels run
     MYQC_CHECK(build_schedule(ctx));
     hc.mark("eri_store: schedule (host, beside the kernels)");
@@ -747,7 +722,7 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
                 for (int r = 0; r < reps && rc == 0; ++r) {
                     float ms = 0.0f;
                     if (hipEventRecord(e0, ctx->stream) != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "event");
-                    launch_class<0>(ctx, c, nullptr, ctx->stream, sh);
+                    launch_class(ctx, c, ctx->stream, sh);
                     if (!rc && (hipGetLastError() != hipSuccess || hipEventRecord(e1, ctx->stream) != hipSuccess ||
                                 hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
                         rc = set_error(ctx, MYQC_E_HIP, "myqc_eri_tune: class %d launch failed", c);
@@ -789,38 +764,6 @@ int eri_set_shapes(myqc_ctx *ctx, const int *shape) {
     for (int c = 0; c < 6; ++c)
         if (shape[2 * c] != 0) g_shape[c] = EriShape{shape[2 * c], shape[2 * c + 1]};
     return 0;
-}
-
-int eri_fill_dense(myqc_ctx *ctx, double tol, double *d_XX) {
-    MYQC_CHECK(eri_schwarz(ctx));
-    const size_t n = ctx->n;
-    MYQC_HIP(ctx, hipMemsetAsync(d_XX, 0, sizeof(double) * n * n * n * n, ctx->stream));
-    // the dense fill shares the class enumeration with the stored build
-    QuartetClass saved[6];
-    bool had = ctx->have_eri;
-    const long long saved_stored = ctx->n_stored, saved_quartets = ctx->n_quartets;
-    const double saved_flops = ctx->eri_flops;
-    for (int c = 0; c < 6; ++c) saved[c] = ctx->cls[c];
-    for (int c = 0; c < 6; ++c) ctx->cls[c] = QuartetClass{};
-    int rc = build_classes(ctx, tol);
-    if (rc == 0) {
-        hipEvent_t ev;
-        rc = timer_begin(ctx, T_ERI, &ev);
-        for (int c = 0; c < 6 && rc == 0; ++c) {
-            launch_class<1>(ctx, c, d_XX, ctx->stream, class_shape(c, ctx->cls[c].nq));
-            if (hipGetLastError() != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "ERI dense-fill launch failed");
-        }
-        if (rc == 0) rc = timer_end(ctx, T_ERI, ev, ctx->eri_flops);
-        if (rc == 0 && hipStreamSynchronize(ctx->stream) != hipSuccess)
-            rc = set_error(ctx, MYQC_E_HIP, "ERI dense fill failed");
-    }
-    for (int c = 0; c < 6; ++c) dfree((void **)&ctx->cls[c].d_cum);
-    for (int c = 0; c < 6; ++c) ctx->cls[c] = saved[c];
-    ctx->have_eri = had;
-    ctx->n_stored = saved_stored;
-    ctx->n_quartets = saved_quartets;
-    ctx->eri_flops = saved_flops;
-    return rc;
 }
 
 }  // namespace myqc
@@ -869,15 +812,23 @@ extern "C" int myqc_set_system(myqc_ctx *ctx, int nnuc, const int *Z, const doub
 extern "C" int myqc_eri_full(myqc_ctx *ctx, double schwarz_tol, double *XX) {
     if (!ctx || !XX) return MYQC_E_ARG;
     if (!ctx->have_system) return set_error(ctx, MYQC_E_STATE, "myqc_eri_full: no system set");
-    const size_t n = ctx->n, n4 = n * n * n * n;
-    double *d_XX = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&d_XX, sizeof(double) * n4));
-    int rc = eri_fill_dense(ctx, schwarz_tol, d_XX);
-    if (rc == 0) {
-        hipError_t e = d2h(ctx, XX, d_XX, sizeof(double) * n4);
-        if (e != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "myqc_eri_full: copy failed: %s", hipGetErrorString(e));
+    const size_t n = ctx->n, n4 = n * n * n * n, bytes = sizeof(double) * n4;
+    // the context's work buffer, unless the array is too large to keep
+    double *own = nullptr, *&d_XX = bytes <= kKeepWork ? ctx->d_xwork : own;
+    MYQC_CHECK(dalloc(ctx, (void **)&d_XX, bytes));
+    int rc = 0;
+    {
+        DenseSource src(ctx);
+        rc = src.open(schwarz_tol);
+        if (rc == 0) rc = src.expand_full(d_XX);
+        if (rc == 0) {
+            hipError_t e = d2h(ctx, XX, d_XX, bytes);
+            if (e != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "myqc_eri_full: copy failed: %s", hipGetErrorString(e));
+        } else {
+            (void)hipStreamSynchronize(ctx->stream);   // nothing in flight when the store is given back
+        }
     }
-    dfree((void **)&d_XX);
+    dfree((void **)&own);
     return rc;
 }
 

@@ -18,7 +18,7 @@
 // intermediate L never leaves the registers.
 #include <cstdint>
 
-#include "context.h"
+#include "dense.h"
 #include "many.h"
 
 namespace myqc {
@@ -49,7 +49,7 @@ template <int NKS>
 __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int n, const double *__restrict__ Cp,
                                                              const double *__restrict__ Cq,
                                                              const double *__restrict__ XX, double *__restrict__ M,
-                                                             long long nld) {
+                                                             int nld, const int *__restrict__ tri) {
     constexpr int LDX = 4 * NKS + 2;                           // padded column of a tile in LDS
     constexpr int XPT = (16 * 4 * NKS + Q12_THREADS - 1) / Q12_THREADS;   // tile doubles per thread
     __shared__ double sX[2][16 * LDX];
@@ -76,8 +76,8 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
         cf[k] = (u < n && p0 + c < np) ? Cp[u + (size_t)n * (p0 + c)] : 0.0;
     }
     // the work items of this workgroup: (ld, vt) for ld = blockIdx.x + j gridDim.x
-    const long long nitem_ld = (nld - blockIdx.x + gridDim.x - 1) / gridDim.x;
-    const long long nitem = nitem_ld * nvt;
+    const int nitem_ld = (nld - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+    const long long nitem = (long long)nitem_ld * nvt;
     double xr[XPT];
     auto load_tile = [&](long long it) {
         const long long ld = blockIdx.x + (it / nvt) * gridDim.x;
@@ -138,13 +138,14 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
             }
         }
         if (vt == nvt - 1) {
-            // M(p, q, l, d) at p + np (q + nq ld)
+            // M(p, q, l, d) at p + np (q + nq tri(l, d))
+            const long long out = tri[ld];
 #pragma unroll
             for (int s = 0; s < Q12_NAT; ++s) {
 #pragma unroll
                 for (int vv = 0; vv < 4; ++vv) {
                     const int q = q0 + 16 * s + g + 4 * vv, p = p0 + c;
-                    if (p < np && q < nq) M[p + (size_t)np * (q + (size_t)nq * ld)] = macc[s][vv];
+                    if (p < np && q < nq) M[p + (size_t)np * (q + (size_t)nq * out)] = macc[s][vv];
                 }
                 macc[s] = (d4_t){0.0, 0.0, 0.0, 0.0};
             }
@@ -157,7 +158,9 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
 
 // ---------------------------------------------------------------------------
 // Steps 3 and 4: C (m x nb, ldc) = A (m x k, lda) B (k x nb, ldb) for `batch`
-// problems (A += bat sA, C += bat sC; B shared), all column-major FP64.
+// problems (A += bat sA, C += bat sC; B shared), all column-major FP64; with
+// tri, column kk of problem bat's A is block (kk, bat) of a triangular array
+// (A + lda (max (max + 1) / 2 + min)).
 // A workgroup of 4 wavefronts owns 128 rows of one problem (blockIdx.x) and
 // 48 columns (blockIdx.y); each wavefront 2 row tiles x 3 column tiles, as
 // C^T = B^T A^T so that lanes store 16 consecutive rows.  A's fragments are
@@ -170,7 +173,7 @@ constexpr int GF_MT = 2, GF_NT = 3, GF_THREADS = 256;
 __global__ __launch_bounds__(GF_THREADS) void k_gemm_f64(int m, int nb, int k, const double *__restrict__ A,
                                                          long long lda, long long sA, const double *__restrict__ B,
                                                          long long ldb, double *__restrict__ C, long long ldc,
-                                                         long long sC, int tiles_m) {
+                                                         long long sC, int tiles_m, int tri) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
     const long long bat = blockIdx.x / tiles_m;
     const int r0 = (int)(blockIdx.x - bat * tiles_m) * (64 * GF_MT) + 16 * GF_MT * w;
@@ -185,10 +188,11 @@ __global__ __launch_bounds__(GF_THREADS) void k_gemm_f64(int m, int nb, int k, c
     double fa[GF_MT], fb[GF_NT];
     auto load = [&](int k0) {
         const int kk = k0 + g;
+        const long long hi = kk > bat ? kk : bat, ka = tri ? hi * (hi + 1) / 2 + (kk > bat ? bat : kk) : kk;
 #pragma unroll
         for (int i = 0; i < GF_MT; ++i) {
             const int r = r0 + 16 * i + c;
-            fa[i] = (r < m && kk < k) ? A[r + lda * kk] : 0.0;
+            fa[i] = (r < m && kk < k) ? A[r + lda * ka] : 0.0;
         }
 #pragma unroll
         for (int j = 0; j < GF_NT; ++j) {
@@ -221,41 +225,41 @@ __global__ __launch_bounds__(GF_THREADS) void k_gemm_f64(int m, int nb, int k, c
 }
 
 template <int NKS>
-static void launch12(dim3 grid, hipStream_t s, int np, int nq, int n, const double *Cp, const double *Cq,
-                     const double *XX, double *M, long long nld) {
-    k_ao2mo12_f64<NKS><<<grid, Q12_THREADS, 0, s>>>(np, nq, n, Cp, Cq, XX, M, nld);
+static void launch12(dim3 grid, hipStream_t s, const TransformJob &j, int n, const double *XX, int nld,
+                     const int *tri) {
+    k_ao2mo12_f64<NKS><<<grid, Q12_THREADS, 0, s>>>(j.np, j.nq, n, j.Cp, j.Cq, XX, j.M, nld, tri);
 }
 
-// Steps 1+2 in FP64: M (np x nq x n x n) from Cp (n x np), Cq (n x nq), both
-// with leading dimension n, and the dense integrals XX (n^4).
-int ao2mo12_f64(myqc_ctx *ctx, int np, const double *Cp, int nq, const double *Cq, int n, const double *XX,
-                double *M) {
-    if (np <= 0 || nq <= 0 || n <= 0) return set_error(ctx, MYQC_E_ARG, "ao2mo12_f64: np=%d nq=%d n=%d", np, nq, n);
+// Steps 1+2 in FP64 of one job over nblk blocks of XX (n^2 each), block b's
+// result at M's block tri[b].
+int ao2mo12_f64(myqc_ctx *ctx, const TransformJob &j, int n, const double *XX, int nblk, const int *tri) {
+    if (j.np <= 0 || j.nq <= 0 || n <= 0 || nblk <= 0)
+        return set_error(ctx, MYQC_E_ARG, "ao2mo12_f64: np=%d nq=%d n=%d blocks=%d", j.np, j.nq, n, nblk);
     const int nks = (n + 3) / 4;
-    const long long nld = (long long)n * n;
-    const int gy = (np + 16 * Q12_WAVES - 1) / (16 * Q12_WAVES), gz = (nq + 16 * Q12_NAT - 1) / (16 * Q12_NAT);
+    const int gy = (j.np + 16 * Q12_WAVES - 1) / (16 * Q12_WAVES), gz = (j.nq + 16 * Q12_NAT - 1) / (16 * Q12_NAT);
     if (gy > 65535 || gz > 65535) return set_error(ctx, MYQC_E_ARG, "ao2mo12_f64: too many orbitals");
     // one workgroup per CU and orbital block (256 CUs), each walking its (l,d) blocks
-    const long long gx = std::min<long long>(nld, std::max(1LL, 256LL / ((long long)gy * gz)));
+    const int gx = (int)std::min<long long>(nblk, std::max(1LL, 256LL / ((long long)gy * gz)));
     const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
     hipStream_t s = ctx->stream;
-    if (nks <= 8) launch12<8>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 16) launch12<16>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 24) launch12<24>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 32) launch12<32>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 48) launch12<48>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 64) launch12<64>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 80) launch12<80>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
-    else if (nks <= 100) launch12<100>(grid, s, np, nq, n, Cp, Cq, XX, M, nld);
+    if (nks <= 8) launch12<8>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 16) launch12<16>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 24) launch12<24>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 32) launch12<32>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 48) launch12<48>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 64) launch12<64>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 80) launch12<80>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 100) launch12<100>(grid, s, j, n, XX, nblk, tri);
     else return set_error(ctx, MYQC_E_ARG, "ao2mo12_f64: n=%d above 400", n);
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
 
-// C = A B (FP64), `batch` problems of A (m x k, lda, stride sA) against the
+// C = A B (FP64), `batch` problems of A (m x k, lda, stride sA, or with tri
+// column kk of problem d at block (kk, d) of a triangular array) against the
 // shared B (k x nb, ldb), into C (m x nb, ldc, stride sC).
 int gemm_f64(myqc_ctx *ctx, int m, int nb, int k, const double *A, long long lda, long long sA, const double *B,
-             long long ldb, double *C, long long ldc, long long sC, int batch) {
+             long long ldb, double *C, long long ldc, long long sC, int batch, bool tri) {
     if (m <= 0 || nb <= 0 || k <= 0 || batch <= 0) return set_error(ctx, MYQC_E_ARG, "gemm_f64: empty problem");
     const long long tiles_m = ((long long)m + 64 * GF_MT - 1) / (64 * GF_MT);
     const long long gx = tiles_m * batch;
@@ -263,7 +267,7 @@ int gemm_f64(myqc_ctx *ctx, int m, int nb, int k, const double *A, long long lda
     if (gx > 0x7fffffffLL || tiles_m > 0x7fffffffLL || gy > 65535)
         return set_error(ctx, MYQC_E_ARG, "gemm_f64: grid too large");
     k_gemm_f64<<<dim3((unsigned)gx, (unsigned)gy), GF_THREADS, 0, ctx->stream>>>(m, nb, k, A, lda, sA, B, ldb, C, ldc,
-                                                                                sC, (int)tiles_m);
+                                                                                sC, (int)tiles_m, tri ? 1 : 0);
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }

@@ -1,7 +1,7 @@
 // mfma_gemm.hip -- split-precision (bf16 hi/lo) GEMM on gfx950 MFMA with FP32
 // accumulation, for the ao2mo quarter transforms.
 //
-//   C = op(A) B,   op(A) = A or A^T,   all column-major FP64 in HBM.
+//   C = A B,   all column-major FP64 in HBM.
 //
 // Each FP64 operand element x is split as
 //   hi = bf16(x),   lo = bf16(x - hi)            (16 significant bits in all)
@@ -25,7 +25,7 @@
 // D[4 (l / 16) + v][l % 16] (checked by the GPU layout test).
 #include <cstdint>
 
-#include "context.h"
+#include "dense.h"
 
 namespace myqc {
 
@@ -59,112 +59,17 @@ __global__ void k_split_rows_t(const double *__restrict__ A, long long lda, int 
     }
 }
 
-// C = A^T B with A's hi/lo planes pre-split (k_split_rows_t) and B (k x n,
-// k-contiguous columns) split on its way into LDS with 16-byte vector loads;
-// the next k-step's B values are loaded into registers while this step's
-// MFMAs run.  Tiling and accumulation as described at the top of this file.
-__global__ __launch_bounds__(256) void k_gemm_bf16x3_tn(int m, int n, int k, int kp, const uint16_t *__restrict__ Ahi,
-                                                        const uint16_t *__restrict__ Alo, const double *__restrict__ B,
-                                                        long long ldb, double *__restrict__ C, long long ldc,
-                                                        int vec_ok) {
-    __shared__ __attribute__((aligned(16))) uint16_t sAh[GM][GKP], sAl[GM][GKP], sBh[GN][GKP], sBl[GN][GKP];
-    const int m0 = blockIdx.y * GM;
-    const long long n0 = (long long)blockIdx.x * GN;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = (w & 1) * 64, wn = (w >> 1) * 32;
-    const int r16 = lane & 15, q = lane >> 4;
-    // B loader: column j, 8 consecutive k
-    const int bj = t >> 2, bk = (t & 3) * 8;
-    const long long gj = n0 + bj;
-    double nb[8];
-    auto load_b = [&](int k0) {
-        const int gk = k0 + bk;
-        if (vec_ok && gj < n && gk + 8 <= k) {
-            const double2 *p = reinterpret_cast<const double2 *>(B + gk + ldb * gj);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const double2 d = p[v];
-                nb[2 * v] = d.x;
-                nb[2 * v + 1] = d.y;
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) nb[e] = (gj < n && gk + e < k) ? B[gk + e + ldb * gj] : 0.0;
-        }
-    };
-    f32x4 acc[4][2], cor[4][2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            cor[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        }
-    load_b(0);
-    for (int k0 = 0; k0 < k; k0 += GK) {
-        // A planes: 128 rows x 32 k, 16-byte chunks (two per thread per plane)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int id = t + 256 * c, row = id >> 2, ch = (id & 3) * 8;
-            const size_t src = (size_t)(m0 + row) * kp + k0 + ch;
-            *reinterpret_cast<uint4 *>(&sAh[row][ch]) = *reinterpret_cast<const uint4 *>(Ahi + src);
-            *reinterpret_cast<uint4 *>(&sAl[row][ch]) = *reinterpret_cast<const uint4 *>(Alo + src);
-        }
-        // B: split the prefetched values, then start loading the next step's
-        uint32_t h[4], l[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            uint16_t h0, l0, h1, l1;
-            split(nb[2 * e], h0, l0);
-            split(nb[2 * e + 1], h1, l1);
-            h[e] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-            l[e] = (uint32_t)l0 | ((uint32_t)l1 << 16);
-        }
-        *reinterpret_cast<uint4 *>(&sBh[bj][bk]) = make_uint4(h[0], h[1], h[2], h[3]);
-        *reinterpret_cast<uint4 *>(&sBl[bj][bk]) = make_uint4(l[0], l[1], l[2], l[3]);
-        if (k0 + GK < k) load_b(k0 + GK);
-        __syncthreads();
-        bf16x8 bh[2], bl[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            bh[j] = *reinterpret_cast<const bf16x8 *>(&sBh[wn + 16 * j + r16][8 * q]);
-            bl[j] = *reinterpret_cast<const bf16x8 *>(&sBl[wn + 16 * j + r16][8 * q]);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(&sAh[wm + 16 * i + r16][8 * q]);
-            const bf16x8 al = *reinterpret_cast<const bf16x8 *>(&sAl[wm + 16 * i + r16][8 * q]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
-                cor[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[j], cor[i][j], 0, 0, 0);
-                cor[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[j], cor[i][j], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int gi = m0 + wm + 16 * i + 4 * q + v;
-                const long long gjj = n0 + wn + 16 * j + r16;
-                if (gi < m && gjj < n) C[gi + ldc * gjj] = (double)acc[i][j][v] + (double)cor[i][j][v];
-            }
-}
-
 // C = A B for `batch` strided problems with A (m x k, column-major, lda,
 // FP64) split on its way into LDS and B's hi/lo planes pre-split once
-// (k_split_rows_t over B's columns; B is shared by the batch).  A wavefront
+// (k_split_rows_t over B's columns; B is shared by the batch); with tri,
+// column kk of problem bat's A is block (kk, bat) of a triangular array.  A wavefront
 // loads 64 consecutive rows of A at one k (coalesced); the next k-step's A
 // values are loaded into registers while this step's MFMAs run.  Tiling and
 // accumulation as described at the top of this file.
 __global__ __launch_bounds__(256) void k_gemm_bf16x3_nn(int m, int n, int k, int kp, const double *__restrict__ A,
                                                         long long lda, long long sA, const uint16_t *__restrict__ Bhi,
                                                         const uint16_t *__restrict__ Blo, double *__restrict__ C,
-                                                        long long ldc, long long sC, long long tilesN) {
+                                                        long long ldc, long long sC, long long tilesN, int tri) {
     __shared__ __attribute__((aligned(16))) uint16_t sAh[GM][GKP], sAl[GM][GKP], sBh[GN][GKP], sBl[GN][GKP];
     const long long bx = blockIdx.x;
     const long long bat = bx / tilesN, tn = bx - bat * tilesN;
@@ -183,7 +88,8 @@ __global__ __launch_bounds__(256) void k_gemm_bf16x3_nn(int m, int n, int k, int
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int gk = k0 + ah + 2 * e;
-            na[e] = (gi < m && gk < k) ? A[gi + lda * gk] : 0.0;
+            const long long hi = gk > bat ? gk : bat, ka = tri ? hi * (hi + 1) / 2 + (gk > bat ? bat : gk) : gk;
+            na[e] = (gi < m && gk < k) ? A[gi + lda * ka] : 0.0;
         }
     };
     // B loader: column bj of the tile, 8 consecutive k
@@ -239,21 +145,22 @@ __global__ __launch_bounds__(256) void k_gemm_bf16x3_nn(int m, int n, int k, int
 }
 
 // Quarter steps 1 and 2 of the transform fused, for one (l,d) block per
-// workgroup (blockIdx.x = l + n d) and a 128-row tile of i (blockIdx.y) and a
+// workgroup (blockIdx.x; its result goes to M's block tri[blockIdx.x]) and a 128-row tile of i (blockIdx.y) and a
 // 64-column tile of a (blockIdx.z), with i over the first orbital block Cp and
 // a over the second, Cq (o and nv below are their widths):
 //   L(i,v) = sum_u Cp(u,i) XX(u,v,l,d),   M(i,a,l,d) = sum_v L(i,v) Cq(v,a)
 // L is formed 32 columns of v at a time in LDS and never leaves the
-// workgroup.  Each step keeps the split arithmetic of k_gemm_bf16x3_tn and
-// k_gemm_bf16x3_nn exactly: L is rounded as the FP64 value acc + cor those
-// kernels would store, then split again, and both k loops run in the same
-// 32-wide order, so M is bitwise the unfused result.  Co: planes of Cp^T
+// workgroup.  Each step keeps the split arithmetic of k_gemm_bf16x3_nn
+// exactly: L is rounded as the FP64 value acc + cor that kernel would store,
+// then split again, and both k loops run in the same 32-wide order, so M is
+// bitwise the unfused result.  Co: planes of Cp^T
 // (k_split_rows_t, rows i, kp), Cv: planes of Cq^T (rows a, kp).
 __global__ __launch_bounds__(256) void k_ao2mo12_bf16x3(int o, int nv, int n, int kp, const uint16_t *__restrict__ Coh,
                                                         const uint16_t *__restrict__ Col,
                                                         const uint16_t *__restrict__ Cvh,
                                                         const uint16_t *__restrict__ Cvl,
-                                                        const double *__restrict__ XX, double *__restrict__ M) {
+                                                        const double *__restrict__ XX, double *__restrict__ M,
+                                                        const int *__restrict__ tri) {
     __shared__ __attribute__((aligned(16))) uint16_t sAh[GM][GKP], sAl[GM][GKP];   // C_occ^T tile (i, u)
     __shared__ __attribute__((aligned(16))) uint16_t sBh[32][GKP], sBl[32][GKP];   // XX tile (v, u)
     __shared__ __attribute__((aligned(16))) uint16_t sLh[GM][GKP], sLl[GM][GKP];   // L slice (i, v)
@@ -363,7 +270,8 @@ __global__ __launch_bounds__(256) void k_ao2mo12_bf16x3(int o, int nv, int n, in
         }
         __syncthreads();   // sL and sV are refilled by the next slice
     }
-    // M(i, a, l, d) at i + o (a + nv (l + n d))
+    // M(i, a, l, d) at i + o (a + nv tri(l, d))
+    const long long out = tri[ld];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -372,63 +280,73 @@ __global__ __launch_bounds__(256) void k_ao2mo12_bf16x3(int o, int nv, int n, in
             for (int vv = 0; vv < 4; ++vv) {
                 const int gi = i0 + wr + 16 * i + 4 * q + vv, ga = a0 + 16 * j + r16;
                 if (gi < o && ga < nv)
-                    M[gi + (long long)o * (ga + (long long)nv * ld)] = (double)accM[i][j][vv] + (double)corM[i][j][vv];
+                    M[gi + (long long)o * (ga + (long long)nv * out)] = (double)accM[i][j][vv] + (double)corM[i][j][vv];
             }
 }
 
-// Quarter steps 1 and 2 of the transform in split-bf16 over two column
-// blocks of orbitals: M (np x nq x n x n), M(p,q,l,d) = sum_uv Cp(u,p) Cq(v,q)
-// XX(u,v,l,d), from Cp (n x np) and Cq (n x nq), both with leading dimension n,
-// and the dense integrals XX (n^4).
-int ao2mo12_bf16x3(myqc_ctx *ctx, int np, const double *Cp, int nq, const double *Cq, int n, const double *XX,
-                   double *M) {
-    if (np <= 0 || nq <= 0) return set_error(ctx, MYQC_E_ARG, "ao2mo12_bf16x3: np=%d nq=%d", np, nq);
-    const int gy = (np + GM - 1) / GM, gz = (nq + 63) / 64;
-    const long long nld = (long long)n * n;
-    if (nld > 0x7fffffffLL || gy > 65535 || gz > 65535) return set_error(ctx, MYQC_E_ARG, "ao2mo12_bf16x3: too large");
-    const int kp = ((n + GK - 1) / GK) * GK;
-    const size_t po = (size_t)gy * GM * kp, pv = (size_t)gz * 64 * kp;
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_planes, sizeof(uint16_t) * 2 * (po + pv)));
-    uint16_t *coh = ctx->d_planes, *col = coh + po, *cvh = col + po, *cvl = cvh + pv;
-    k_split_rows_t<<<256, 256, 0, ctx->stream>>>(Cp, n, np, n, gy * GM, kp, coh, col);
-    k_split_rows_t<<<256, 256, 0, ctx->stream>>>(Cq, n, nq, n, gz * 64, kp, cvh, cvl);
-    k_ao2mo12_bf16x3<<<dim3((unsigned)nld, (unsigned)gy, (unsigned)gz), 256, 0, ctx->stream>>>(np, nq, n, kp, coh, col,
-                                                                                             cvh, cvl, XX, M);
+// planes of one job's orbital blocks within ctx->d_planes
+struct JobPlanes {
+    int gy, gz, kp;
+    size_t po, pv;   // values per plane of Cp^T and Cq^T
+    JobPlanes(const TransformJob &j, int n)
+        : gy((j.np + GM - 1) / GM), gz((j.nq + 63) / 64), kp(((n + GK - 1) / GK) * GK), po((size_t)gy * GM * kp),
+          pv((size_t)gz * 64 * kp) {}
+    size_t values() const { return 2 * (po + pv); }
+};
+
+// The hi/lo planes of every job's Cp and Cq, one job after another in
+// ctx->d_planes, for the ao2mo12_bf16x3 calls that follow.
+int bf16x3_planes(myqc_ctx *ctx, const TransformJob *jobs, int njobs, int n) {
+    size_t total = 0;
+    for (int j = 0; j < njobs; ++j) total += JobPlanes(jobs[j], n).values();
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_planes, sizeof(uint16_t) * total));
+    uint16_t *at = ctx->d_planes;
+    for (int j = 0; j < njobs; ++j) {
+        const JobPlanes p(jobs[j], n);
+        k_split_rows_t<<<256, 256, 0, ctx->stream>>>(jobs[j].Cp, n, jobs[j].np, n, p.gy * GM, p.kp, at, at + p.po);
+        k_split_rows_t<<<256, 256, 0, ctx->stream>>>(jobs[j].Cq, n, jobs[j].nq, n, p.gz * 64, p.kp, at + 2 * p.po,
+                                                     at + 2 * p.po + p.pv);
+        at += p.values();
+    }
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
 
-// C (m x n, ldc) = op(A) (m x k) * B (k x n, ldb) for `batch` strided
-// problems; FP64 in and out, split-bf16 MFMA products inside.  The transposed
-// single problem (the first quarter transform: a small A against a large,
-// k-contiguous B) pre-splits A once.
-int gemm_bf16x3(myqc_ctx *ctx, bool transA, int m, int n, int k, const double *A, int lda, long long strideA,
-                const double *B, int ldb, long long strideB, double *C, int ldc, long long strideC, int batch) {
+// Quarter steps 1 and 2 in split-bf16 of one of the jobs whose planes
+// bf16x3_planes laid out, over nblk blocks of XX (n^2 each), block b's result
+// at M's block tri[b].
+int ao2mo12_bf16x3(myqc_ctx *ctx, const TransformJob *jobs, int njobs, int job, int n, const double *XX, int nblk,
+                   const int *tri) {
+    const TransformJob &j = jobs[job];
+    if (j.np <= 0 || j.nq <= 0 || nblk <= 0 || job >= njobs)
+        return set_error(ctx, MYQC_E_ARG, "ao2mo12_bf16x3: np=%d nq=%d blocks=%d", j.np, j.nq, nblk);
+    const uint16_t *at = ctx->d_planes;
+    for (int q = 0; q < job; ++q) at += JobPlanes(jobs[q], n).values();
+    const JobPlanes p(j, n);
+    if (p.gy > 65535 || p.gz > 65535) return set_error(ctx, MYQC_E_ARG, "ao2mo12_bf16x3: too large");
+    k_ao2mo12_bf16x3<<<dim3((unsigned)nblk, (unsigned)p.gy, (unsigned)p.gz), 256, 0, ctx->stream>>>(
+        j.np, j.nq, n, p.kp, at, at + p.po, at + 2 * p.po, at + 2 * p.po + p.pv, XX, j.M, tri);
+    MYQC_HIP(ctx, hipGetLastError());
+    return 0;
+}
+
+// C (m x n, ldc) = A (m x k) * B (k x n, ldb, shared) for `batch` strided
+// problems (or, with tri, column kk of problem d's A at block (kk, d) of a
+// triangular array); FP64 in and out, split-bf16 MFMA products inside.
+int gemm_bf16x3(myqc_ctx *ctx, int m, int n, int k, const double *A, int lda, long long strideA, const double *B,
+                int ldb, double *C, int ldc, long long strideC, int batch, bool tri) {
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return set_error(ctx, MYQC_E_ARG, "gemm_bf16x3: empty problem");
     const long long tilesN = ((long long)n + GN - 1) / GN;
     const long long gx = tilesN * batch;
     const int gy = (m + GM - 1) / GM;
     if (gx > 0x7fffffffLL || gy > 65535) return set_error(ctx, MYQC_E_ARG, "gemm_bf16x3: grid too large");
-    if (transA && batch != 1) return set_error(ctx, MYQC_E_ARG, "gemm_bf16x3: op(A) = A^T takes one problem");
-    if (transA) {
-        const int mp = gy * GM, kp = ((k + GK - 1) / GK) * GK;
-        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_planes, sizeof(uint16_t) * 2 * (size_t)mp * kp));
-        uint16_t *hi = ctx->d_planes, *lo = ctx->d_planes + (size_t)mp * kp;
-        k_split_rows_t<<<256, 256, 0, ctx->stream>>>(A, lda, m, k, mp, kp, hi, lo);
-        const int vec_ok = (ldb % 2 == 0) && ((reinterpret_cast<uintptr_t>(B) & 15) == 0);
-        k_gemm_bf16x3_tn<<<dim3((unsigned)tilesN, (unsigned)gy), 256, 0, ctx->stream>>>(m, n, k, kp, hi, lo, B, ldb, C,
-                                                                                      ldc, vec_ok);
-        MYQC_HIP(ctx, hipGetLastError());
-        return 0;
-    }
-    // op(A) = A: B (shared by the batch) is split into planes once
-    if (strideB != 0) return set_error(ctx, MYQC_E_ARG, "gemm_bf16x3: B must be shared by the batch");
+    // B is split into planes once
     const int np_ = (int)(tilesN * GN), kp = ((k + GK - 1) / GK) * GK;
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_planes, sizeof(uint16_t) * 2 * (size_t)np_ * kp));
     uint16_t *hi = ctx->d_planes, *lo = ctx->d_planes + (size_t)np_ * kp;
     k_split_rows_t<<<256, 256, 0, ctx->stream>>>(B, ldb, n, k, np_, kp, hi, lo);
     k_gemm_bf16x3_nn<<<dim3((unsigned)gx, (unsigned)gy), 256, 0, ctx->stream>>>(m, n, k, kp, A, lda, strideA, hi, lo, C,
-                                                                                ldc, strideC, tilesN);
+                                                                                ldc, strideC, tilesN, tri ? 1 : 0);
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
