@@ -7,22 +7,18 @@
 
 namespace myqc {
 
-// Function pairs (l, d) expanded by one workgroup: the same element of up to
-// kExpPairs shell pairs of consecutive Schwarz rank.
-constexpr int kExpPairs = 16;
+// One function pair l >= d: its class-sorted shell pair, the element of it,
+// and the block it goes to.
 struct ExpandRec {
-    int pos0, cls, ep, pad;      // first pair (class-sorted position), its class, the element
-    int ld[kExpPairs];           // l + n d of each pair's element, -1: none
-    int blk[kExpPairs];          // its block
+    int pos, ep, l, d, blk;
 };
 
-// A run of records whose blocks fit the work buffer
+// A run of function pairs whose blocks fit the work buffer
 struct ExpandChunk {
-    int rec0, nrec;              // records
-    int blk0, nblk;              // blocks, as a range of the triangular indices below
+    int blk0, nblk;
 };
 
-// The unscreened-or-screened value store at threshold `tol`, opened for
+// The values of the quartets above the Schwarz threshold `tol`, opened for
 // expansion: the context's stored integrals when they were built at that
 // threshold, else a build of its own, which leaves the context's stored
 // integrals as they are.  close() (or the destructor) gives back what the
@@ -47,6 +43,7 @@ class DenseSource {
 
   private:
     int tables(bool full);
+    int launch(const ExpandChunk &c, double *X, int full);
     myqc_ctx *ctx;
     bool opened = false, swapped = false;
     // the context's own store, put aside while another is open
@@ -62,11 +59,10 @@ class DenseSource {
         int ns;
     } saved;
     // device tables (ctx->d_dtab)
-    const int *d_T = nullptr;
     const long long *d_off = nullptr;
-    const int2 *d_range = nullptr;
+    const int *d_range = nullptr, *d_inv = nullptr;
     const ExpandRec *d_rec = nullptr;
-    int nrec = 0, pos1 = 0, pos2 = 0;
+    int nrec = 0, pos[4] = {0, 0, 0, 0}, inv0[3] = {0, 0, 0};
 };
 
 // One product of quarter steps 1 and 2: M(p, q, l d) from the orbital blocks

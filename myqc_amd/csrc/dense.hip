@@ -14,125 +14,142 @@
 
 namespace myqc {
 
+constexpr int kExpParts = 64;   // ranges of u at most (n <= 1500)
 struct ExpandArgs {
     const double *x;
-    const int *T;              // [u + n v]: position of the function pair's shell pair << 4 | element
-    const long long *off;      // [3 pos + ket class]: value offset (element e of ket rank r at off + r + e len)
-    const int2 *range;         // [3 pos + ket class]: its ket ranks [lo, hi)
+    const int *inv;            // per class-sorted pair and element: 2 (u (u + 1) / 2 + v) + (u == v), -1: not kept
+    const long long *off;      // [ket class][pos]: value offset (element e of ket rank r at off + r + e len)
+    const int *range;          // [ket class][pos]: its ket ranks {lo, hi}
     const ExpandRec *rec;
     double *X;
-    int n, pos1, pos2;         // first position of classes 1 and 2
+    int n, nrec;
+    int pos[4];                // first position of each class, and the end
+    int inv0[3];               // first entry of inv of each class
     int full;                  // blocks at l + n d and d + n l
+    int m[kExpParts + 1];      // the ranges of u (blockIdx.y)
 };
 
-// One record's blocks over one 32 x 32 tile of (u, v) and its mirror image
-// (tiles tu >= tv).  A lane owns four (u, v) of the tile; for the record's
-// pairs P in turn it reads the element of (P | Q), Q the shell pair of (u, v),
-// from whichever of the two is the bra.  As P runs over consecutive ranks,
-// the reads from Q's block walk along one cache line; the reads from P's
-// block are spread over it by Q's rank, but all of it is read by the
-// record's other tiles.  Bound by those line fetches from L2: 24 waters,
-// 3.2 GB of blocks in 3.4 ms (before: 20 ms of scattered stores and 0.83
-// ms of clearing).
-__global__ __launch_bounds__(256) void k_expand(ExpandArgs a) {
-    constexpr int G = 4;   // pairs at a time
-    __shared__ double s_t[G][32][33];
-    const ExpandRec &rec = a.rec[blockIdx.x];
-    int tu = 0, rem = blockIdx.y;
-    while (rem > tu) rem -= ++tu;
-    const int tv = rem;   // blockIdx.y = tu (tu + 1) / 2 + tv
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const int n = a.n, cp = rec.cls, ep = rec.ep;
-    const size_t nn = (size_t)n * n;
-    const int base_p = cp == 0 ? 0 : cp == 1 ? a.pos1 : a.pos2;
+// wave-uniform read-only records through scalar loads
+template <typename T>
+using cptr = const __attribute__((address_space(4))) T *;
+
+// The block of one function pair (l, d), element ep of shell pair P, over the
+// u >= v with u in [m0, m1), assembled in LDS and written out as the square.
+//
+// Its values lie in two places: where P is the bra, P's own rows of the
+// store, read along the ket ranks (contiguous); where Q is the bra, one value
+// per (Q, element), at P's rank.  Those single values share their cache lines
+// with the pairs of neighbouring rank, so 32 consecutive pairs (same element)
+// run on one XCD at a time (workgroup b runs on XCD b mod 8), in step, and a
+// line is fetched from memory once for 16 of them.  The scatter into (u, v)
+// order happens in LDS, and the stores are whole columns.
+// Bound by one workgroup's phases in turn (LDS holds one block; two half
+// blocks per CU read P's rows twice: 2.5 ms): 24 waters, 3.2 GB of blocks in
+// 1.8 ms, of which their plain write is 0.7.  Before: 3.4
+// ms with lanes in (u, v) order gathering from both places (0.96 GB fetched
+// per 290 MB chunk), 20.9 ms with the integral kernels storing to the dense
+// array themselves.
+// LDS: VALS values, THREADS threads: 16 KiB for n <= 63, several workgroups
+// per CU; 128 KiB above, n > 180 in several ranges of u.
+template <int VALS, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_expand(ExpandArgs a) {
+    const int m0 = a.m[blockIdx.y], m1 = a.m[blockIdx.y + 1];
+    __shared__ double s_b[VALS];
+    const int b = blockIdx.x, irec = (b & ~255) + (b & 7) * 32 + ((b & 255) >> 3);
+    if (irec >= a.nrec) return;   // (uniform over the workgroup)
+    const cptr<ExpandRec> rec = (cptr<ExpandRec>)(a.rec + irec);
+    const cptr<long long> c_off = (cptr<long long>)a.off;
+    const cptr<int> c_range = (cptr<int>)a.range;
+    const int n = a.n, p = rec->pos, ep = rec->ep, l = rec->l, d = rec->d;
+    const int cp = (p >= a.pos[1]) + (p >= a.pos[2]);
     const int nfp = cp == 0 ? 1 : cp == 1 ? 3 : 9;
-    const int u = tu * 32 + tx;
-    // the lane's four (u, v): position, element and class of Q, and Q's
-    // block for kets of P's class
-    int q[4], eq[4], cq[4], lenq[4], loq[4], hiq[4];
-    long long offq[4];
+    const int rp = p - (cp == 0 ? a.pos[0] : cp == 1 ? a.pos[1] : a.pos[2]);
+    const int t0 = m0 * (m0 + 1) / 2, t1 = m1 * (m1 + 1) / 2, own = l * (l + 1) / 2 + d;
+    const int t = threadIdx.x;
+    for (int i = t; i < t1 - t0; i += THREADS) s_b[i] = 0.0;
+    __syncthreads();
+    // a value of (P | Q) to its place, without the degeneracy weights the
+    // store carries (powers of two)
+    const double w = l == d ? 2.0 : 1.0;
+    auto put = [&](int code, double x) {
+        const int at = code >> 1;
+        if (code < 0 || at < t0 || at >= t1) return;
+        x *= w;
+        if (code & 1) x *= 2.0;
+        if (at == own) x *= 2.0;
+        s_b[at - t0] = x;
+    };
+    // P the bra: kets of its own class from its own rank on, and of the lower
+    // classes; four values per thread in flight
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int v = tv * 32 + ty + 8 * k;
-        const int t = (u < n && v < n) ? a.T[u + n * v] : a.T[0];
-        q[k] = t >> 4;
-        eq[k] = t & 15;
-        cq[k] = (q[k] >= a.pos1) + (q[k] >= a.pos2);
-        const int2 r = a.range[3 * q[k] + cp];
-        loq[k] = r.x;
-        hiq[k] = r.y;
-        lenq[k] = r.y - r.x;
-        offq[k] = a.off[3 * q[k] + cp] + (long long)(eq[k] * nfp + ep) * lenq[k];
-    }
-    for (int h = 0; h < kExpPairs; h += G) {
-        double val[G][4];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            const int ld = rec.ld[h + j];
-            if (ld < 0) continue;   // (uniform over the workgroup)
-            const int p = rec.pos0 + h + j, rp = p - base_p;
-            const int l = ld % n, d = ld / n;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int v = tv * 32 + ty + 8 * k;
-                const int rq = q[k] - (cq[k] == 0 ? 0 : cq[k] == 1 ? a.pos1 : a.pos2);
-                const int nfq = cq[k] == 0 ? 1 : cq[k] == 1 ? 3 : 9;
-                bool ok;
-                long long at;
-                if (cp > cq[k] || (cp == cq[k] && rp <= rq)) {
-                    const int2 r = a.range[3 * p + cq[k]];
-                    ok = rq >= r.x && rq < r.y;
-                    // within one pair only the elements in ascending order are kept
-                    const int e = p == q[k] ? min(ep, eq[k]) * nfq + max(ep, eq[k]) : ep * nfq + eq[k];
-                    at = a.off[3 * p + cq[k]] + rq + (long long)e * (r.y - r.x);
-                } else {
-                    ok = rp >= loq[k] && rp < hiq[k];
-                    at = offq[k] + rp;
-                }
-                double x = ok ? a.x[at] : 0.0;
-                // the degeneracy weights the store carries (powers of two)
-                if (l == d) x *= 2.0;
-                if (u == v) x *= 2.0;
-                if ((u == l && v == d) || (u == d && v == l)) x *= 2.0;
-                val[j][k] = x;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            if (rec.ld[h + j] < 0) continue;
-            double *X = a.X + nn * rec.blk[h + j];
-            const int l = rec.ld[h + j] % n, d = rec.ld[h + j] / n;
-            double *X2 = a.full && l != d ? a.X + nn * ((size_t)d + (size_t)n * l) : nullptr;
+    for (int c = 0; c < 3; ++c) {
+        if (c > cp) break;
+        const int nfq = c == 0 ? 1 : c == 1 ? 3 : 9;
+        const int lo = c_range[2 * ((size_t)a.pos[3] * c + p)], len = c_range[2 * ((size_t)a.pos[3] * c + p) + 1] - lo;
+        const int total = len * nfq;
+        if (total == 0) continue;
+        const double *src = a.x + c_off[(size_t)a.pos[3] * c + p] + lo;
+        const int *inv = a.inv + a.inv0[c] + lo * nfq;
+        const int self = c == cp ? rp - lo : -1;   // the ket that is P itself
+        for (int i0 = t; i0 < total; i0 += 4 * THREADS) {
+            int code[4];
+            double x[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int v = tv * 32 + ty + 8 * k;
-                s_t[j][ty + 8 * k][tx] = val[j][k];
-                if (u >= n || v >= n) continue;
-                X[u + (size_t)n * v] = val[j][k];
-                if (X2) X2[u + (size_t)n * v] = val[j][k];
+                const int i = min(i0 + k * THREADS, total - 1);
+                const int eq = c == 0 ? 0 : i / len, r = i - eq * len;
+                // within one pair only the elements in ascending order are kept
+                const int e = r == self ? min(ep, eq) * nfq + max(ep, eq) : ep * nfq + eq;
+                code[k] = inv[r * nfq + eq];
+                x[k] = src[r + (long long)e * len];
             }
-        }
-        if (tu != tv) {
-            __syncthreads();
 #pragma unroll
-            for (int j = 0; j < G; ++j) {
-                if (rec.ld[h + j] < 0) continue;
-                double *X = a.X + nn * rec.blk[h + j];
-                const int l = rec.ld[h + j] % n, d = rec.ld[h + j] / n;
-                double *X2 = a.full && l != d ? a.X + nn * ((size_t)d + (size_t)n * l) : nullptr;
-                const int v = tv * 32 + tx;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int uu = tu * 32 + ty + 8 * k;
-                    if (uu >= n || v >= n) continue;
-                    const double x = s_t[j][tx][ty + 8 * k];
-                    X[v + (size_t)n * uu] = x;
-                    if (X2) X2[v + (size_t)n * uu] = x;
-                }
-            }
-            __syncthreads();
+            for (int k = 0; k < 4; ++k)
+                if (i0 + k * THREADS < total) put(code[k], x[k]);
         }
     }
+    // Q the bra: the higher classes, and its own class up to the rank before
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (c < cp) continue;
+        constexpr int kQ[3] = {4, 2, 1};   // pairs Q per thread in flight
+        const int nfq = c == 0 ? 1 : c == 1 ? 3 : 9;
+        const int q0 = a.pos[c], q1 = c == cp ? p : a.pos[c + 1];
+        const int *inv = a.inv + a.inv0[c];
+        const long long *off = a.off + (size_t)a.pos[3] * cp;
+        const int2 *range = reinterpret_cast<const int2 *>(a.range) + (size_t)a.pos[3] * cp;
+        for (int qt = q0 + t; qt < q1; qt += kQ[c] * THREADS) {
+            double v[4][9];
+            bool ok[4];
+#pragma unroll
+            for (int k = 0; k < kQ[c]; ++k) {
+                const int q = min(qt + k * THREADS, q1 - 1);
+                const int2 r = range[q];
+                ok[k] = qt + k * THREADS < q1 && rp >= r.x && rp < r.y;
+                const int len = r.y - r.x, at = min(max(rp, r.x), max(r.y - 1, r.x));
+                const double *src = a.x + (len > 0 ? off[q] + at + (long long)ep * len : 0);
+                const long long step = len > 0 ? (long long)nfp * len : 0;
+#pragma unroll
+                for (int e = 0; e < nfq; ++e) v[k][e] = src[e * step];
+            }
+#pragma unroll
+            for (int k = 0; k < kQ[c]; ++k)
+                if (ok[k])
+#pragma unroll
+                    for (int e = 0; e < nfq; ++e) put(inv[(qt + k * THREADS - q0) * nfq + e], v[k][e]);
+        }
+    }
+    __syncthreads();
+    // the square: a wavefront per column v, rows u with max(u, v) in [m0, m1)
+    double *X = a.X + (size_t)n * n * rec->blk;
+    double *X2 = a.full && l != d ? a.X + (size_t)n * n * ((size_t)d + (size_t)n * l) : nullptr;
+    for (int v = t >> 6; v < m1; v += THREADS / 64)
+        for (int u = (v < m0 ? m0 : 0) + (t & 63); u < m1; u += 64) {
+            const int hi = max(u, v), lo = min(u, v);
+            const double x = s_b[hi * (hi + 1) / 2 + lo - t0];
+            X[u + (size_t)n * v] = x;
+            if (X2) X2[u + (size_t)n * v] = x;
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -206,77 +223,58 @@ void DenseSource::close() {
 int DenseSource::tables(bool full) {
     const DigestPlan &pl = ctx->plan;
     const int n = ctx->n, np = (int)ctx->pairs.size();
-    pos1 = (int)ctx->pair_ids[0].size();
-    pos2 = pos1 + (int)ctx->pair_ids[1].size();
-    const int pos0[3] = {0, pos1, pos2};
+    pos[0] = inv0[0] = 0;
+    int ninv = 0;
+    for (int c = 0; c < 3; ++c) {
+        pos[c + 1] = pos[c] + (int)ctx->pair_ids[c].size();
+        inv0[c] = ninv;
+        ninv += (int)ctx->pair_ids[c].size() * dig_ncd(c);
+    }
     std::vector<long long> off(3 * (size_t)np);
-    std::vector<int> range(6 * (size_t)np), T((size_t)n * n), tri;
+    std::vector<int> range(6 * (size_t)np), inv(ninv), tri;
     std::vector<ExpandRec> recs;
-    const size_t nn8 = sizeof(double) * (size_t)n * n;
-    long long most = full ? 1LL << 60 : std::max<long long>(kExpPairs, (long long)(kChunkBytes / nn8));
-    if (!full && most > 256) most -= most % 256;   // whole rounds of a workgroup per CU
-    chunks.clear();
-    ExpandChunk ch{0, 0, 0, 0};
+    recs.reserve((size_t)n * (n + 1) / 2);
+    tri.reserve((size_t)n * (n + 1) / 2);
     for (int c = 0; c < 3; ++c) {
         const auto &ids = ctx->pair_ids[c];
+        const int nf = dig_ncd(c), nb = c == 2 ? 3 : 1;
         for (size_t r = 0; r < ids.size(); ++r) {
-            const int p = ids[r], pos = pos0[c] + (int)r;
+            const int p = ids[r];
+            const size_t q = pos[c] + r;
             for (int k = 0; k < 3; ++k) {
-                off[3 * (size_t)pos + k] = pl.off[3 * (size_t)p + k];
-                range[6 * (size_t)pos + 2 * k] = pl.lo[3 * (size_t)p + k];
-                range[6 * (size_t)pos + 2 * k + 1] = pl.hi[3 * (size_t)p + k];
+                const size_t at = (size_t)np * k + q;
+                off[at] = pl.off[3 * (size_t)p + k];
+                range[2 * at] = pl.lo[3 * (size_t)p + k];
+                range[2 * at + 1] = pl.hi[3 * (size_t)p + k];
             }
-            const ShellPair &sp = ctx->pairs[p];
-            const int na = sp.la ? 3 : 1, nb = sp.lb ? 3 : 1;
-            for (int x = 0; x < na; ++x)
-                for (int y = 0; y < nb; ++y) {
-                    // of a shell with itself only the elements x <= y are kept
-                    const int e = sp.same && x > y ? y * nb + x : x * nb + y;
-                    T[(sp.ao_a + x) + (size_t)n * (sp.ao_b + y)] = pos << 4 | e;
-                    T[(sp.ao_b + y) + (size_t)n * (sp.ao_a + x)] = pos << 4 | e;
-                }
         }
-        // records: element by element over runs of pairs
-        const int nf = c == 0 ? 1 : c == 1 ? 3 : 9, nb = c == 2 ? 3 : 1;
-        for (size_t r0 = 0; r0 < ids.size(); r0 += kExpPairs)
-            for (int e = 0; e < nf; ++e) {
-                ExpandRec rec;
-                rec.pos0 = pos0[c] + (int)r0;
-                rec.cls = c;
-                rec.ep = e;
-                rec.pad = 0;
-                int cnt = 0;
-                for (int j = 0; j < kExpPairs; ++j) {
-                    rec.ld[j] = rec.blk[j] = -1;
-                    if (r0 + j >= ids.size()) continue;
-                    const ShellPair &sp = ctx->pairs[ids[r0 + j]];
-                    const int x = e / nb, y = e % nb;
-                    if (sp.same && x > y) continue;
-                    const int l = std::max(sp.ao_a + x, sp.ao_b + y), d = std::min(sp.ao_a + x, sp.ao_b + y);
-                    rec.ld[j] = l + n * d;
-                    ++cnt;
-                }
-                if (cnt == 0) continue;
-                if (ch.nblk + cnt > most) {
-                    chunks.push_back(ch);
-                    ch = ExpandChunk{ch.rec0 + ch.nrec, 0, ch.blk0 + ch.nblk, 0};
-                }
-                for (int j = 0; j < kExpPairs; ++j) {
-                    if (rec.ld[j] < 0) continue;
-                    const int l = rec.ld[j] % n, d = rec.ld[j] / n;
-                    rec.blk[j] = full ? rec.ld[j] : ch.nblk;
-                    tri.push_back(l * (l + 1) / 2 + d);
-                    ++ch.nblk;
-                }
-                ++ch.nrec;
-                recs.push_back(rec);
+        // element by element over the class's pairs: neighbours in rank are
+        // neighbours in the list.  Of a shell with itself only the elements
+        // in ascending order are kept.
+        for (int e = 0; e < nf; ++e)
+            for (size_t r = 0; r < ids.size(); ++r) {
+                const ShellPair &sp = ctx->pairs[ids[r]];
+                const int x = e / nb, y = e % nb, i = sp.ao_a + x, j = sp.ao_b + y;
+                const int l = std::max(i, j), d = std::min(i, j), at = l * (l + 1) / 2 + d;
+                const bool kept = !(sp.same && x > y);
+                inv[inv0[c] + r * nf + e] = kept ? 2 * at + (l == d) : -1;
+                if (!kept) continue;
+                recs.push_back(ExpandRec{pos[c] + (int)r, e, l, d, 0});
+                tri.push_back(at);
             }
     }
-    if (ch.nrec) chunks.push_back(ch);
     nrec = (int)recs.size();
+    // chunks of whole rounds of a workgroup per CU
+    const size_t nn8 = sizeof(double) * (size_t)n * n;
+    int most = full ? nrec : (int)std::min<size_t>(nrec, std::max<size_t>(1, kChunkBytes / nn8));
+    if (most > 256 && most < nrec) most -= most % 256;
+    chunks.clear();
+    for (int r = 0; r < nrec; r += most) chunks.push_back(ExpandChunk{r, std::min(most, nrec - r)});
+    for (int r = 0; r < nrec; ++r) recs[r].blk = full ? recs[r].l + n * recs[r].d : r % most;
     const size_t b_off = sizeof(long long) * off.size(), b_range = sizeof(int) * range.size(),
-                 b_rec = sizeof(ExpandRec) * recs.size(), b_T = sizeof(int) * T.size(), b_tri = sizeof(int) * tri.size();
-    std::vector<unsigned char> h(b_off + b_range + b_rec + b_T + b_tri);
+                 b_rec = sizeof(ExpandRec) * recs.size(), b_inv = sizeof(int) * inv.size(),
+                 b_tri = sizeof(int) * tri.size();
+    std::vector<unsigned char> h(b_off + b_range + b_rec + b_inv + b_tri);
     unsigned char *w = h.data();
     auto put = [&](const void *src, size_t b) {
         memcpy(w, src, b);
@@ -285,43 +283,59 @@ int DenseSource::tables(bool full) {
     put(off.data(), b_off);
     put(range.data(), b_range);
     put(recs.data(), b_rec);
-    put(T.data(), b_T);
+    put(inv.data(), b_inv);
     put(tri.data(), b_tri);
     MYQC_CHECK(dalloc(ctx, &ctx->d_dtab, h.size()));
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_dtab, h.data(), h.size(), hipMemcpyHostToDevice, ctx->stream));
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));   // (h goes out of scope)
     const unsigned char *dev = static_cast<const unsigned char *>(ctx->d_dtab);
     d_off = reinterpret_cast<const long long *>(dev);
-    d_range = reinterpret_cast<const int2 *>(dev + b_off);
+    d_range = reinterpret_cast<const int *>(dev + b_off);
     d_rec = reinterpret_cast<const ExpandRec *>(dev + b_off + b_range);
-    d_T = reinterpret_cast<const int *>(dev + b_off + b_range + b_rec);
-    d_tri = reinterpret_cast<const int *>(dev + b_off + b_range + b_rec + b_T);
+    d_inv = reinterpret_cast<const int *>(dev + b_off + b_range + b_rec);
+    d_tri = reinterpret_cast<const int *>(dev + b_off + b_range + b_rec + b_inv);
     return 0;
 }
 
 int DenseSource::plan_chunks() { return tables(false); }
 
 size_t DenseSource::chunk_bytes() const {
-    size_t most = 1;
-    for (const auto &c : chunks) most = std::max(most, (size_t)c.nblk);
-    return sizeof(double) * (size_t)ctx->n * ctx->n * most;
+    return chunks.empty() ? 0 : sizeof(double) * (size_t)ctx->n * ctx->n * chunks[0].nblk;
 }
 
-int DenseSource::expand(const ExpandChunk &c, double *X) {
-    const int tiles = (ctx->n + 31) / 32;
-    ExpandArgs a{ctx->d_x64, d_T, d_off, d_range, d_rec + c.rec0, X, ctx->n, pos1, pos2, 0};
-    k_expand<<<dim3((unsigned)c.nrec, (unsigned)(tiles * (tiles + 1) / 2)), 256, 0, ctx->stream>>>(a);
+int DenseSource::launch(const ExpandChunk &c, double *X, int full) {
+    const int n = ctx->n;
+    ExpandArgs a{ctx->d_x64, d_inv, d_off, d_range, d_rec + c.blk0, X, n, c.nblk, {pos[0], pos[1], pos[2], pos[3]},
+                 {inv0[0], inv0[1], inv0[2]}, full, {}};
+    const unsigned grid = (unsigned)((c.nblk + 255) / 256 * 256);
+    constexpr int kSmall = 2048, kLarge = 16384, kLT = 1024;
+    const int tri = n * (n + 1) / 2;
+    if (tri <= kSmall) {
+        a.m[1] = n;
+        k_expand<kSmall, 256><<<grid, 256, 0, ctx->stream>>>(a);
+    } else {
+        // ranges of u of about equal size
+        int parts = 0, m = 0;
+        const int want = (tri + kLarge - 1) / kLarge;
+        for (; m < n && parts < kExpParts; ++parts) {
+            const int t0 = m * (m + 1) / 2;
+            const long long goal = std::min<long long>((long long)tri * (parts + 1) / want, (long long)t0 + kLarge);
+            while (m < n && (long long)(m + 1) * (m + 2) / 2 <= goal) ++m;
+            a.m[parts + 1] = m;
+            if (m * (m + 1) / 2 == t0) return set_error(ctx, MYQC_E_ARG, "dense integrals: n=%d too large", n);
+        }
+        if (m < n) return set_error(ctx, MYQC_E_ARG, "dense integrals: n=%d too large", n);
+        k_expand<kLarge, kLT><<<dim3(grid, (unsigned)parts), kLT, 0, ctx->stream>>>(a);
+    }
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
+
+int DenseSource::expand(const ExpandChunk &c, double *X) { return launch(c, X, 0); }
 
 int DenseSource::expand_full(double *XX) {
     MYQC_CHECK(tables(true));
-    const int tiles = (ctx->n + 31) / 32;
-    ExpandArgs a{ctx->d_x64, d_T, d_off, d_range, d_rec, XX, ctx->n, pos1, pos2, 1};
-    k_expand<<<dim3((unsigned)nrec, (unsigned)(tiles * (tiles + 1) / 2)), 256, 0, ctx->stream>>>(a);
-    MYQC_HIP(ctx, hipGetLastError());
-    return 0;
+    return launch(ExpandChunk{0, nrec}, XX, 1);
 }
 
 }  // namespace myqc

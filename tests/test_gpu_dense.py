@@ -40,6 +40,31 @@ def test_dense_integrals_at_tile_edges(ctx, Z, xyz):
     assert np.max(np.abs(XX - O.eri_full(O.System(Z, x, basis, ftab)))) <= 1e-10
 
 
+def test_blocks_in_several_ranges(ctx):
+    """27 waters (n = 189): a block no longer fits one workgroup's LDS.  The
+    transform's (ia|jb) for orbitals that are single functions are the
+    integrals themselves, compared with the Fock build of one density
+    element, G(j,b) for D at (i,a).  Tolerance 1e-10 as above."""
+    Z, x = M.water_cluster(27, 5, 10.6)
+    xyz = M.to_bohr(Z, x)
+    ctx.set_system(Z, xyz)
+    n = ctx.n
+    assert n == 189
+    perm = np.random.default_rng(6).permutation(n)
+    C, o = np.eye(n)[:, perm], 4
+    ctx.eri_build(1e-13)
+    t = ctx.ao2mo(C, o)                            # (ia|jb), i, j of the first four functions of perm
+    for i in range(o):
+        for a in (0, 57, 180):
+            D = np.zeros((n, n))
+            D[perm[i], perm[o + a]] = D[perm[o + a], perm[i]] = 0.5
+            J = ctx.fock_G_uhf(D, D)[0]          # 2 J[D] - K[D]
+            K = -ctx.fock_G_uhf(D, -D)[0]          # K[D]
+            Jd = (J + K) / 2
+            want = Jd[np.ix_(perm[:o], perm[o:])]
+            assert np.max(np.abs(t[i, a] - want)) <= 1e-10
+
+
 def test_dense_call_keeps_the_stored_integrals(ctx):
     Z, x = M.water_cluster(5, 3, 8.0)
     xyz = M.to_bohr(Z, x)
