@@ -162,66 +162,108 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
 // tri, column kk of problem bat's A is block (kk, bat) of a triangular array
 // (A + lda (max (max + 1) / 2 + min)).
 // A workgroup of 4 wavefronts owns 128 rows of one problem (blockIdx.x) and
-// 48 columns (blockIdx.y); each wavefront 2 row tiles x 3 column tiles, as
-// C^T = B^T A^T so that lanes store 16 consecutive rows.  A's fragments are
-// 16 consecutive rows at 4 k each (coalesced), B's come from L1/L2 (B is a
-// small block of orbital coefficients); the next k-step's fragments are
-// loaded while this one's MFMAs run.
+// 16 NT columns (blockIdx.y), NT chosen so that the columns are covered with
+// the fewest tiles (all of them up to 128: A, the large operand, is then read
+// once); each wavefront 32 rows x NT column tiles, as C^T = B^T A^T so that
+// lanes store 16 consecutive rows.  k goes through LDS in slices of 16,
+// double-buffered, the next slice's loads in flight during this slice's
+// 8 NT MFMAs.  LDS: A as [k][row], rows of 144 doubles (the two k's of a
+// half-wavefront's read fall in distinct banks), B as [column][k], columns of
+// 18 (its 16 columns likewise).
+// Bound by the matrix cores at about half their rate, the rest the issue of
+// loads and LDS traffic in between: 24 waters, step 3 (5760 x 168 x 120, 168
+// problems) 0.98 ms, 40 TFLOP/s, and step 4 0.31 ms; with 16 rows per
+// wavefront 1.28 and 0.34, and slices of 8 1.49; with fragments loaded
+// straight from memory one k-step ahead and 48 columns per workgroup (A read
+// three times) 1.56 and 0.41.
 // ---------------------------------------------------------------------------
-constexpr int GF_MT = 2, GF_NT = 3, GF_THREADS = 256;
+constexpr int GF_RT = 2, GF_M = 64 * GF_RT, GF_K = 16, GF_THREADS = 256, GF_NT = 8;
 
+template <int NT>
 __global__ __launch_bounds__(GF_THREADS) void k_gemm_f64(int m, int nb, int k, const double *__restrict__ A,
                                                          long long lda, long long sA, const double *__restrict__ B,
                                                          long long ldb, double *__restrict__ C, long long ldc,
                                                          long long sC, int tiles_m, int tri) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
-    const long long bat = blockIdx.x / tiles_m;
-    const int r0 = (int)(blockIdx.x - bat * tiles_m) * (64 * GF_MT) + 16 * GF_MT * w;
-    const int j0 = blockIdx.y * (16 * GF_NT);
+    constexpr int LA = GF_M + 16, LB = GF_K + 2;
+    __shared__ double s_a[2][GF_K * LA], s_b[2][16 * NT * LB];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, g = lane >> 4, c = lane & 15;
+    const int bat = blockIdx.x / tiles_m;
+    const int r0 = (int)(blockIdx.x - bat * tiles_m) * GF_M, j0 = blockIdx.y * (16 * NT);
     A += bat * sA;
+    int ar[GF_RT];
+#pragma unroll
+    for (int x = 0; x < GF_RT; ++x) ar[x] = min(r0 + (t & 63) + 64 * x, m - 1);
     C += bat * sC;
-    d4_t acc[GF_MT][GF_NT];
+    // the thread's share of a slice: A row t & 63 at k = (t >> 6) + 4 q;
+    // B k = t & 15 of column (t >> 4) + 16 q.  Rows and columns past the end
+    // repeat the last one (their results are not stored); k's past the end are
+    // zero on both sides.
+    const int ak = t >> 6, bk = t & 15;
+    const double *pB[NT];
 #pragma unroll
-    for (int i = 0; i < GF_MT; ++i)
-#pragma unroll
-        for (int j = 0; j < GF_NT; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
-    double fa[GF_MT], fb[GF_NT];
+    for (int q = 0; q < NT; ++q) pB[q] = B + ldb * min(j0 + (t >> 4) + 16 * q, nb - 1);
+    double pa[4][GF_RT], pb[NT];
     auto load = [&](int k0) {
-        const int kk = k0 + g;
-        const long long hi = kk > bat ? kk : bat, ka = tri ? hi * (hi + 1) / 2 + (kk > bat ? bat : kk) : kk;
 #pragma unroll
-        for (int i = 0; i < GF_MT; ++i) {
-            const int r = r0 + 16 * i + c;
-            fa[i] = (r < m && kk < k) ? A[r + lda * ka] : 0.0;
+        for (int q = 0; q < 4; ++q) {
+            const int kk = min(k0 + ak + 4 * q, k - 1);
+            const int hi = max(kk, bat);
+            const unsigned ka = tri ? hi * (hi + 1) / 2 + min(kk, bat) : kk;
+            const double *col = A + (size_t)ka * (unsigned)lda;
+#pragma unroll
+            for (int x = 0; x < GF_RT; ++x) {
+                const double v = col[ar[x]];
+                pa[q][x] = k0 + ak + 4 * q < k ? v : 0.0;
+            }
         }
+        const int kk = min(k0 + bk, k - 1);
 #pragma unroll
-        for (int j = 0; j < GF_NT; ++j) {
-            const int col = j0 + 16 * j + c;
-            fb[j] = (col < nb && kk < k) ? B[kk + ldb * col] : 0.0;
+        for (int q = 0; q < NT; ++q) {
+            const double x = pB[q][kk];
+            pb[q] = k0 + bk < k ? x : 0.0;
         }
     };
+    d4_t acc[GF_RT][NT];
+#pragma unroll
+    for (int x = 0; x < GF_RT; ++x)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[x][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
     load(0);
-    for (int k0 = 0; k0 < k; k0 += 4) {
-        double a[GF_MT], b[GF_NT];
+    int buf = 0;
+    for (int k0 = 0; k0 < k; k0 += GF_K, buf ^= 1) {
 #pragma unroll
-        for (int i = 0; i < GF_MT; ++i) a[i] = fa[i];
+        for (int q = 0; q < 4; ++q) 
 #pragma unroll
-        for (int j = 0; j < GF_NT; ++j) b[j] = fb[j];
-        if (k0 + 4 < k) load(k0 + 4);
+            for (int x = 0; x < GF_RT; ++x) s_a[buf][((t >> 6) + 4 * q) * LA + (t & 63) + 64 * x] = pa[q][x];
 #pragma unroll
-        for (int i = 0; i < GF_MT; ++i)
+        for (int q = 0; q < NT; ++q) s_b[buf][((t >> 4) + 16 * q) * LB + bk] = pb[q];
+        __syncthreads();
+        if (k0 + GF_K < k) load(k0 + GF_K);
 #pragma unroll
-            for (int j = 0; j < GF_NT; ++j) acc[i][j] = mfma16x16x4(b[j], a[i], acc[i][j]);
+        for (int ks = 0; ks < GF_K; ks += 4) {
+            double fa[GF_RT];
+#pragma unroll
+            for (int x = 0; x < GF_RT; ++x) fa[x] = s_a[buf][(ks + g) * LA + 16 * (GF_RT * w + x) + c];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const double fb = s_b[buf][(16 * j + c) * LB + ks + g];
+#pragma unroll
+                for (int x = 0; x < GF_RT; ++x) acc[x][j] = mfma16x16x4(fb, fa[x], acc[x][j]);
+            }
+        }
     }
 #pragma unroll
-    for (int i = 0; i < GF_MT; ++i)
+    for (int x = 0; x < GF_RT; ++x) {
+        const int r = r0 + 16 * (GF_RT * w + x) + c;
+        if (r >= m) continue;
 #pragma unroll
-        for (int j = 0; j < GF_NT; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int vv = 0; vv < 4; ++vv) {
-                const int r = r0 + 16 * i + c, col = j0 + 16 * j + g + 4 * vv;
-                if (r < m && col < nb) C[r + ldc * col] = acc[i][j][vv];
+                const int col = j0 + 16 * j + g + 4 * vv;
+                if (col < nb) C[r + ldc * col] = acc[x][j][vv];
             }
+    }
 }
 
 template <int NKS>
@@ -261,13 +303,27 @@ int ao2mo12_f64(myqc_ctx *ctx, const TransformJob &j, int n, const double *XX, i
 int gemm_f64(myqc_ctx *ctx, int m, int nb, int k, const double *A, long long lda, long long sA, const double *B,
              long long ldb, double *C, long long ldc, long long sC, int batch, bool tri) {
     if (m <= 0 || nb <= 0 || k <= 0 || batch <= 0) return set_error(ctx, MYQC_E_ARG, "gemm_f64: empty problem");
-    const long long tiles_m = ((long long)m + 64 * GF_MT - 1) / (64 * GF_MT);
+    const long long tiles_m = ((long long)m + GF_M - 1) / GF_M;
     const long long gx = tiles_m * batch;
-    const int gy = (nb + 16 * GF_NT - 1) / (16 * GF_NT);
+    if (lda > 0xffffffffLL) return set_error(ctx, MYQC_E_ARG, "gemm_f64: leading dimension too large");
+    // column tiles, in the fewest blocks of at most GF_NT, equally filled
+    const int ct = (nb + 15) / 16, gy = (ct + GF_NT - 1) / GF_NT, nt = (ct + gy - 1) / gy;
     if (gx > 0x7fffffffLL || tiles_m > 0x7fffffffLL || gy > 65535)
         return set_error(ctx, MYQC_E_ARG, "gemm_f64: grid too large");
-    k_gemm_f64<<<dim3((unsigned)gx, (unsigned)gy), GF_THREADS, 0, ctx->stream>>>(m, nb, k, A, lda, sA, B, ldb, C, ldc,
-                                                                                sC, (int)tiles_m, tri ? 1 : 0);
+    const dim3 grid((unsigned)gx, (unsigned)gy);
+    auto run = [&](auto kern) {
+        kern<<<grid, GF_THREADS, 0, ctx->stream>>>(m, nb, k, A, lda, sA, B, ldb, C, ldc, sC, (int)tiles_m, tri ? 1 : 0);
+    };
+    switch (nt) {
+        case 1: run(k_gemm_f64<1>); break;
+        case 2: run(k_gemm_f64<2>); break;
+        case 3: run(k_gemm_f64<3>); break;
+        case 4: run(k_gemm_f64<4>); break;
+        case 5: run(k_gemm_f64<5>); break;
+        case 6: run(k_gemm_f64<6>); break;
+        case 7: run(k_gemm_f64<7>); break;
+        default: run(k_gemm_f64<8>); break;
+    }
     MYQC_HIP(ctx, hipGetLastError());
     return 0;
 }
