@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void k_mp2_fold(const double *__restrict__ par
 // XX, and so M, is symmetric in (l,d): only l >= d is formed, M's block at
 // l (l + 1) / 2 + d (np x nq x n (n + 1) / 2 in all).  The blocks of XX are
 // expanded from the stored integrals a buffer's worth at a time.  24 waters,
-// FP64: 4.8 ms for the expansion and both steps (all n^2 blocks of a
+// FP64: 4.3 ms for the expansion and both steps (all n^2 blocks of a
 // dense XX of 6.4 GB: 5.6 ms, and 20.9 to fill it).
 static int transform12(myqc_ctx *ctx, DenseSource &src, const TransformJob *jobs, int njobs, int precision) {
     const int n = ctx->n;

@@ -39,9 +39,12 @@ __device__ __forceinline__ d4_t mfma16x16x4(double a, double b, d4_t c) {
 // each, v tiles of 16 columns: the tile X(:, v0..v0+15 | l,d) is 16 n
 // contiguous doubles, copied into LDS (double-buffered, the next tile's loads
 // in flight during this tile's MFMAs) and shared by the 8 wavefronts.  Per v
-// tile a wavefront runs NKS MFMAs of step 1 (two accumulators over even and
-// odd k-steps) and 4 NAT of step 2; after the last v tile of an (l,d) block it
-// stores M^T and clears the accumulators.
+// tile a wavefront runs NKS MFMAs of step 1 (four accumulators in turn) and
+// 4 NAT of step 2; after the last v tile of an (l,d) block it stores M^T and
+// clears the accumulators.  Bound by the matrix cores, busy 70 % of the time:
+// 24 waters, 14196 blocks, 2.53 ms, 49 TFLOP/s.  (3.04 ms with the next tile's
+// loads under branches, for which the compiler waited before the first MFMA,
+// and NKS in steps of 8 to 20: n = 168 ran 48 of its 42 k-steps.)
 // ---------------------------------------------------------------------------
 constexpr int Q12_WAVES = 8, Q12_THREADS = 64 * Q12_WAVES, Q12_NAT = 3;
 
@@ -75,43 +78,49 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
         const int u = 4 * k + g;
         cf[k] = (u < n && p0 + c < np) ? Cp[u + (size_t)n * (p0 + c)] : 0.0;
     }
-    // the work items of this workgroup: (ld, vt) for ld = blockIdx.x + j gridDim.x
-    const int nitem_ld = (nld - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
-    const long long nitem = (long long)nitem_ld * nvt;
+    // the work items of this workgroup: (ld, vt) for ld = blockIdx.x + j gridDim.x,
+    // walked with counters (no divisions in the loop, nor in the copy to LDS:
+    // the places of a thread's elements are the same for every tile)
+    int lofs[XPT];
+#pragma unroll
+    for (int r = 0; r < XPT; ++r) {
+        const int e = t + r * Q12_THREADS, col = e / n;
+        lofs[r] = e < 16 * n ? col * LDX + (e - col * n) : -1;
+    }
     double xr[XPT];
-    auto load_tile = [&](long long it) {
-        const long long ld = blockIdx.x + (it / nvt) * gridDim.x;
-        const int v0 = (int)(it % nvt) * 16;
-        const double *src = XX + ld * nn + (size_t)v0 * n;
-        const int valid = min(16, n - v0) * n;   // doubles of the tile inside the block
+    auto load_tile = [&](int ld, int vt) {
+        const double *src = XX + (size_t)ld * nn + (size_t)(16 * vt) * n;
+        const int last = min(16, n - 16 * vt) * n - 1;   // of the tile's doubles inside the block
 #pragma unroll
-        for (int r = 0; r < XPT; ++r) {
-            const int e = t + r * Q12_THREADS;
-            xr[r] = e < valid ? src[e] : 0.0;
-        }
+        for (int r = 0; r < XPT; ++r) xr[r] = src[min(t + r * Q12_THREADS, last)];
     };
-    auto store_tile = [&](int buf) {
+    auto store_tile = [&](int buf, int vt) {
+        const int valid = min(16, n - 16 * vt) * n;
 #pragma unroll
-        for (int r = 0; r < XPT; ++r) {
-            const int e = t + r * Q12_THREADS;
-            if (e < 16 * n) {
-                const int col = e / n, u = e - col * n;
-                sX[buf][col * LDX + u] = xr[r];
-            }
-        }
+        for (int r = 0; r < XPT; ++r)
+            if (lofs[r] >= 0) sX[buf][lofs[r]] = t + r * Q12_THREADS < valid ? xr[r] : 0.0;
     };
     d4_t macc[Q12_NAT];
 #pragma unroll
     for (int s = 0; s < Q12_NAT; ++s) macc[s] = (d4_t){0.0, 0.0, 0.0, 0.0};
-    if (nitem > 0) load_tile(0);
+    int ld = blockIdx.x, vt = 0;
+    load_tile(min(ld, nld - 1), 0);
     __syncthreads();   // the zero fill is complete before the first tile lands
-    if (nitem > 0) store_tile(0);
+    store_tile(0, 0);
     __syncthreads();
     int cur = 0;
-    for (long long it = 0; it < nitem; ++it) {
-        if (it + 1 < nitem) load_tile(it + 1);
-        const long long ld = blockIdx.x + (it / nvt) * gridDim.x;
-        const int vt = (int)(it % nvt), v0 = vt * 16;
+    while (ld < nld) {
+        int ld1 = ld, vt1 = vt + 1;
+        if (vt1 == nvt) {
+            vt1 = 0;
+            ld1 += gridDim.x;
+        }
+        // the next tile's loads, issued on every path (this tile's again when
+        // there is no next) and without a branch, so that the wait the
+        // compiler places for them is the one before their copy to LDS
+        const bool more = ld1 < nld;
+        load_tile(more ? ld1 : ld, more ? vt1 : vt);
+        const int v0 = vt * 16;
         // step 1: L^T(v0 + ., p0 + .) over all u, four independent chains
         const double *xs = &sX[cur][c * LDX + g];
         d4_t ac[4];
@@ -150,9 +159,11 @@ __global__ __launch_bounds__(Q12_THREADS) void k_ao2mo12_f64(int np, int nq, int
                 macc[s] = (d4_t){0.0, 0.0, 0.0, 0.0};
             }
         }
-        if (it + 1 < nitem) store_tile(cur ^ 1);
+        if (more) store_tile(cur ^ 1, vt1);
         __syncthreads();
         cur ^= 1;
+        ld = ld1;
+        vt = vt1;
     }
 }
 
@@ -284,13 +295,25 @@ int ao2mo12_f64(myqc_ctx *ctx, const TransformJob &j, int n, const double *XX, i
     const int gx = (int)std::min<long long>(nblk, std::max(1LL, 256LL / ((long long)gy * gz)));
     const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
     hipStream_t s = ctx->stream;
-    if (nks <= 8) launch12<8>(grid, s, j, n, XX, nblk, tri);
+    if (nks <= 4) launch12<4>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 8) launch12<8>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 12) launch12<12>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 16) launch12<16>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 20) launch12<20>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 24) launch12<24>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 28) launch12<28>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 32) launch12<32>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 36) launch12<36>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 40) launch12<40>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 44) launch12<44>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 48) launch12<48>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 52) launch12<52>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 56) launch12<56>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 60) launch12<60>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 64) launch12<64>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 72) launch12<72>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 80) launch12<80>(grid, s, j, n, XX, nblk, tri);
+    else if (nks <= 90) launch12<90>(grid, s, j, n, XX, nblk, tri);
     else if (nks <= 100) launch12<100>(grid, s, j, n, XX, nblk, tri);
     else return set_error(ctx, MYQC_E_ARG, "ao2mo12_f64: n=%d above 400", n);
     MYQC_HIP(ctx, hipGetLastError());
