@@ -19,6 +19,7 @@
 
 #include "context.h"
 #include "many.h"
+#include "scf_small.h"
 
 namespace myqc {
 
@@ -159,7 +160,7 @@ struct ScfBuffers {
         const size_t tiles = (size_t)(nb + 15) / 16;   // purification trace partials: 2 steps x tiles^2 x 2
         MYQC_CHECK(dalloc(ctx, (void **)&sp2t, sizeof(double) * 4 * tiles * tiles));
         MYQC_CHECK(dalloc(ctx, (void **)&part, sizeof(double) * kRedJobs * kRedBlocks));
-        MYQC_CHECK(dalloc(ctx, (void **)&red, sizeof(double) * kRedJobs));
+        MYQC_CHECK(dalloc(ctx, (void **)&red, sizeof(double) * std::max(kRedJobs, kDiisSlots * kDiisSlots)));
         MYQC_CHECK(dalloc(ctx, (void **)&hF, sizeof(double) * nn * kDiis));
         MYQC_CHECK(dalloc(ctx, (void **)&hE, sizeof(double) * nn * kDiis));
         MYQC_CHECK(dalloc(ctx, (void **)&info, sizeof(int)));
@@ -387,6 +388,150 @@ static bool diis_coeffs(const std::vector<double> &B, int m, std::vector<double>
 // core-Hamiltonian guess the shift slows convergence, so it is not used there.
 constexpr double kShift = 0.5, kShiftErr = 1.0;
 
+// The loop below for a system whose dense steps fit one workgroup (n <=
+// kSmallScfN, scf_small.hip): the same iteration, decisions and results, with
+// one launch and one synchronisation per iteration around the Fock build.  The
+// step that follows a Fock build is launched before its convergence is known;
+// when the loop ends (or rebuilds in FP64) there, its density is dropped.
+static int rhf_scf_small(myqc_ctx *ctx, ScfBuffers &b, const double *H, const double *S, int nocc, double e_nuc,
+                         const double *C_guess, const double *D_guess, double e_tol, double d_tol, int max_iter,
+                         int precision, double *energy, double *C_out, double *eig_out, int *iters_out) {
+    const int n = ctx->n, MD = ScfBuffers::kDiis;
+    const size_t nn = (size_t)n * n;
+    static_assert(ScfBuffers::kDiis == SO_OK - SO_B, "DIIS slots");
+    double *pin = static_cast<double *>(ctx->h_pin), *out = pin + kPinBytes / sizeof(double) - SO_COUNT;
+    MYQC_HIP(ctx, hipMemcpyAsync(b.H, H, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
+    MYQC_HIP(ctx, hipMemcpyAsync(b.S, S, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
+    MYQC_CHECK(small_inv_sqrt(ctx, n, b.S, b.X, b.Xi, b.T2, b.P2, out));
+    MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (out[0] != 1.0) MYQC_CHECK(inv_sqrt_eig(ctx, b, n));
+    SmallStep st{};
+    st.n = n;
+    st.nocc = nocc;
+    st.shift_err = kShiftErr;
+    st.shift = (C_guess || D_guess) ? kShift : 0.0;
+    st.H = b.H;
+    st.G = b.G;
+    st.X = b.X;
+    st.hF = b.hF;
+    st.hE = b.hE;
+    st.B = b.red;
+    st.Fx = b.Fx;
+    st.out = out;
+    // the densities in turn: current, previous, next; and the projectors
+    double *D = b.D, *Dp = b.Dn, *Dx = b.T1, *Do = b.Do, *Don = b.Don;
+    // after a step: the eigenvectors' projector where purification found no clean gap
+    auto finish = [&]() -> int {
+        if (nocc == 0 || nocc == n) return 0;
+        ++ctx->scf_purify;
+        ctx->scf_sp2_steps = (int)out[SO_STEPS];
+        if (out[SO_OK] == 1.0) return 0;
+        ++ctx->scf_diag;
+        MYQC_CHECK(small_orbitals(ctx, n, st.Fx, b.X, b.C, b.eig));
+        // (b.C = X U: its occupied columns give D = 2 C C^T, and P = Xi C C^T Xi)
+        MYQC_CHECK(density(ctx, b.C, nocc, Dx, n));
+        MYQC_CHECK(gemm(ctx, NN, NN, n, n, n, 1.0, Dx, n, b.Xi, n, 0.0, b.T2, n));
+        return gemm(ctx, NN, NN, n, n, n, 0.5, b.Xi, n, b.T2, n, 0.0, Don, n);
+    };
+    auto advance = [&]() {
+        double *x = Dp;
+        Dp = D;
+        D = Dx;
+        Dx = x;
+        std::swap(Do, Don);
+    };
+    if (C_guess || D_guess) {
+        if (C_guess) {
+            MYQC_HIP(ctx, hipMemcpyAsync(b.C, C_guess, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
+            MYQC_CHECK(density(ctx, b.C, nocc, D, n));
+        } else {
+            MYQC_HIP(ctx, hipMemcpyAsync(D, D_guess, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
+        }
+        // Do = S^{1/2} D S^{1/2} / 2
+        MYQC_CHECK(gemm(ctx, NN, NN, n, n, n, 1.0, D, n, b.Xi, n, 0.0, b.T2, n));
+        MYQC_CHECK(gemm(ctx, NN, NN, n, n, n, 0.5, b.Xi, n, b.T2, n, 0.0, Do, n));
+    } else {
+        // core Hamiltonian guess (scf.f90:410-512)
+        st.core = 1;
+        st.Don = Don;
+        st.Dnext = Dx;
+        MYQC_CHECK(small_step(ctx, st));
+        MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        MYQC_CHECK(finish());
+        advance();
+        st.core = 0;
+    }
+    int hist = 0, head = 0, since_full = 0, it = 1;
+    double E = 0.0, E_old = 0.0, dE_prev = 1e300, err_prev = 1e300, E32 = 0.0;
+    bool prev64 = false, final_fp64 = false, conv = false, redo = false, redo_next = false;
+    const bool incr = (precision == MYQC_FP32), trace = getenv("MYQC_SCF_TRACE") != nullptr;
+    while (true) {
+        redo = redo_next;
+        redo_next = false;
+        const bool full = !incr || final_fp64 || since_full == 0 || since_full >= 8;
+        if (full) {
+            MYQC_CHECK(digest_G(ctx, D, b.G, MYQC_FP64));
+            since_full = 1;
+        } else {
+            MYQC_CHECK(digest_G(ctx, D, b.G, MYQC_FP32, Dp));
+            ++since_full;
+        }
+        const int hn = std::min(hist + 1, MD);
+        st.head = head;
+        st.hn = hn;
+        st.with_dd = it > 1;
+        st.D = D;
+        st.Dprev = Dp;
+        st.Do = Do;
+        st.Don = Don;
+        st.Dnext = Dx;
+        MYQC_CHECK(small_step(ctx, st));
+        MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        E = 0.5 * (out[SO_DF] + out[SO_DH]) + e_nuc;
+        const double dd = out[SO_DD], err = sqrt(fabs(out[SO_B + head]));
+        if (trace)
+            fprintf(stderr, "[scf] it %2d %s E %.12f dE %.2e max|dD| %.2e |err| %.2e hist %d\n", it,
+                    full ? "fp64" : "fp32", E, fabs(E - E_old), it > 1 ? dd : -1.0, err, hn);
+        if (it > 2 && dE_prev < e_tol && dd < d_tol && err_prev < 100 * d_tol) {
+            if (!incr || (prev64 && full)) {
+                conv = true;
+                break;
+            }
+            if (redo && err < 100 * d_tol && fabs(E - E32) < e_tol) {
+                conv = true;
+                break;
+            }
+            if (!final_fp64) {
+                final_fp64 = true;
+                if (!full) {
+                    E32 = E;
+                    redo_next = true;
+                    continue;
+                }
+            }
+        }
+        if (it > max_iter) break;
+        hist = hn;
+        err_prev = err;
+        dE_prev = fabs(E - E_old);
+        E_old = E;
+        prev64 = full;
+        head = (head + 1) % MD;
+        MYQC_CHECK(finish());
+        advance();
+        ++it;
+    }
+    // orbitals of the plain Fock matrix of the reported density
+    MYQC_CHECK(small_orbitals(ctx, n, b.hF + nn * head, b.X, b.C, b.eig));
+    if (energy) *energy = E;
+    if (C_out) MYQC_HIP(ctx, d2h(ctx, C_out, b.C, sizeof(double) * nn));
+    if (eig_out) MYQC_HIP(ctx, d2h(ctx, eig_out, b.eig, sizeof(double) * n));
+    if (iters_out) *iters_out = it - 1;
+    MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (!conv) return set_error(ctx, MYQC_E_NOCONV, "RHF did not converge in %d iterations", max_iter);
+    return 0;
+}
+
 static int rhf_scf(myqc_ctx *ctx, const double *H, const double *S, int nocc, double e_nuc, const double *C_guess,
                    const double *D_guess, double e_tol, double d_tol, int max_iter, int precision, double *energy,
                    double *C_out, double *eig_out, int *iters_out) {
@@ -396,6 +541,9 @@ static int rhf_scf(myqc_ctx *ctx, const double *H, const double *S, int nocc, do
     if (!ctx->scf) ctx->scf = new ScfBuffers();
     ScfBuffers &b = *ctx->scf;
     MYQC_CHECK(b.ensure(ctx, n));
+    if (n <= kSmallScfN)
+        return rhf_scf_small(ctx, b, H, S, nocc, e_nuc, C_guess, D_guess, e_tol, d_tol, max_iter, precision, energy,
+                             C_out, eig_out, iters_out);
     MYQC_HIP(ctx, hipMemcpyAsync(b.H, H, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
     MYQC_HIP(ctx, hipMemcpyAsync(b.S, S, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
     int ok = 0;
