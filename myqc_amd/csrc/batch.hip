@@ -973,6 +973,21 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
         const std::string why = build_system(nnuc, xyz.data(), si[0], set_alpha + o[0], si, bas + o[2], norb,
                                              basinfo + o[3], shells, mp, mpr, ids);
         if (!why.empty()) return set_error(ctx, MYQC_E_ARG, "myqc_batch_set: molecule %d: %s", m, why.c_str());
+        // kets with similar numbers of primitive pairs above the screen run in
+        // the same wavefronts (of 5 waters, a wavefront executed 0.62 of all
+        // primitive quartets of (ss|ss) in the pairs' own order, 0.39 in this one;
+        // 0.28 survive; 1024 clusters 2.98 -> 2.21 ms): by the primitive pairs
+        // that pass alone halfway to it, then at it
+        {
+            std::vector<int> weight(mp.size());
+            for (size_t q = 0; q < mp.size(); ++q)
+                for (int i = 0; i < mp[q].npp; ++i) {
+                    const double e = mpr[mp[q].pp0 + i].EIJ;
+                    weight[q] += e >= 1e-7 ? 101 : e >= 1e-14 ? 1 : 0;
+                }
+            for (auto &v : ids)
+                std::stable_sort(v.begin(), v.end(), [&](int x, int y) { return weight[x] > weight[y]; });
+        }
         BMol &mol = b.mols[m];
         mol.n = norb;
         mol.nocc = mol_nocc[m];

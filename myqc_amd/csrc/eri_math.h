@@ -361,12 +361,16 @@ MYQC_HD void quartet_prims_f(const ShellPair &bra, const ShellPair &ket, const P
     const double c0 = 2.0 * pow(PI_SP, 2.5);
     // ket primitives outer: a lane's own ket data is loaded once per quartet,
     // and the inner loop reads the bra's primitives, whose addresses the lanes
-    // of a wavefront (one bra pair, consecutive kets) mostly share
+    // of a wavefront (one bra pair, consecutive kets) mostly share.  A pair's
+    // primitives stand with the largest screen factor first (system.h), so a
+    // row ends at the first one screened: a third to a half of the primitive
+    // quartets survive, and testing all of them cost 14 % of the kernels'
+    // time (40 waters 2.33 -> 2.00 ms)
     for (int j = 0; j < ket.npp; ++j) {
         const PrimPair k = kprim(j);
         for (int i = 0; i < bra.npp; ++i) {
             const PrimPair b = ppb[bra.pp0 + i];
-            if (SCREEN && b.EIJ * k.EIJ < 1.0e-14) continue;          // int2e.f90:257
+            if (SCREEN && b.EIJ * k.EIJ < 1.0e-14) break;          // int2e.f90:257; the rest are smaller
             prim_quartet<LA, LB, LC, LD>(b, k, Q, c0, ftT, acc);
         }
     }

@@ -139,20 +139,36 @@ inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int n
             const double *RA = xyz + 3 * sa.center, *RB = xyz + 3 * sb.center;
             const double ab2 = sp.AB[0] * sp.AB[0] + sp.AB[1] * sp.AB[1] + sp.AB[2] * sp.AB[2];
             PrimPair *out = prims.data() + sp.pp0;
-            for (size_t i = 0; i < sa.alpha.size(); ++i)
-                for (size_t j = 0; j < sb.alpha.size(); ++j) {
-                    const double aa = sa.alpha[i], bb = sb.alpha[j], p = aa + bb;
-                    PrimPair &pp = *out++;
-                    pp.p = p;
-                    for (int d = 0; d < 3; ++d) {
-                        pp.P[d] = (aa * RA[d] + bb * RB[d]) / p;
-                        pp.PA[d] = pp.P[d] - RA[d];
-                    }
-                    pp.EIJ = exp(-aa * bb * ab2 / p);       // int2e.f90:223
-                    pp.K = pp.EIJ * sa.coef[i] * sb.coef[j];
-                    pp.beta = bb;
-                    pp.ip = 1.0 / p;
+            // largest screen factor first: the primitive quartets of a shell
+            // quartet that pass the screen are then a prefix of each row
+            const int na = (int)sa.alpha.size(), nb = (int)sb.alpha.size();
+            double eij[36];
+            int order[36];
+            for (int x = 0; x < na * nb; ++x) {
+                const double aa = sa.alpha[x / nb], bb = sb.alpha[x % nb];
+                const double e = exp(-aa * bb * ab2 / (aa + bb));       // int2e.f90:223
+                int y = x;
+                for (; y > 0 && eij[y - 1] < e; --y) {
+                    eij[y] = eij[y - 1];
+                    order[y] = order[y - 1];
                 }
+                eij[y] = e;
+                order[y] = x;
+            }
+            for (int x = 0; x < na * nb; ++x) {
+                const int i = order[x] / nb, j = order[x] % nb;
+                const double aa = sa.alpha[i], bb = sb.alpha[j], p = aa + bb;
+                PrimPair &pp = *out++;
+                pp.p = p;
+                for (int d = 0; d < 3; ++d) {
+                    pp.P[d] = (aa * RA[d] + bb * RB[d]) / p;
+                    pp.PA[d] = pp.P[d] - RA[d];
+                }
+                pp.EIJ = eij[x];
+                pp.K = pp.EIJ * sa.coef[i] * sb.coef[j];
+                pp.beta = bb;
+                pp.ip = 1.0 / p;
+            }
         }
     };
     const size_t np = pairs.size();
