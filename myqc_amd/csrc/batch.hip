@@ -25,6 +25,7 @@
 #include <string>
 #include <vector>
 
+#include "boys_dev.h"
 #include "context.h"
 #include "guess.h"
 #include "ket_soa.h"
@@ -58,15 +59,14 @@ __global__ __launch_bounds__(128) void k_batch_one_e(const ShellPair *__restrict
                                                      const double *__restrict__ atoms, const int *__restrict__ pair_mol,
                                                      const BMol *__restrict__ mols, int npairs, double *__restrict__ S,
                                                      double *__restrict__ H) {
-    __shared__ double s_ft[FT_TOTAL];
-    for (int i = threadIdx.x; i < FT_TOTAL; i += blockDim.x) s_ft[i] = ftT[i];
-    __syncthreads();
+    __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(2)];
+    const BoysTab ft = stage_boys<2>(ftT, s_ft);
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= npairs) return;
     const ShellPair sp = pairs[t];
     const BMol mol = mols[pair_mol[t]];
     double s[3][3], h[3][3];
-    one_e_pair(sp, prims, s_ft, atoms + 4 * mol.atom0, mol.nnuc, s, h);
+    one_e_pair(sp, prims, ft, atoms + 4 * mol.atom0, mol.nnuc, s, h);
     const int na = sp.la ? 3 : 1, nb = sp.lb ? 3 : 1;
     const long long n = mol.n;
     double *Sm = S + mol.mat0, *Hm = H + mol.mat0;
@@ -99,9 +99,9 @@ struct BEriArgs {
 
 template <int CB, int CK>
 __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
-    __shared__ double s_ft[FT_TOTAL];
-    for (int i = threadIdx.x; i < FT_TOTAL; i += blockDim.x) s_ft[i] = a.ftT[i];
-    __syncthreads();
+    constexpr int M = CB + CK;
+    __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(M)];
+    const BoysTab ft = stage_boys<M>(a.ftT, s_ft);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.nq) return;
     int lo = 0, hi = a.nmol;   // last m with qcum[m] <= t
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
     constexpr int LA = BPL<CB>::a, LB = BPL<CB>::b, LC = BPL<CK>::a, LD = BPL<CK>::b;
     constexpr int na = ncart(LA), nb = ncart(LB), nc = ncart(LC), nd = ncart(LD);
     QuartetAcc<LA, LB, LC, LD> acc;
-    quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, mol.cls0[CK] + r}, s_ft, acc);
+    quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, mol.cls0[CK] + r}, ft, acc);
     const double CD[3] = {ket.AB[0], ket.AB[1], ket.AB[2]};
     double out[na * nb * nc * nd];
     quartet_hrr<LA, LB, LC, LD>(acc, bra.AB, CD, out);
@@ -1078,7 +1078,8 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
         b.nq[c] = qc[nmol];
         MYQC_CHECK(upload(ctx, &b.d_qcum[c], qc));
     }
-    const std::vector<double> ftT = build_ftT(Ftab);
+    std::vector<double> ftT(FT_TOTAL);
+    boys_inputs(Ftab, ftT.data() + FT_EG);
     MYQC_CHECK(upload(ctx, &b.d_mols, b.mols));
     MYQC_CHECK(upload(ctx, &b.d_order, b.order));
     MYQC_CHECK(upload(ctx, &b.d_pair_mol, pair_mol));
@@ -1100,6 +1101,8 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
     MYQC_CHECK(upload(ctx, &b.d_atoms, atoms));
     b.natom = (int)(atoms.size() / 4);
     MYQC_CHECK(upload(ctx, &b.d_ftT, ftT));
+    k_boys_rows<<<kBoysRowBlocks, 64, 0, ctx->stream>>>(b.d_ftT);
+    MYQC_HIP(ctx, hipGetLastError());
     const size_t M = (size_t)std::max<long long>(b.total_mat, 1);
     MYQC_CHECK(dalloc(ctx, (void **)&b.d_eri, sizeof(double) * std::max<long long>(b.total_eri, 1)));
     MYQC_CHECK(dalloc(ctx, (void **)&b.d_S, sizeof(double) * M));

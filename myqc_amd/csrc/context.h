@@ -68,7 +68,7 @@ struct myqc_ctx {
     std::vector<myqc::PrimPair> prims;
     std::vector<int> pair_ids[3];         // per pair class, sorted by Schwarz value (descending)
     std::vector<double> schwarz;          // per pair
-    std::vector<double> ftT;              // Ftab transposed: [Tk][m]
+    std::vector<double> ftT;              // the Boys tables' inputs (boys_inputs)
     myqc::ShellPair *d_pairs = nullptr;
     myqc::PrimPair *d_prims = nullptr;
     double *d_ftT = nullptr;

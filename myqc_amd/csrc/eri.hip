@@ -21,6 +21,7 @@
 #include <thread>
 #include <unordered_map>
 
+#include "boys_dev.h"
 #include "context.h"
 #include "dense.h"
 #include "wave.h"
@@ -159,21 +160,25 @@ __device__ __forceinline__ void find_quartet(const long long *__restrict__ cum, 
     rk = t - cum[lo] + (same ? lo : 0);
 }
 
-__device__ __forceinline__ void load_ft(const double *__restrict__ ftT, double *s_ft) {
-    for (int i = threadIdx.x; i < FT_TOTAL; i += blockDim.x) s_ft[i] = ftT[i];
-    __syncthreads();
-}
-
 // SPLIT lanes per shell quartet: they share its primitive quartets, add their
 // sums (group_sum), and each stores every SPLIT-th element of the block.
 // Waves per SIMD asked of the register allocator per class (the staged
-// table's 23 KB of LDS allows seven 256-thread workgroups per CU): ss|ss 6,
+// tables' 39 to 41 KB of LDS allow four 256-thread workgroups per CU): ss|ss 6,
 // ps|ss 5, ps|ps and pp|ss 4, the rest unconstrained.
+//
+// Bounded by FP64 VALU issue (70 to 80 % of it): about 90 instructions per
+// primitive quartet of ss|ss, 30 of the 81 surviving the screen.  40 waters,
+// the six classes together: 2.33 ms with every primitive pair tested and the
+// reference's downward recursion from F_Q, 2.00 with rows cut at the screen
+// (eri_math.h), 1.90 with F_M tabulated, 1.78 with one transcendental less, K/p
+// and fewer conversions.  512 threads (eight waves per SIMD on the same
+// staged tables): 1.79, and small systems 30 % slower.
 constexpr int eri_waves(int cb, int ck) { return cb + ck == 0 ? 6 : cb + ck == 1 ? 5 : cb + ck == 2 ? 4 : 1; }
 template <int CB, int CK, int SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(CB, CK)))) void k_eri(EriArgs a) {
-    __shared__ double s_ft[FT_TOTAL];
-    load_ft(a.ftT, s_ft);
+    constexpr int M = CB + CK;
+    __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(M)];
+    const BoysTab ft = stage_boys<M>(a.ftT, s_ft);
     const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long t = tid / SPLIT;
     const int sub = (int)(tid % SPLIT);
@@ -196,7 +201,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(C
     ShellPair bra;
     if constexpr (SPLIT > 1) {
         bra = a.pairs[pb];
-        quartet_prims_split<LA, LB, LC, LD, SPLIT>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, s_ft, acc, sub);
+        quartet_prims_split<LA, LB, LC, LD, SPLIT>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, ft, acc, sub);
         using AQ = QuartetAcc<LA, LB, LC, LD>;
 #pragma unroll
         for (int e = 0; e < AQ::NE; ++e)
@@ -204,10 +209,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(C
             for (int f = 0; f < AQ::NF; ++f) acc.v[e][f] = group_sum<SPLIT>(acc.v[e][f]);
     } else if (kUniformPath && __all(pb == pb0)) {
         bra = a.pairs[pb0];
-        quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, s_ft, acc);
+        quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, ft, acc);
     } else {
         bra = a.pairs[pb];
-        quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, s_ft, acc);
+        quartet_prims_f<LA, LB, LC, LD>(bra, ket, a.prims, KetSoa{a.ksoa, a.nket, rk}, ft, acc);
     }
     double CD[3] = {ket.AB[0], ket.AB[1], ket.AB[2]};
     double out[BLK];
@@ -245,14 +250,15 @@ constexpr int kSchwarzLanes = 8, kSchwarzPairs = 256 / kSchwarzLanes;
 
 template <int C>
 __device__ __forceinline__ void schwarz_pair(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
-                                             const double *s_ft, int p, bool on, int sub, double *__restrict__ q) {
+                                             const double *__restrict__ ftT, double *s_ft, int p, bool on, int sub, double *__restrict__ q) {
     constexpr int LA = PairL<C>::a, LB = PairL<C>::b;
     constexpr int na = ncart(LA), nb = ncart(LB);
+    const BoysTab ft = stage_boys<2 * C>(ftT, s_ft);
     const ShellPair sp = pairs[p];
     using AQ = QuartetAcc<LA, LB, LA, LB>;
     AQ acc;
     quartet_prims_split<LA, LB, LA, LB, kSchwarzLanes, false>(sp, sp, prims, [&](int j) { return prims[sp.pp0 + j]; },
-                                                              s_ft, acc, sub);
+                                                              ft, acc, sub);
 #pragma unroll
     for (int e = 0; e < AQ::NE; ++e)
 #pragma unroll
@@ -275,16 +281,15 @@ struct SchwarzArgs {
 
 __global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
                                                  const double *__restrict__ ftT, SchwarzArgs a, double *__restrict__ q) {
-    __shared__ double s_ft[FT_TOTAL];
-    load_ft(ftT, s_ft);
+    __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(4)];
     const int b = blockIdx.x, c = b >= a.blk[0] ? 0 : b >= a.blk[1] ? 1 : 2;
     // lanes past the last pair repeat it (the group sums need every lane)
     const int t = (b - a.blk[c]) * kSchwarzPairs + threadIdx.x / kSchwarzLanes, sub = threadIdx.x % kSchwarzLanes;
     const bool on = t < a.np[c];
     const int p = a.ids[c][on ? t : a.np[c] - 1];
-    if (c == 0) schwarz_pair<0>(pairs, prims, s_ft, p, on, sub, q);
-    else if (c == 1) schwarz_pair<1>(pairs, prims, s_ft, p, on, sub, q);
-    else schwarz_pair<2>(pairs, prims, s_ft, p, on, sub, q);
+    if (c == 0) schwarz_pair<0>(pairs, prims, ftT, s_ft, p, on, sub, q);
+    else if (c == 1) schwarz_pair<1>(pairs, prims, ftT, s_ft, p, on, sub, q);
+    else schwarz_pair<2>(pairs, prims, ftT, s_ft, p, on, sub, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -489,7 +494,7 @@ static void launch_class(myqc_ctx *ctx, int c, hipStream_t s, EriShape sh) {
 // count.  They include lanes that sit idle while a neighbour computes a
 // primitive quartet that its own pair screen drops, and both sides of a
 // divergent Boys branch, so they count issued rather than strictly useful work.
-static const double kQuartetFlops[6] = {3589.3, 4008.7, 5969.1, 6161.0, 11273.7, 34674.3};
+static const double kQuartetFlops[6] = {2319.9, 2920.7, 4588.6, 4724.8, 9633.6, 31778.1};
 
 static int build_classes(myqc_ctx *ctx, double tol) {
     std::vector<long long> cum;
@@ -791,17 +796,19 @@ extern "C" int myqc_set_system(myqc_ctx *ctx, int nnuc, const int *Z, const doub
                                          ctx->shells, ctx->pairs, ctx->prims, ctx->pair_ids);
     if (!why.empty()) return set_error(ctx, MYQC_E_ARG, "myqc_set_system: %s", why.c_str());
     hc.mark("set_system: shells and pairs");
-    // Boys table transposed to [Tk][m] so the 7 Taylor rows are contiguous
-    ctx->ftT = build_ftT(Ftab);
+    ctx->ftT.resize(FT_TOTAL - FT_EG);
+    boys_inputs(Ftab, ctx->ftT.data());
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_pairs, sizeof(ShellPair) * ctx->pairs.size()));
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_prims, sizeof(PrimPair) * ctx->prims.size()));
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_ftT, sizeof(double) * ctx->ftT.size()));
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_ftT, sizeof(double) * FT_TOTAL));
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_pairs, ctx->pairs.data(), sizeof(ShellPair) * ctx->pairs.size(),
                                  hipMemcpyHostToDevice, ctx->stream));
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_prims, ctx->prims.data(), sizeof(PrimPair) * ctx->prims.size(),
                                  hipMemcpyHostToDevice, ctx->stream));
-    MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_ftT, ctx->ftT.data(), sizeof(double) * ctx->ftT.size(), hipMemcpyHostToDevice,
-                                 ctx->stream));
+    MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_ftT + FT_EG, ctx->ftT.data(), sizeof(double) * ctx->ftT.size(),
+                                 hipMemcpyHostToDevice, ctx->stream));
+    k_boys_rows<<<kBoysRowBlocks, 64, 0, ctx->stream>>>(ctx->d_ftT);
+    MYQC_HIP(ctx, hipGetLastError());
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     hc.mark("set_system: uploads");
     ctx->have_system = true;

@@ -34,15 +34,49 @@ constexpr double PI_SP = (double)3.1415926535897931f;
 
 constexpr int FT_NT = 121;   // Tk = 0..120  (T = 0 .. 12 step 0.1)
 constexpr int FT_NM = 19;    // m  = 0..18 of the record's 23: the largest order read is Q + 6 = 18 (Q <= 12)
-// The staged table also holds e^{-k/10}, k = 0..600, after the Boys values
-// (FT_E0 on): e^{-T} for T < 60 (the largest T at which it is used, 2Q + 36
-// with Q <= 12) from one entry and a short series
-constexpr int FT_NE = 601;
-constexpr int FT_E0 = FT_NT * FT_NM;
-// and, from FT_G0 on, the coefficients of BoysG's g(T) = c0 + c1/T + c2/T^2 +
-// c3/T^3 on its four ranges of T (12-15, 15-18, 18-24, 24 on)
-constexpr int FT_G0 = FT_E0 + FT_NE;
-constexpr int FT_TOTAL = FT_G0 + 16;
+// The Boys tables as the kernels use them.  For T < 12 the reference expands
+// F_Q about Tk and recurs downward to F_M (below), up to 12 dependent steps for
+// each primitive quartet.  On the interval of one Tk that whole procedure is a
+// polynomial in x = Tk/10 - T times known functions, so its value F_M is
+// tabulated instead, per (M, Q / 3, Tk), as a polynomial of degree 6 (7 for
+// M >= 2, the last coefficient in a float) in x, |x| <= 0.05: the series to
+// degree 9, telescoped.  Against the procedure in 80 bits its largest error is
+// 0.6 to 1.1e-15 relative, the recursion's in doubles 1.0 to 1.5e-15.
+//
+// One block of FT_BLOCK per M = 0..4: FT_POLY coefficients ([Q / 3][Tk][power];
+// seven, an odd stride, spread a wavefront's rows over the LDS banks), then the
+// FT_TOP floats of degree 7 (Q >= 3: Q = 0 is the Taylor sum itself, degree 6).
+// After the blocks, at FT_EG: e^{-k/10}, k = 0..600 (e^{-T} for T < 60, the
+// largest T at which it is used, 2Q + 36 with Q <= 12, from one entry and a
+// short series), then the coefficients of BoysG's g(T) = c0 + c1/T + c2/T^2 +
+// c3/T^3 on its four ranges of T (12-15, 15-18, 18-24, 24 on); at FT_RAW the
+// record's Boys values, which the blocks are made from.
+constexpr int FT_NC = 7, FT_NQ = 5;
+constexpr int FT_POLY = FT_NQ * FT_NT * FT_NC + 1;         // even
+constexpr int FT_TOP = (FT_NQ - 1) * FT_NT / 2;            // in doubles
+constexpr int FT_BLOCK = FT_POLY + FT_TOP;
+constexpr int FT_NE = 601, FT_EGN = FT_NE + 17;            // even
+constexpr int FT_EG = 5 * FT_BLOCK, FT_RAW = FT_EG + FT_EGN, FT_RAWN = FT_NT * FT_NM;
+constexpr int FT_TOTAL = FT_RAW + FT_RAWN;
+
+// The tables of one order M, wherever they lie
+struct BoysTab {
+    const double *poly, *eg;
+    const float *top;
+};
+// in the full array
+template <int M>
+__host__ __device__ __forceinline__ BoysTab boys_tab(const double *full) {
+    const double *b = full + M * FT_BLOCK;
+    return {b, full + FT_EG, reinterpret_cast<const float *>(b + FT_POLY)};
+}
+template <int M>
+__host__ __device__ __forceinline__ BoysTab boys_tab(const BoysTab &t) {
+    return t;
+}
+// staged for a kernel: polynomials, e and g, and the degree-7 floats for M >= 2
+// (with these 40752 B, four workgroups per CU)
+constexpr int ft_staged(int M) { return FT_POLY + FT_EGN + (M >= 2 ? FT_TOP : 0); }
 
 // Cartesian components up to l = 2: 0 s | 1 x 2 y 3 z | 4 xx 5 xy 6 xz 7 yy 8 yz 9 zz
 MYQC_HD constexpr int cexp(int idx, int d) {
@@ -88,110 +122,154 @@ MYQC_HD double rsqrt_hd(double x) {
 #endif
 }
 
-// The predicate on some active lane of the wavefront (device; the value is
-// wave-uniform, so a branch on it jumps over code no lane needs instead of
-// running it under a mask), or the predicate itself (host).
-MYQC_HD bool any_lane(bool p) {
+// 1/x from r = rsqrt_hd(x): r^2 and one Newton-Raphson step (within about an
+// ulp of the quotient), one transcendental for both.  The host divides.
+MYQC_HD double recip_rsq(double x, double r) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_ballot_w64(p) != 0;
-#else
-    return p;
-#endif
-}
-
-// 1/x for x > 0 in the normal range: the device's reciprocal estimate refined
-// by two Newton-Raphson steps (within about an ulp of the quotient, without
-// the full division sequence), or the host's division
-MYQC_HD double recip_hd(double x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
+    const double y = r * r;
+    return fma(y, fma(-x, y, 1.0), y);
 #else
     return 1.0 / x;
 #endif
 }
 
-// The staged table ftT of (Boys table transposed, ftT[Tk*FT_NM + m]; then
-// e^{-k/10} at FT_E0 + k; then g's coefficients at FT_G0 + 4 range + power),
-// built from the Ftab record (Ft(Tk, m) at Tk + 121 m).  Host only.
-inline std::vector<double> build_ftT(const double *Ftab) {
-    std::vector<double> ftT(FT_TOTAL);
-    for (int tk = 0; tk < FT_NT; ++tk)
-        for (int m = 0; m < FT_NM; ++m) ftT[tk * FT_NM + m] = Ftab[tk + FT_NT * m];
-    for (int k = 0; k < FT_NE; ++k) ftT[FT_E0 + k] = std::exp(-0.1 * k);
+// a b for 0 <= a, b < 2^24
+MYQC_HD int mul24(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (int)__umul24((unsigned)a, (unsigned)b);
+#else
+    return a * b;
+#endif
+}
+
+// The part of the array from FT_EG on, which comes from the host: e, g and the
+// record's values (Ft(Tk, m) at Tk + 121 m).
+inline void boys_inputs(const double *Ftab, double *e) {
+    for (int k = 0; k < FT_NE; ++k) e[k] = std::exp(-0.1 * k);
     // BoysG (auxilary.f90:271-283); beyond T = 30 the reference's g is
     // undefined and 0.49 is used (changes F_0 by at most 3e-15 |g|)
     const double gc[16] = {0.4999489092, -0.2473631686, 0.321180909, -0.3811559346,
                            0.4998436875, -0.24249438,   0.24642845,  0.0,
                            0.499093162,  -0.2152832,    0.0,         0.0,
                            0.490,        0.0,           0.0,         0.0};
-    for (int k = 0; k < 16; ++k) ftT[FT_G0 + k] = gc[k];
-    return ftT;
+    for (int k = 0; k < 16; ++k) e[FT_NE + k] = gc[k];
+    e[FT_NE + 16] = 0.0;
+    for (int k = 0; k < FT_RAWN; ++k) e[FT_EGN + k] = Ftab[k];
 }
 
-// Boys F_0..F_M(T) as the reference computes them at order Q (M <= Q <= 16).
-// ftT: the staged table (build_ftT).
-template <int M>
-MYQC_HD void boys_ref(int Q, double T, const double *__restrict__ ftT, double (&F)[M + 1]) {
+// Row (q = Q / 3, Tk) of every block.  a[k]: the coefficients of F_j about Tk,
+// first F_Q's Taylor terms Ft(Tk, Q + k) / k! to k = 6 as the reference sums
+// them (auxilary.f90:152-155), then F_j = (2 T F_{j+1} + e^{-T}) / (2j + 1)
+// (:158-160) with T = Tk/10 - x and e^{-T} = e^{-Tk/10} e^x.  Orders above Q
+// are never formed: their row holds F_Q.
+MYQC_HD void boys_row(double *full, int q, int Tk) {
+    constexpr int ND = 10;
+    constexpr double h = 0.05;
+    const double *F = full + FT_RAW + Tk;
+    const int Q = 3 * q;
+    const double T0 = Tk / 10.0, E = full[FT_EG + Tk];
+    double a[ND], ek[ND];
+    double f = 1.0;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        if (k > 0) f *= k;
+        a[k] = k <= 6 ? F[FT_NT * (Q + k)] / f : 0.0;
+        ek[k] = E / f;
+    }
+    for (int j = Q; j >= 0; --j) {
+        if (j < Q) {
+            const double d = 1.0 / (2.0 * j + 1.0);
+#pragma unroll
+            for (int k = ND - 1; k >= 0; --k) a[k] = (2.0 * T0 * a[k] - (k > 0 ? 2.0 * a[k > 0 ? k - 1 : 0] : 0.0) + ek[k]) * d;
+        }
+        if (j > 4) continue;
+        double b[ND], hk = 1.0;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+            b[k] = a[k] * hk;
+            hk *= h;
+        }
+        // u^9, u^8 (and u^7) by the Chebyshev polynomials of their degree
+        b[7] += b[9] * (576.0 / 256.0);
+        b[5] -= b[9] * (432.0 / 256.0);
+        b[3] += b[9] * (120.0 / 256.0);
+        b[1] -= b[9] * (9.0 / 256.0);
+        b[6] += b[8] * 2.0;
+        b[4] -= b[8] * 1.25;
+        b[2] += b[8] * 0.25;
+        b[0] -= b[8] * (1.0 / 128.0);
+        for (int M = j; M <= (j == Q ? 4 : j); ++M) {
+            double c5 = b[5], c3 = b[3], c1 = b[1];
+            if (M < 2 || q == 0) {
+                c5 += b[7] * 1.75;
+                c3 -= b[7] * 0.875;
+                c1 += b[7] * (7.0 / 64.0);
+            }
+            double *r = full + M * FT_BLOCK + (q * FT_NT + Tk) * FT_NC;
+            constexpr double ih = 20.0;
+            r[0] = b[0];
+            r[1] = c1 * ih;
+            r[2] = b[2] * (ih * ih);
+            r[3] = c3 * (ih * ih * ih);
+            r[4] = b[4] * (ih * ih * ih * ih);
+            r[5] = c5 * (ih * ih * ih * ih * ih);
+            r[6] = b[6] * (ih * ih * ih * ih * ih * ih);
+            if (q > 0)
+                reinterpret_cast<float *>(full + M * FT_BLOCK + FT_POLY)[(q - 1) * FT_NT + Tk] =
+                    (float)(b[7] * (ih * ih * ih * ih * ih * ih * ih));
+        }
+    }
+}
+
+// The whole array on the host
+inline std::vector<double> build_ftT(const double *Ftab) {
+    std::vector<double> full(FT_TOTAL);
+    boys_inputs(Ftab, full.data() + FT_EG);
+    for (int q = 0; q < FT_NQ; ++q)
+        for (int Tk = 0; Tk < FT_NT; ++Tk) boys_row(full.data(), q, Tk);
+    return full;
+}
+
+// Boys F_0..F_M(T) as the reference computes them at order Q (a multiple of 3,
+// at most 12: sets have max L <= 1, which is checked when the system is built,
+// and Q = 3 (sum of four set L's)).  ft: the array, or order M's tables.
+template <int M, typename FT>
+MYQC_HD void boys_ref(int Q, double T, const FT &ft, double (&F)[M + 1]) {
+    const BoysTab tab = boys_tab<M>(ft);
     // Tk = NINT(10 T) (T >= 0; T clamped to 60, beyond every table use) and
-    // x = Tk / 10 - T, |x| <= 0.05.  Tk / 10 without a division: the product
-    // and one fma correction equal the correctly rounded quotient for every
-    // integer 0..1000 (checked exhaustively)
+    // x = Tk / 10 - T, |x| <= 0.05, with 1/10 in two doubles
     const double Tc = T < 60.0 ? T : 60.0;
-    const int Tk = (int)floor(Tc * 10.0 + 0.5);
-    const double tkd = (double)Tk, q10 = tkd * 0.1;
-    const double x = fma(fma(-q10, 10.0, tkd), 0.1, q10) - Tc;
-    // e^{-T} feeds the downward recursion below T = 12 (when Q > 0) and the
+    const double tkd = floor(fma(Tc, 10.0, 0.5));
+    const int Tk = (int)tkd;
+    const double x = fma(tkd, -0x1.999999999999ap-58, fma(tkd, 0.1, -Tc));
+    // e^{-T} feeds the downward recursion below T = 12 (M > 0) and the
     // asymptotic form up to 2Q + 36; one evaluation serves both branches (the
     // lanes of a wavefront usually fall on both sides of T = 12):
     // e^{-T} = e^{-Tk/10} e^x with the Taylor series of e^x to x^7 (the next
-    // term is below 1e-15 relative)
+    // term is below 1e-15 relative); to x^5 for M = 0, where it enters F_0 only
+    // above T = 12, as at most 1e-6 of it
     double e = 0.0;
-    if ((Q > 0 || T >= 12.0) && T < 2.0 * Q + 36.0) {
-        double s = 1.0 / 5040.0;
-        s = fma(s, x, 1.0 / 720.0);
-        s = fma(s, x, 1.0 / 120.0);
+    if (((M > 0 && Q > 0) || T >= 12.0) && T < 2.0 * Q + 36.0) {
+        double s = 1.0 / 120.0;
+        if constexpr (M > 0) s = fma(fma(1.0 / 5040.0, x, 1.0 / 720.0), x, s);
         s = fma(s, x, 1.0 / 24.0);
         s = fma(s, x, 1.0 / 6.0);
         s = fma(s, x, 0.5);
         s = fma(s, x, 1.0);
         s = fma(s, x, 1.0);
-        e = ftT[FT_E0 + Tk] * s;
+        e = tab.eg[Tk] * s;
     }
     if (T < 12.0) {
-        const double *r = ftT + Tk * FT_NM + Q;
-        // sum_{k=0..6} Ft(Tk,Q+k) x^k / k!   (auxilary.f90:152-155), in
-        // Horner form r0 + x (r1 + x/2 (r2 + x/3 (r3 + ...)))
+        const int q = Q / 3, row = q * FT_NT + Tk;
+        const double *r = tab.poly + mul24(row, FT_NC);
         double fq = r[6];
+        if constexpr (M >= 2) fq = fma(q > 0 ? (double)tab.top[max(row - FT_NT, 0)] : 0.0, x, fq);
 #pragma unroll
-        for (int k = 5; k >= 0; --k) fq = fma(fq, x * (1.0 / (k + 1)), r[k]);
-        // with Q = 0 (sets of s functions only) there is no recursion: F_0 is
-        // the Taylor sum itself
-        const int top = Q < M ? Q : M;
-        double t2 = 2.0 * T;
-        // downward recursion F_j = (2T F_{j+1} + e^{-T}) / (2j+1)  (auxilary.f90:158-160),
-        // with 1/(2j+1) as constants; the reference divides (rounding-level difference)
-        // Q <= 12: sets have max L <= 1 (checked when the system is built), so
-        // Q = 3 (sum of four set L's) <= 12.  Q is a multiple of 3, so the
-        // steps j = Q-1 .. M run in blocks of three (j = 3b+2, 3b+1, 3b for
-        // Q > 3b), each behind one branch that a wavefront skips when none of
-        // its lanes needs it (any_lane)
-#pragma unroll
-        for (int b = 3; b >= 0; --b) {
-            if (3 * b + 2 < M) continue;
-            if (any_lane(Q > 3 * b)) {
-                const bool on = Q > 3 * b;
-#pragma unroll
-                for (int j = 3 * b + 2; j >= 3 * b; --j)
-                    if (j >= M) {
-                        const double v = (t2 * fq + e) * (1.0 / (2.0 * j + 1.0));
-                        fq = on ? v : fq;
-                    }
-            }
-        }
-        // fq now holds F_top, top = min(Q, M); the reference never forms F_j for
-        // j > Q, and callers only read F_j for j <= Q
+        for (int k = 5; k >= 0; --k) fq = fma(fq, x, r[k]);
+        // fq holds F_top; the reference never forms F_j for j > Q, and callers
+        // only read F_j for j <= Q
+        const int top = M > 0 && Q < M ? Q : M;
+        const double t2 = 2.0 * T;
 #pragma unroll
         for (int j = M; j >= 0; --j) {
             if (j > top) F[j] = 0.0;
@@ -208,7 +286,7 @@ MYQC_HD void boys_ref(int Q, double T, const double *__restrict__ ftT, double (&
             // for T's range from the staged table, one polynomial for every
             // lane (no branch per range)
             const int rg = (T >= 15.0) + (T >= 18.0) + (T >= 24.0);
-            const double *gc = ftT + FT_G0 + 4 * rg;
+            const double *gc = tab.eg + FT_NE + 4 * rg;
             const double g = fma(fma(fma(gc[3], iT, gc[2]), iT, gc[1]), iT, gc[0]);
             F[0] = half_sqrt_pi * rt - e * g * iT;
 #pragma unroll
@@ -230,6 +308,7 @@ struct PrimPair {
     double EIJ;      // exp(-alpha beta |AB|^2 / p): the reference's pair screen factor
     double beta;     // exponent of the second shell's primitive (kinetic energy)
     double ip;       // 1 / p
+    double KI;       // K / p
     // default construction leaves the fields unset: arrays of primitive pairs
     // are sized before they are filled
     MYQC_HD PrimPair() {}
@@ -261,16 +340,16 @@ struct QuartetAcc {
 // values, the bra vertical recursion [e0|00]^(m), the ket vertical recursion
 // [e0|f0]^(m), and the targets.  Q: the Boys order rule of the shell
 // quartet; c0 = 2 pi^2.5.
-template <int LA, int LB, int LC, int LD>
+template <int LA, int LB, int LC, int LD, typename FT>
 MYQC_HD __forceinline__ void prim_quartet(const PrimPair &b, const PrimPair &k, int Q, double c0,
-                                          const double *__restrict__ ftT, QuartetAcc<LA, LB, LC, LD> &acc) {
+                                          const FT &ftT, QuartetAcc<LA, LB, LC, LD> &acc) {
     using A = QuartetAcc<LA, LB, LC, LD>;
     constexpr int EB = A::EB, EK = A::EK, M = A::M;
     constexpr int NB = nupto(EB);
     const double p = b.p, q = k.p, pq = p + q;
-    const double ipq = recip_hd(pq);
-    const double rho = p * q * ipq;
     const double rsq = rsqrt_hd(pq);
+    const double ipq = recip_rsq(pq, rsq);
+    const double rho = p * q * ipq;
     double PQ[3], WP[3], WQ[3], QC[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -281,7 +360,7 @@ MYQC_HD __forceinline__ void prim_quartet(const PrimPair &b, const PrimPair &k, 
         QC[d] = k.PA[d];
     }
     const double T = rho * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
-    const double pref = c0 * b.ip * k.ip * rsq * b.K * k.K;
+    const double pref = c0 * k.KI * (b.KI * rsq);
     double F[M + 1];
     boys_ref<M>(Q, T, ftT, F);
     // bra vertical recursion [e0|00]^(m)
@@ -349,9 +428,9 @@ MYQC_HD __forceinline__ void prim_quartet(const PrimPair &b, const PrimPair &k, 
 // Schwarz factors, since a primitive pair dropped from (ab|ab) by
 // EIJ^2 < 1e-14 can survive EIJ*EGH >= 1e-14 against a compact ket pair.
 // The ket's primitive pairs come from kprim(j), j < ket.npp.
-template <int LA, int LB, int LC, int LD, bool SCREEN = true, typename KF>
+template <int LA, int LB, int LC, int LD, bool SCREEN = true, typename KF, typename FT>
 MYQC_HD void quartet_prims_f(const ShellPair &bra, const ShellPair &ket, const PrimPair *__restrict__ ppb,
-                             KF &&kprim, const double *__restrict__ ftT, QuartetAcc<LA, LB, LC, LD> &acc) {
+                             KF &&kprim, const FT &ftT, QuartetAcc<LA, LB, LC, LD> &acc) {
     using A = QuartetAcc<LA, LB, LC, LD>;
     const int Q = 3 * (bra.bl + ket.bl);
 #pragma unroll
@@ -363,15 +442,24 @@ MYQC_HD void quartet_prims_f(const ShellPair &bra, const ShellPair &ket, const P
     // and the inner loop reads the bra's primitives, whose addresses the lanes
     // of a wavefront (one bra pair, consecutive kets) mostly share.  A pair's
     // primitives stand with the largest screen factor first (system.h), so a
-    // row ends at the first one screened: a third to a half of the primitive
-    // quartets survive, and testing all of them cost 14 % of the kernels'
-    // time (40 waters 2.33 -> 2.00 ms)
+    // row ends at the first one screened (int2e.f90:257), and the rows at the
+    // first that starts with one: a third to a half of the primitive quartets
+    // survive.  The next primitive of either side is loaded before the work on
+    // the current one: where the lanes' bras differ (batch.hip), the wait for
+    // each was a fifth of the time.
+    const PrimPair *bp = ppb + bra.pp0;
+    const PrimPair b0 = bp[0];
+    PrimPair kn = kprim(0);
     for (int j = 0; j < ket.npp; ++j) {
-        const PrimPair k = kprim(j);
-        for (int i = 0; i < bra.npp; ++i) {
-            const PrimPair b = ppb[bra.pp0 + i];
-            if (SCREEN && b.EIJ * k.EIJ < 1.0e-14) break;          // int2e.f90:257; the rest are smaller
+        const PrimPair k = kn;
+        if (SCREEN && b0.EIJ * k.EIJ < 1.0e-14) break;
+        kn = kprim(j + 1 < ket.npp ? j + 1 : j);
+        PrimPair b = b0;
+        for (int i = 1; ; ++i) {
+            const PrimPair bn = bp[i < bra.npp ? i : 0];
             prim_quartet<LA, LB, LC, LD>(b, k, Q, c0, ftT, acc);
+            if (i >= bra.npp || (SCREEN && bn.EIJ * k.EIJ < 1.0e-14)) break;
+            b = bn;
         }
     }
 }
@@ -379,9 +467,9 @@ MYQC_HD void quartet_prims_f(const ShellPair &bra, const ShellPair &ket, const P
 // The same sum split over SPLIT lanes: lane `sub` of the quartet's group
 // takes the primitive quartets t = j npp_bra + i with t = sub (mod SPLIT);
 // the group's partial sums are added afterwards (split_reduce on the device).
-template <int LA, int LB, int LC, int LD, int SPLIT, bool SCREEN = true, typename KF>
+template <int LA, int LB, int LC, int LD, int SPLIT, bool SCREEN = true, typename KF, typename FT>
 MYQC_HD void quartet_prims_split(const ShellPair &bra, const ShellPair &ket, const PrimPair *__restrict__ ppb,
-                                 KF &&kprim, const double *__restrict__ ftT, QuartetAcc<LA, LB, LC, LD> &acc,
+                                 KF &&kprim, const FT &ftT, QuartetAcc<LA, LB, LC, LD> &acc,
                                  int sub) {
     using A = QuartetAcc<LA, LB, LC, LD>;
     const int Q = 3 * (bra.bl + ket.bl);
@@ -409,10 +497,9 @@ MYQC_HD void quartet_prims_split(const ShellPair &bra, const ShellPair &ket, con
     }
 }
 
-template <int LA, int LB, int LC, int LD, bool SCREEN = true>
+template <int LA, int LB, int LC, int LD, bool SCREEN = true, typename FT>
 MYQC_HD void quartet_prims(const ShellPair &bra, const ShellPair &ket, const PrimPair *__restrict__ ppb,
-                           const PrimPair *__restrict__ ppk, const double *__restrict__ ftT,
-                           QuartetAcc<LA, LB, LC, LD> &acc) {
+                           const PrimPair *__restrict__ ppk, const FT &ftT, QuartetAcc<LA, LB, LC, LD> &acc) {
     quartet_prims_f<LA, LB, LC, LD, SCREEN>(bra, ket, ppb, [&](int j) { return ppk[ket.pp0 + j]; }, ftT, acc);
 }
 

@@ -1,6 +1,6 @@
 // ket_soa.h -- the primitive pairs of a list of shell pairs as structure of
 // arrays, for the ERI kernels that give consecutive lanes consecutive kets of
-// such a list: field f (p, P[3], PA[3], K, EIJ, 1/p) of primitive j of list
+// such a list: field f (p, P[3], PA[3], K/p, EIJ, 1/p) of primitive j of list
 // entry r sits at [(j * kKetFields + f) * np + r], so a wavefront reads each
 // field with one coalesced load.  STO-3G pairs have 3 x 3 primitive pairs;
 // callers refuse more when they build the arrays.
@@ -21,7 +21,7 @@ static __global__ void k_ket_soa(const ShellPair *__restrict__ pairs, const Prim
     double f[kKetFields] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     if (j < sp.npp) {
         const PrimPair q = prims[sp.pp0 + j];
-        const double g[kKetFields] = {q.p, q.P[0], q.P[1], q.P[2], q.PA[0], q.PA[1], q.PA[2], q.K, q.EIJ, q.ip};
+        const double g[kKetFields] = {q.p, q.P[0], q.P[1], q.P[2], q.PA[0], q.PA[1], q.PA[2], q.KI, q.EIJ, q.ip};
 #pragma unroll
         for (int k = 0; k < kKetFields; ++k) f[k] = g[k];
     }
@@ -43,8 +43,9 @@ struct KetSoa {
         q.PA[0] = b[4 * np];
         q.PA[1] = b[5 * np];
         q.PA[2] = b[6 * np];
-        q.K = b[7 * np];
+        q.KI = b[7 * np];
         q.EIJ = b[8 * np];
+        q.K = 0.0;   // (unused by the quartets, as beta)
         q.beta = 0.0;
         q.ip = b[9 * np];
         return q;

@@ -5,6 +5,7 @@
 // SCF dipole moment of cphf_dipole_rhf (src/props/cphf.f90:106-121).
 #include <cmath>
 
+#include "boys_dev.h"
 #include "context.h"
 #include "one_e_math.h"
 
@@ -13,9 +14,8 @@ namespace myqc {
 __global__ __launch_bounds__(256) void k_one_e(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
                                                const double *__restrict__ ftT, const double *__restrict__ atoms,
                                                int nnuc, int npairs, int n, double *__restrict__ S, double *__restrict__ H) {
-    __shared__ double s_ft[FT_TOTAL];
-    for (int i = threadIdx.x; i < FT_TOTAL; i += blockDim.x) s_ft[i] = ftT[i];
-    __syncthreads();
+    __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(2)];
+    const BoysTab ft = stage_boys<2>(ftT, s_ft);
     // one wavefront per shell pair: lane l takes the nuclei l, l + 64, ... of
     // the attraction integrals and the primitive pairs l, l + 64, ... of S and
     // T, then the lanes' sums are added across the wavefront
@@ -24,7 +24,7 @@ __global__ __launch_bounds__(256) void k_one_e(const ShellPair *__restrict__ pai
     if (t >= npairs) return;   // whole wavefronts
     const ShellPair sp = pairs[t];
     double s[3][3], h[3][3];
-    one_e_pair(sp, prims, s_ft, atoms, nnuc, s, h, lane, 64);
+    one_e_pair(sp, prims, ft, atoms, nnuc, s, h, lane, 64);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll

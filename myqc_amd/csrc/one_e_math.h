@@ -71,8 +71,8 @@ MYQC_HD void dipole_pair(const ShellPair &sp, const PrimPair *__restrict__ prims
 // wavefront) summing their s and h cover the pair once; the defaults take
 // everything.
 // LA, LB are the pair's angular momenta (the first shell carries the larger).
-template <int LA, int LB>
-MYQC_HD void one_e_pair_t(const ShellPair &sp, const PrimPair *__restrict__ prims, const double *__restrict__ ftT,
+template <int LA, int LB, typename FT>
+MYQC_HD void one_e_pair_t(const ShellPair &sp, const PrimPair *__restrict__ prims, const FT &ftT,
                           const double *__restrict__ atoms, int nnuc, double s[3][3], double h[3][3], int c0,
                           int cstep) {
     constexpr int na = LA ? 3 : 1, nb = LB ? 3 : 1;
@@ -147,7 +147,8 @@ MYQC_HD void one_e_pair_t(const ShellPair &sp, const PrimPair *__restrict__ prim
 }
 
 // S, H of one shell pair with runtime angular momenta (first shell larger)
-MYQC_HD void one_e_pair(const ShellPair &sp, const PrimPair *__restrict__ prims, const double *__restrict__ ftT,
+template <typename FT>
+MYQC_HD void one_e_pair(const ShellPair &sp, const PrimPair *__restrict__ prims, const FT &ftT,
                         const double *__restrict__ atoms, int nnuc, double s[3][3], double h[3][3], int c0 = 0,
                         int cstep = 1) {
     if (sp.la && sp.lb) one_e_pair_t<1, 1>(sp, prims, ftT, atoms, nnuc, s, h, c0, cstep);

@@ -168,6 +168,7 @@ inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int n
                 pp.K = pp.EIJ * sa.coef[i] * sb.coef[j];
                 pp.beta = bb;
                 pp.ip = 1.0 / p;
+                pp.KI = pp.K * pp.ip;
             }
         }
     };
