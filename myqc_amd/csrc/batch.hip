@@ -9,12 +9,15 @@
 //                        pair-class combination: the same OS/HGP code and
 //                        reference numerics as the single-molecule path,
 //                        written into the molecule's packed 8-fold-unique
-//                        array (ij|kl), i>=j, k>=l, ij>=kl
+//                        array (ij|kl), i>=j, k>=l, ij>=kl, halved where i = j
+//                        and where ij = kl
 //   k_batch_scf          persistent: each workgroup takes molecules from an
 //                        atomic queue (largest first) and runs the whole SCF
-//                        on-chip -- G(D) by streaming the packed integrals
-//                        from HBM into LDS accumulators, DIIS, and a cyclic
-//                        Jacobi eigensolver in LDS -- with no host round trip
+//                        on-chip -- G(D) from the packed integrals streamed
+//                        from HBM, products on the FP64 matrix cores, DIIS,
+//                        Newton-Schulz for S^-1/2 and purification for the
+//                        density (cyclic Jacobi where either does not
+//                        converge) -- with no host round trip
 //
 // The launch shapes (threads per ERI and SCF workgroup) are chosen by timing
 // the candidates on the batch itself (batch_tune), and the whole sequence is
@@ -30,6 +33,7 @@
 #include "guess.h"
 #include "ket_soa.h"
 #include "one_e_math.h"
+#include "small_dense.h"
 
 namespace myqc {
 
@@ -144,7 +148,9 @@ __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
                 for (int id = 0; id < nd; ++id) {
                     const int i = bra.ao_a + ia, j = bra.ao_b + ib, k = ket.ao_a + ic, l = ket.ao_b + id;
                     const long long IJ = tri(max(i, j)) + min(i, j), KL = tri(max(k, l)) + min(k, l);
-                    E[tri(max(IJ, KL)) + min(IJ, KL)] = out[((ia * nb + ib) * nc + ic) * nd + id];
+                    const bool same = IJ >= KL ? i == j : k == l;
+                    E[tri(max(IJ, KL)) + min(IJ, KL)] =
+                        (same ? 0.5 : 1.0) * (IJ == KL ? 0.5 : 1.0) * out[((ia * nb + ib) * nc + ic) * nd + id];
                 }
 }
 
@@ -173,21 +179,11 @@ struct BScfArgs {
 
 // Workgroup reductions: a wavefront butterfly, then the per-wave results
 // summed in a fixed order (every thread returns the same value).
-__device__ __forceinline__ double wave_red_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-__device__ __forceinline__ double wave_red_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 __device__ __forceinline__ double wg_sum(double v, double *s_red) {
-    v = wave_red_sum(v);
+    const int t = thread_index();
+    v = wave_total(v);
     __syncthreads();   // s_red free
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+    if ((t & 63) == 0) s_red[t >> 6] = v;
     __syncthreads();
     double r = 0.0;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r += s_red[w];
@@ -195,31 +191,14 @@ __device__ __forceinline__ double wg_sum(double v, double *s_red) {
 }
 
 __device__ __forceinline__ double wg_max(double v, double *s_red) {
-    v = wave_red_max(v);
+    const int t = thread_index();
+    v = wave_largest(v);
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+    if ((t & 63) == 0) s_red[t >> 6] = v;
     __syncthreads();
     double r = -1e300;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) r = fmax(r, s_red[w]);
     return r;
-}
-
-// C = alpha A B (or A B^T); all n x n column-major; caller synchronises.
-// Operands may sit in HBM: the k loop is unrolled so that their loads issue
-// together.
-__device__ __forceinline__ void mm(double *C, const double *A, const double *B, int n, bool transB, double alpha) {
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-        const int i = e % n, j = e / n;
-        double s = 0.0;
-        if (transB) {
-#pragma unroll 8
-            for (int k = 0; k < n; ++k) s += A[i + n * k] * B[j + n * k];
-        } else {
-#pragma unroll 8
-            for (int k = 0; k < n; ++k) s += A[i + n * k] * B[k + n * j];
-        }
-        C[e] = alpha * s;
-    }
 }
 
 // Cyclic Jacobi on the symmetric A (n x n, LDS): eigenvalues on A's diagonal,
@@ -227,12 +206,13 @@ __device__ __forceinline__ void mm(double *C, const double *A, const double *B, 
 // the n/2 rotations of a round are disjoint; each thread applies J^T A J to
 // whole 2x2 blocks in place, so one barrier separates the rounds.
 __device__ void jacobi(double *A, double *U, int n, double *s_rot, double *s_red) {
+    const int t0 = thread_index();
     const int npad = n + (n & 1), half = npad >> 1;
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) U[e] = (e % n == e / n) ? 1.0 : 0.0;
+    for (int e = t0; e < n * n; e += blockDim.x) U[e] = (e % n == e / n) ? 1.0 : 0.0;
     __syncthreads();
     for (int sweep = 0; sweep < 30; ++sweep) {
         double off = 0.0, dia = 0.0;
-        for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+        for (int e = t0; e < n * n; e += blockDim.x) {
             const double v = A[e];
             if (e % n == e / n) dia += v * v;
             else off += v * v;
@@ -242,7 +222,7 @@ __device__ void jacobi(double *A, double *U, int n, double *s_rot, double *s_red
         if (off <= 1e-28 * fmax(dia, 1e-300)) break;
         for (int r = 0; r < npad - 1; ++r) {
             // rotation of pair k: s_rot[4k] = p, [4k+1] = q, [4k+2] = c, [4k+3] = s
-            for (int k = threadIdx.x; k < half; k += blockDim.x) {
+            for (int k = t0; k < half; k += blockDim.x) {
                 const int a = k == 0 ? 0 : ((k - 1 + r) % (npad - 1)) + 1;
                 const int kb = npad - 1 - k;
                 const int b = ((kb - 1 + r) % (npad - 1)) + 1;
@@ -264,7 +244,7 @@ __device__ void jacobi(double *A, double *U, int n, double *s_rot, double *s_red
             }
             __syncthreads();
             // A <- J^T A J on 2x2 blocks (pair k1 rows, pair k2 columns)
-            for (int w = threadIdx.x; w < half * half; w += blockDim.x) {
+            for (int w = t0; w < half * half; w += blockDim.x) {
                 const int k1 = w % half, k2 = w / half;
                 const int p1 = (int)s_rot[4 * k1], q1 = (int)s_rot[4 * k1 + 1];
                 const int p2 = (int)s_rot[4 * k2], q2 = (int)s_rot[4 * k2 + 1];
@@ -283,7 +263,7 @@ __device__ void jacobi(double *A, double *U, int n, double *s_rot, double *s_red
                 if (q1ok && q2ok) A[q1 + n * q2] = T10 * s2 + T11 * c2;
             }
             // U <- U J
-            for (int w = threadIdx.x; w < n * half; w += blockDim.x) {
+            for (int w = t0; w < n * half; w += blockDim.x) {
                 const int row = w % n, k = w / n;
                 const int p = (int)s_rot[4 * k], q = (int)s_rot[4 * k + 1];
                 if (q >= n) continue;
@@ -295,63 +275,6 @@ __device__ void jacobi(double *A, double *U, int n, double *s_rot, double *s_red
             __syncthreads();
         }
     }
-}
-
-__device__ __forceinline__ void wg_sum2(double &x, double &y, double *s_red) {
-    x = wave_red_sum(x);
-    y = wave_red_sum(y);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
-        s_red[2 * (threadIdx.x >> 6)] = x;
-        s_red[2 * (threadIdx.x >> 6) + 1] = y;
-    }
-    __syncthreads();
-    x = y = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-        x += s_red[2 * w];
-        y += s_red[2 * w + 1];
-    }
-}
-
-// Projector onto the nocc lowest levels of the symmetric A (n x n, LDS, left
-// unchanged) into P by trace-correcting purification (Niklasson, PRB 66,
-// 155115 (2002)): P0 = (hi I - A)/(hi - lo) from Gershgorin bounds, then
-// P <- P^2 or 2P - P^2, whichever trace lands nearer nocc (tr P^2 = ||P||_F^2
-// for symmetric P).  Two steps after P is idempotent to 1e-8 with trace nocc
-// to 1e-6 it is final.  T: n x n LDS scratch.  False when that does not
-// happen within 100 steps (near-degenerate frontier levels).
-__device__ bool purify_lds(const double *A, double *P, double *T, int n, int nocc, double *s_red) {
-    double lo = 1e300, hi = -1e300;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        double r = 0.0;
-        for (int j = 0; j < n; ++j)
-            if (j != i) r += fabs(A[i + n * j]);
-        const double c = A[i * (n + 1)];
-        lo = fmin(lo, c - r);
-        hi = fmax(hi, c + r);
-    }
-    lo = -wg_max(-lo, s_red);
-    hi = wg_max(hi, s_red);
-    const double sc = 1.0 / fmax(hi - lo, 1e-300);
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) P[e] = ((e % n == e / n ? hi : 0.0) - A[e]) * sc;
-    int cs = -1;
-    for (int step = 0; step < 100; ++step) {
-        double t = 0.0, f = 0.0;
-        for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-            const double v = P[e];
-            f += v * v;
-            if (e % n == e / n) t += v;
-        }
-        wg_sum2(t, f, s_red);   // also orders the previous step's writes of P
-        if (cs < 0 && step >= 8 && fabs(t - f) < 1e-8 && fabs(t - nocc) < 1e-6) cs = step;
-        if (cs >= 0 && step >= cs + 2) return true;
-        const bool square = fabs(f - nocc) < fabs(2.0 * t - f - nocc);
-        mm(T, P, P, n, false, 1.0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < n * n; e += blockDim.x) P[e] = square ? T[e] : 2.0 * P[e] - T[e];
-    }
-    __syncthreads();
-    return false;
 }
 
 // indices of the nocc lowest eigenvalues (diagonal of A) into s_occ; thread 0
@@ -371,318 +294,452 @@ __device__ void select_occ(const double *A, int n, int nocc, int *s_occ, int *s_
     __syncthreads();
 }
 
-// P = U_occ U_occ^T
-__device__ __forceinline__ void occ_projector(double *P, const double *U, const int *s_occ, int n, int nocc) {
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+// Element (i, j), i >= j, of the packed lower triangle
+__device__ __forceinline__ int packed(int i, int j) { return i * (i + 1) / 2 + j; }
+
+// T = A + A^T (packed) for the A of G(D) = A + A^T, from the packed unique
+// integrals (degeneracy weights 1/2 per index coincidence).  A wavefront takes
+// rows ij of the triangle (one, two of up to 32 functions or four of up to 16):
+//   - its 64 lanes load the row, kets kl = lane, lane + 64, ..., ahead of the
+//     work on the row before, apply the weights, sum the row's J(ij) and, in
+//     registers over all rows, J(kl), and lay the row down in LDS;
+//   - then lane m takes row m of the symmetric matrix V(kl) whose triangle the
+//     row is, and forms (V D_j)_m and (V D_i)_m for the exchange rows i and j.
+//     The lane's LDS addresses in V are the same for every ij and stay in
+//     registers; for t <= m they start at m (m + 1) / 2, which falls in distinct
+//     banks for 32 consecutive m, and for t > m they are consecutive.  D is read
+//     by broadcasts of two, and no two lanes add into one element.
+// Every integral costs one HBM read, an LDS write and two LDS reads, against
+// five reads of D, two of the index tables and three colliding atomics per
+// value when each value is digested by itself.  Bounded by LDS (the broadcasts
+// of D are half of its cycles): 35 functions, eight wavefronts alone on a CU
+// 123 us, two workgroups of four 192 us each, against 400 us with two of eight;
+// the integrals' HBM read alone is 83 us when every CU has its own.
+template <class C>
+struct FockRows {
+    static constexpr int LANES = C::NP <= 16 ? 16 : C::NP <= 32 ? 32 : 64, ROWS = 64 / LANES;
+    static constexpr int NMAX = C::NP < kBatchMaxN ? C::NP : kBatchMaxN;
+    static constexpr int U = (NMAX * (NMAX + 1) / 2 + 63) / 64;
+    static __host__ __device__ constexpr int ld(int n) { return (n + 7) & ~7; }
+    // a row in LDS, with the zeros that its last 64 loads bring
+    static __host__ __device__ constexpr int row(int n) {
+        return ld(n) * (ld(n) + 1) / 2 > 64 * U ? ld(n) * (ld(n) + 1) / 2 : 64 * U;
+    }
+    // doubles of LDS: D's rows, T, and each wavefront's rows
+    static __host__ __device__ constexpr int lds(int n) {
+        return ld(n) * n + ((n * (n + 1) / 2 + 1) & ~1) + C::WAVES * ROWS * row(n);
+    }
+};
+__device__ __forceinline__ void row_of(int r, int &i, int &j) {
+    i = (int)((__builtin_amdgcn_sqrtf(8.0f * r + 1.0f) - 1.0f) * 0.5f);
+    i += (i + 1) * (i + 2) / 2 <= r ? 1 : 0;   // (the root is within a rounding of it)
+    i -= i * (i + 1) / 2 > r ? 1 : 0;
+    j = r - i * (i + 1) / 2;
+}
+
+template <class C>
+__device__ __forceinline__ void batch_fock(const double *__restrict__ eri, const double *__restrict__ D, double *arena,
+                                           int n) {
+    using R = FockRows<C>;
+    constexpr int U = R::U, G = R::ROWS, STEP = C::WAVES * G;
+    const int t = thread_index(), lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int P = n * (n + 1) / 2, ld = R::ld(n), PS = R::row(n);
+    double *Dt = arena, *T = Dt + ld * n, *rows = T + ((P + 1) & ~1) + w * G * PS;
+    // row i of D at Dt + ld i, zero beyond n
+    for (int e = t; e < ld * n; e += C::THREADS) {
         const int i = e % n, j = e / n;
-        double s = 0.0;
-        for (int a = 0; a < nocc; ++a) s += U[i + n * s_occ[a]] * U[j + n * s_occ[a]];
-        P[e] = s;
+        Dt[j + ld * i] = j < n ? D[i + n * j] : 0.0;
     }
-}
-
-// DIIS coefficients from the (m+1)^2 system on thread 0, worked in the LDS
-// array M ((kBatchDiis + 1) (kBatchDiis + 2) doubles); false if singular
-__device__ bool diis_solve(const double *B, int MD, int m, double *M, double *c) {
-    const int N = m + 1, W = N + 1;
-    for (int i = 0; i < N; ++i)
-        for (int j = 0; j < W; ++j) M[i * W + j] = 0.0;
-    for (int i = 0; i < m; ++i) {
-        for (int j = 0; j < m; ++j) M[i * W + j] = B[i * MD + j];
-        M[i * W + m] = -1.0;
-    }
-    for (int j = 0; j < m; ++j) M[m * W + j] = -1.0;
-    M[m * W + N] = -1.0;
-    for (int col = 0; col < N; ++col) {
-        int piv = col;
-        for (int r = col + 1; r < N; ++r)
-            if (fabs(M[r * W + col]) > fabs(M[piv * W + col])) piv = r;
-        if (fabs(M[piv * W + col]) < 1e-300) return false;
-        if (piv != col)
-            for (int k = 0; k < W; ++k) {
-                const double t = M[col * W + k];
-                M[col * W + k] = M[piv * W + k];
-                M[piv * W + k] = t;
+    for (int e = t; e < P; e += C::THREADS) T[e] = 0.0;
+    for (int e = lane; e < G * PS; e += 64) rows[e] = 0.0;   // a row's entries beyond its own stay zero
+    // a row's loads end at its length: buffer loads past it give 0 and read nothing
+    double v[G][U];
+    auto fetch = [&](int base) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int r = min(base + g, P - 1);
+            const auto row = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(eri + r * (r + 1) / 2), (short)0,
+                                                               8 * (r + 1), 0x00020000);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                typedef int i2_t __attribute__((ext_vector_type(2)));
+                const i2_t x = __builtin_amdgcn_raw_buffer_load_b64(row, 8 * lane + 512 * u, 0, 0);
+                v[g][u] = __longlong_as_double(((long long)x.y << 32) | (unsigned)x.x);
             }
-        for (int r = 0; r < N; ++r) {
-            if (r == col) continue;
-            const double f = M[r * W + col] / M[col * W + col];
-            for (int k = col; k < W; ++k) M[r * W + k] -= f * M[col * W + k];
         }
-    }
-    for (int i = 0; i < m; ++i) c[i] = M[i * W + N] / M[i * W + i];
-    return true;
-}
-
-// G(D) = A + A^T accumulated from the packed unique integrals (degeneracy
-// weights 1/2 per index coincidence); F = H + G.  A wavefront takes one bra
-// pair IJ at a time and each lane four consecutive kets KL <= IJ (a
-// contiguous run of the packed array), loaded a step ahead.  The J(ij)
-// term is reduced across the wavefront; the K terms on (i,k) and (j,k), whose
-// k repeats along a run of kets, are summed in registers while k stays the
-// same; the other three go to LDS per value.  Aacc and the copy Dl of D have
-// an odd leading dimension, so the updates and reads of a column (same i,
-// consecutive l) fall in distinct LDS banks.
-__device__ void fock(const double *__restrict__ eri, const double *__restrict__ H, const double *D, double *Aacc,
-                     double *Dl, double *F, int n, const unsigned char *s_pi, const unsigned char *s_pj) {
-    const int la = n | 1;
-    for (int e = threadIdx.x; e < la * n; e += blockDim.x) {
-        const int i = e % la, j = e / la;
-        Aacc[e] = 0.0;
-        Dl[e] = i < n ? D[i + n * j] : 0.0;
-    }
+    };
+    fetch(w * G);
     __syncthreads();
-    const int P = (int)tri(n);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
-    constexpr int U = 4, STEP = 64 * U;
-    auto advance = [&](int &ij, int &kl) {
-        kl += STEP;
-        if (kl > ij) {
-            ij += nwave;
-            kl = 0;
-        }
+    // the lane's kets: first the chunks of 64 that every row has work in, then the others
+    constexpr int UA = (U + 1) / 2, UB = U - UA;
+    double dka[UA], jka[UA], dkb[UB + 1], jkb[UB + 1];
+    auto ket = [&](int u) {
+        int k, l;
+        row_of(min(lane + 64 * u, P - 1), k, l);
+        return lane + 64 * u < P ? (k == l ? 1.0 : 2.0) * Dt[l + ld * k] : 0.0;
     };
-    auto load = [&](int ij, int kl, double (&v)[U]) {
-        const int x = kl + U * lane;
-        const double *row = eri + tri(ij);
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = (ij < P && x + u <= ij) ? row[x + u] : 0.0;
-    };
-    int pij = wave, pkl = 0;
-    double v0[U], v2[U];
-    load(pij, pkl, v0);
-    advance(pij, pkl);
-    int IJ = wave, KL0 = 0;
-    double jr = 0.0;
-    while (IJ < P) {
+    for (int u = 0; u < UA; ++u) {
+        dka[u] = ket(u);
+        jka[u] = 0.0;
+    }
 #pragma unroll
-        for (int u = 0; u < U; ++u) v2[u] = v0[u];
-        load(pij, pkl, v0);
-        advance(pij, pkl);
-        const int i = s_pi[IJ], j = s_pj[IJ];
-        const double dij = Dl[i + la * j];
-        const double wij = (i == j) ? 0.5 : 1.0;
-        int kc = -1;
-        double aik = 0.0, ajk = 0.0;
+    for (int u = 0; u < UB; ++u) {
+        dkb[u] = ket(UA + u);
+        jkb[u] = 0.0;
+    }
+    const int g = lane / R::LANES, m = lane % R::LANES;
+    // where row min(m, n - 1) of V holds column s
+    const double *Vs[R::NMAX];
+    {
+        const int mm = min(m, n - 1);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int KL = KL0 + U * lane + u;
-            if (KL <= IJ) {
-                const int k = s_pi[KL], l = s_pj[KL];
-                double v = v2[u] * wij;
-                if (k == l) v *= 0.5;
-                if (IJ == KL) v *= 0.5;
-                if (k != kc) {
-                    if (kc >= 0) {
-                        atomicAdd(&Aacc[i + la * kc], aik);
-                        atomicAdd(&Aacc[j + la * kc], ajk);
-                    }
-                    kc = k;
-                    aik = ajk = 0.0;
+        for (int s = 0; s < R::NMAX; ++s) Vs[s] = rows + g * PS + packed(max(mm, s), min(mm, s));
+    }
+    for (int base = w * G; base < P; base += STEP) {
+        int imax = 0;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int r = min(base + q, P - 1);   // (past the last row: it again, its sums dropped)
+            int i, j;
+            row_of(r, i, j);
+            imax = __builtin_amdgcn_readfirstlane(i);
+            const double d2 = base + q < P ? 2.0 * Dt[j + ld * i] : 0.0;
+            double jr = 0.0, *to = rows + q * PS + lane;
+#pragma unroll
+            for (int u = 0; u < UA; ++u) {
+                jr += v[q][u] * dka[u];
+                jka[u] += v[q][u] * d2;
+                to[64 * u] = v[q][u];
+            }
+            if (r >= 64 * UA) {   // (uniform)
+#pragma unroll
+                for (int u = 0; u < UB; ++u) {
+                    jr += v[q][UA + u] * dkb[u];
+                    jkb[u] += v[q][UA + u] * d2;
+                    to[64 * (UA + u)] = v[q][UA + u];
                 }
-                jr += 2.0 * Dl[k + la * l] * v;
-                aik -= 0.5 * Dl[j + la * l] * v;
-                ajk -= 0.5 * Dl[i + la * l] * v;
-                atomicAdd(&Aacc[k + la * l], 2.0 * dij * v);
-                atomicAdd(&Aacc[i + la * l], -0.5 * Dl[j + la * k] * v);
-                atomicAdd(&Aacc[j + la * l], -0.5 * Dl[i + la * k] * v);
+            }
+            jr = wave_total(jr);
+            if (lane == 0 && base + q < P) atomicAdd(&T[r], i == j ? 2.0 * jr : jr);
+        }
+        fetch(base + STEP);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the rows' writes before their reads
+        const int r = base + g;
+        int i, j;
+        row_of(min(r, P - 1), i, j);
+        const double *Di = Dt + ld * i, *Dj = Dt + ld * j;
+        double y = 0.0, z = 0.0;
+#pragma unroll
+        for (int s = 0; s < R::NMAX; s += 8) {
+            if (s <= imax) {   // (uniform)
+                double vs[8];
+                double2 di[4], dj[4];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) vs[k] = *Vs[s + k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    di[k] = *reinterpret_cast<const double2 *>(Di + s + 2 * k);
+                    dj[k] = *reinterpret_cast<const double2 *>(Dj + s + 2 * k);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    y += vs[2 * k] * dj[k].x;
+                    z += vs[2 * k] * di[k].x;
+                    y += vs[2 * k + 1] * dj[k].y;
+                    z += vs[2 * k + 1] * di[k].y;
+                }
             }
         }
-        if (kc >= 0) {
-            atomicAdd(&Aacc[i + la * kc], aik);
-            atomicAdd(&Aacc[j + la * kc], ajk);
+        if (r < P && m <= i) {
+            atomicAdd(&T[packed(i, m)], m == i ? -y : -0.5 * y);
+            atomicAdd(&T[packed(max(j, m), min(j, m))], m == j ? -z : -0.5 * z);
         }
-        KL0 += STEP;
-        if (KL0 > IJ) {   // row done (uniform across the wavefront)
-            jr = wave_red_sum(jr);
-            if (lane == 0) atomicAdd(&Aacc[i + la * j], jr);
-            jr = 0.0;
-            IJ += nwave;
-            KL0 = 0;
-        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the reads before the next rows' writes
     }
-    __syncthreads();
-    for (int x = threadIdx.x; x < n * n; x += blockDim.x) {
-        const int i = x % n, j = x / n;
-        F[x] = H[x] + Aacc[i + la * j] + Aacc[j + la * i];
-    }
+#pragma unroll
+    for (int u = 0; u < UA; ++u)
+        if (lane + 64 * u < P) atomicAdd(&T[lane + 64 * u], jka[u]);
+#pragma unroll
+    for (int u = 0; u < UB; ++u)
+        if (lane + 64 * (UA + u) < P) atomicAdd(&T[lane + 64 * (UA + u)], jkb[u]);
     __syncthreads();
 }
 
-// LDS: L0 (G accumulator / Jacobi matrix) and L2 (padded D in the Fock build
-// / U / purification), (nmax | 1) nmax doubles each; L1 (D), L3 (temp), nmax^2
-// doubles each; then reductions, rotations, DIIS matrix and index tables.
-__host__ __device__ inline size_t scf_lds_bytes(int nmax, int threads) {
-    const size_t n2 = (size_t)nmax * nmax;
-    return sizeof(double) * (4 * n2 + 2 * nmax + threads + 2 * (nmax + 2) + kBatchDiis * kBatchDiis + kBatchDiis + 8 +
-                             (kBatchDiis + 1) * (kBatchDiis + 2)) +
-           sizeof(int) * 2 * nmax + 2 * (size_t)tri(nmax) + 16;
+// LDS of a workgroup: the arena (two matrices of the dense part, the Fock
+// build's D, T and rows, or the Jacobi fallback's matrices), then reductions
+struct BScfLds {
+    double *arena, *red, *part, *sum, *c, *B, *rot;
+    int *occ, *tmp;
+};
+template <int WV>
+__host__ __device__ constexpr int scf_tail_doubles() {
+    // red, part, sum, c, B, rot, occ and tmp, the job
+    return WV + 16 * WV + 10 * WV + kBatchDiis + kBatchDiis * kBatchDiis + 2 * (kBatchMaxN + 2) + kBatchMaxN + 2;
+}
+template <class C>
+__host__ __device__ constexpr int scf_arena_doubles(int n) {
+    const int dense = 2 * C::NP * (C::LD > C::NP + 1 ? C::LD : C::NP + 1), fock = FockRows<C>::lds(n);
+    const int jac = 2 * n * n;
+    const int x = dense > fock ? dense : fock;
+    return ((x > jac ? x : jac) + 1) & ~1;
 }
 
-// (at most 128 VGPRs: two 512-thread workgroups per CU)
-__global__ __launch_bounds__(512, 4) void k_batch_scf(BScfArgs a, int nmax) {
-    extern __shared__ __attribute__((aligned(16))) double smem[];
-    const size_t n2max = (size_t)nmax * nmax;
-    // L0 and L2: (nmax | 1) x nmax (the Fock build's padded accumulator and D)
-    double *L0 = smem, *L1 = L0 + n2max + nmax, *L2 = L1 + n2max, *L3 = L2 + n2max + nmax;
-    double *s_red = L3 + n2max;
-    double *s_rot = s_red + blockDim.x;                  // 2 (nmax + 2)
-    double *s_B = s_rot + 2 * (nmax + 2);                // kBatchDiis^2
-    double *s_c = s_B + kBatchDiis * kBatchDiis;         // kBatchDiis
-    double *s_misc = s_c + kBatchDiis;                   // 8
-    double *s_M = s_misc + 8;                            // DIIS system
-    int *s_occ = reinterpret_cast<int *>(s_M + (kBatchDiis + 1) * (kBatchDiis + 2));
-    int *s_tmp = s_occ + nmax;
-    unsigned char *s_pi = reinterpret_cast<unsigned char *>(s_tmp + nmax);
-    unsigned char *s_pj = s_pi + tri(nmax);
-    int *s_job = reinterpret_cast<int *>(s_misc + 7);
-    const int MD = kBatchDiis;
-    while (true) {
-        if (threadIdx.x == 0) *s_job = atomicAdd(a.counter, 1);
+template <class C>
+__device__ __forceinline__ void batch_solve(const BScfArgs &a, const BMol &mol, int m, const BScfLds &s) {
+    constexpr int NP = C::NP, LD = C::LD, MD = kBatchDiis, MT = C::MT, TH = C::THREADS, WV = C::WAVES;
+    constexpr int EL = (NP * NP + TH - 1) / TH;
+    const int n = mol.n, nocc = mol.nocc, nn = n * n;
+    const double *Sg = a.S + mol.mat0, *Hg = a.H + mol.mat0, *eri = a.eri + mol.eri0;
+    double *X = a.scratch + 4 * mol.mat0, *Do = X + nn, *Fx = Do + nn, *D1 = Fx + nn, *D0 = a.Dout + mol.mat0;
+    double *hF = a.hist + 2 * MD * mol.mat0, *hE = hF + MD * nn;
+    double *sA = s.arena, *sB = s.arena + NP * LD;
+    d4_t acc[MT];
+    // X = S^-1/2 and S^1/2 (the latter in the DIIS history's place until that
+    // is written); where 24 steps do not converge (condition numbers beyond
+    // about 1e8) by the eigen-decomposition, which sees a singular S
+    double *Xi = hE;
+    {
+    const int t = thread_index();
+    if (!inv_sqrt_ns<C>(n, Sg, X, Xi, hF, hF + nn, s.arena, s.red, 24)) {
+        double *A = s.arena, *Uv = A + nn;
         __syncthreads();
-        const int job = *s_job;
+        for (int e = t; e < nn; e += TH) A[e] = Sg[e];
         __syncthreads();
-        if (job >= a.nmol) break;
-        const int m = a.order[job];
-        const BMol mol = a.mols[m];
-        const int n = mol.n, nocc = mol.nocc;
-        const size_t nn = (size_t)n * n;
-        const double *Sg = a.S + mol.mat0, *Hg = a.H + mol.mat0, *eri = a.eri + mol.eri0;
-        double *X = a.scratch + 4 * mol.mat0, *Fp = X + nn, *Dp = Fp + nn, *W = Dp + nn;
-        double *hF = a.hist + 2 * MD * mol.mat0, *hE = hF + MD * nn;
-        for (int x = threadIdx.x; x < tri(n); x += blockDim.x) {
-            int i = (int)floor((sqrt(8.0 * x + 1.0) - 1.0) * 0.5);
-            while (tri(i) > x) --i;
-            while (tri(i + 1) <= x) ++i;
-            s_pi[x] = (unsigned char)i;
-            s_pj[x] = (unsigned char)(x - tri(i));
-        }
-        // X = S^{-1/2} by the eigen-decomposition of S
-        for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) L0[e] = Sg[e];
-        __syncthreads();
-        jacobi(L0, L2, n, s_rot, s_red);
+        jacobi(A, Uv, n, s.rot, s.red);
         double smin = 1e300;
-        for (int i = threadIdx.x; i < n; i += blockDim.x) smin = fmin(smin, L0[i * (n + 1)]);
-        smin = -wg_max(-smin, s_red);
+        for (int i = t; i < n; i += TH) smin = fmin(smin, A[i * (n + 1)]);
+        smin = -wg_max(-smin, s.red);
         if (smin <= 1e-10) {
-            if (threadIdx.x == 0) {
+            if (t == 0) {
                 a.energy[m] = 0.0;
                 a.iters[m] = 0;
                 a.conv[m] = -1;   // overlap numerically singular
                 if (a.fallback) a.fallback[m] = 0;
             }
-            __syncthreads();
-            continue;
+            return;
         }
-        for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) L3[e] = L2[e] / sqrt(L0[(e / n) * (n + 1)]);
+        for (int e = t; e < nn; e += TH) {
+            const int i = e % n, j = e / n;
+            double x = 0.0, y = 0.0;
+            for (int k = 0; k < n; ++k) {
+                const double q = sqrt(A[k * (n + 1)]), uu = Uv[i + n * k] * Uv[j + n * k];
+                x += uu / q;
+                y += uu * q;
+            }
+            X[e] = x;
+            Xi[e] = y;
+        }
         __syncthreads();
-        mm(X, L3, L2, n, true, 1.0);
+    }
+    }
+    // From the Fock matrix in sA (and in Fx): the projector onto its nocc lowest
+    // levels by purification, or by diagonalisation when the frontier levels
+    // are too close for it, into Do; the density 2 X P X into Dn.
+    auto new_density = [&](double *Dn) {
+        const int t = thread_index();
+        int steps;
+        if (nocc == n) {
+            for (int e = t; e < NP * NP; e += TH) {
+                const int i = e % NP, j = e / NP;
+                sA[i + LD * j] = i == j && i < n ? 1.0 : 0.0;
+            }
+        } else if (!purify<C>(sA, sB, n, nocc, 100, s.red, s.part, steps)) {
+            double *A = s.arena, *Uv = A + nn;
+            __syncthreads();
+            for (int e = t; e < nn; e += TH) A[e] = Fx[e];
+            __syncthreads();
+            jacobi(A, Uv, n, s.rot, s.red);
+            select_occ(A, n, nocc, s.occ, s.tmp);
+            double p[EL];
+#pragma unroll
+            for (int q = 0; q < EL; ++q) {
+                const int e = t + q * TH, i = e % NP, j = e / NP;
+                p[q] = 0.0;
+                if (i < n && j < n)
+                    for (int x = 0; x < nocc; ++x) p[q] += Uv[i + n * s.occ[x]] * Uv[j + n * s.occ[x]];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < EL; ++q) {
+                const int e = t + q * TH;
+                if (e < NP * NP) sA[e % NP + LD * (e / NP)] = p[q];
+            }
+        }
         __syncthreads();
-        // a start from the given density gets learned_iter iterations; if it
-        // does not converge, the molecule restarts from the core guess in the
-        // same workgroup with the full budget
-        int it_total = 0, conv = 0, it = 0;
-        double E = 0.0;
-        for (int attempt = a.guess ? 0 : 1; attempt < 2; ++attempt) {
+        for (int e = t; e < nn; e += TH) Do[e] = sA[e % n + LD * (e / n)];
+        load<C>(sB, X, n);
+        __syncthreads();
+        product<C>(sB, sA, acc);   // X P
+        __syncthreads();
+        to_lds<C>(sA, acc);
+        __syncthreads();
+        product<C>(sA, sB, acc);
+        each<C>(acc, [&](int i, int j, double v) {
+            if (i < n && j < n) Dn[i + n * j] = 2.0 * v;
+        });
+        __syncthreads();
+    };
+    // the Fock matrix in sB to the orthonormal basis, into sA
+    auto orthonormal = [&]() {
+        load<C>(sA, X, n);
+        __syncthreads();
+        product<C>(sA, sB, acc);   // X F
+        __syncthreads();
+        to_lds<C>(sB, acc);
+        __syncthreads();
+        product<C>(sB, sA, acc);
+        __syncthreads();
+        to_lds<C>(sA, acc);
+    };
+    // a start from the given density gets learned_iter iterations; if it
+    // does not converge, the molecule restarts from the core guess in the
+    // same workgroup with the full budget
+    int it_total = 0, conv = 0, it = 0;
+    double E = 0.0;
+    double *D = D0;
+    for (int attempt = a.guess ? 0 : 1; attempt < 2; ++attempt) {
         const bool from_guess = attempt == 0;
         const int maxit = from_guess ? a.learned_iter : a.max_iter;
+        D = D0;
         if (from_guess) {
-            // Dp = S^{1/2} D S^{1/2} / 2
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) L3[e] = L2[e] * sqrt(L0[(e / n) * (n + 1)]);
+            const int t = thread_index(), lane = t & 63, w = t >> 6;
+            // Do = S^{1/2} D S^{1/2} / 2; the given D need not be symmetric
+            for (int e = t; e < nn; e += TH) D0[e] = a.guess[mol.mat0 + e];
+            load<C>(sA, a.guess + mol.mat0, n);
+            load<C>(sB, Xi, n);
             __syncthreads();
-            mm(W, L3, L2, n, true, 1.0);              // S^{1/2}
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) L1[e] = a.guess[mol.mat0 + e];
+            product<C>(sA, sB, acc);
             __syncthreads();
-            mm(L3, W, L1, n, false, 1.0);
+            to_lds<C>(sA, acc);
             __syncthreads();
-            mm(Dp, L3, W, n, false, 0.5);
+            const int g = lane >> 4, c = lane & 15;
+#pragma unroll
+            for (int q = 0; q < MT; ++q) {
+                const int tile = w + q * WV;
+                if (tile >= C::T2) break;
+                const double *pa = sB + 16 * (tile % C::NT) + c + LD * g, *pb = sA + LD * (16 * (tile / C::NT) + c) + g;
+                acc[q] = (d4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int k = 0; k < NP; k += 4) acc[q] = mfma64(pa[LD * k], pb[k], acc[q]);
+            }
+            each<C>(acc, [&](int i, int j, double v) {
+                if (i < n && j < n) Do[i + n * j] = 0.5 * v;
+            });
             __syncthreads();
         } else {
             // core Hamiltonian guess (scf.f90:410-512)
-            mm(L3, Hg, X, n, false, 1.0);
+            load<C>(sB, Hg, n);
+            orthonormal();
+            each<C>(acc, [&](int i, int j, double v) {
+                if (i < n && j < n) Fx[i + n * j] = v;
+            });
             __syncthreads();
-            mm(L0, X, L3, n, false, 1.0);
-            __syncthreads();
-            jacobi(L0, L2, n, s_rot, s_red);
-            select_occ(L0, n, nocc, s_occ, s_tmp);
-            occ_projector(Dp, L2, s_occ, n, nocc);
-            __syncthreads();
-            mm(L3, Dp, X, n, false, 1.0);
-            __syncthreads();
-            mm(L1, X, L3, n, false, 2.0);
-            __syncthreads();
+            new_density(D0);
         }
         int hist = 0, head = 0;
         double E_old = 0.0, dE_prev = 1e300, err_prev = 1e300;
         bool abandoned = false;
         E = 0.0;
         for (it = 1; it <= maxit + 1; ++it) {
-            // F = H + G(D) into W; E = (D.F + D.H)/2 + E_nuc
-            fock(eri, Hg, L1, L0, L2, W, n, s_pi, s_pj);
-            double ed = 0.0;
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) ed += L1[e] * (W[e] + Hg[e]);
-            E = 0.5 * wg_sum(ed, s_red) + mol.e_nuc;
-            // the previous iteration's density change, then its convergence
-            if (it > 1) {
-                double dd = 0.0;
-                for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) dd = fmax(dd, fabs(L1[e] - L3[e]));
-                dd = wg_max(dd, s_red);
-                if (it > 2 && dE_prev < a.e_tol && dd < a.d_tol && err_prev < 100.0 * a.d_tol) {
-                    conv = 1;
-                    break;
-                }
-            }
-            if (it > maxit) break;
-            // F' = X F X into the history; error F' Dp - Dp F'
-            double *fs = hF + head * nn, *es = hE + head * nn;
-            mm(L3, W, X, n, false, 1.0);
-            __syncthreads();
-            mm(fs, X, L3, n, false, 1.0);
-            __syncthreads();
-            mm(L3, fs, Dp, n, false, 1.0);
-            __syncthreads();
-            const int hn = min(hist + 1, MD);
-            double dots[kBatchDiis];
+            // F = H + G(D); E = (D.F + D.H)/2 + E_nuc, and the density's change
+            const int t = thread_index(), lane = t & 63, w = t >> 6;
+            double *Dn = D == D0 ? D1 : D0;   // D_{k-1}, and D_{k+1}'s place
+            batch_fock<C>(eri, D, s.arena, n);
+            double f[EL], ed = 0.0, dd = 0.0;
+            {
+                const int ld = FockRows<C>::ld(n);
+                const double *Dt = s.arena, *T = Dt + ld * n;
 #pragma unroll
-            for (int q = 0; q < kBatchDiis; ++q) dots[q] = 0.0;
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) {
-                const int i = e % n, j = e / n;
-                const double ev = L3[e] - L3[j + n * i];
-                es[e] = ev;
-#pragma unroll
-                for (int q = 0; q < kBatchDiis; ++q) {
-                    const double hv = q == head ? ev : (q < hn ? hE[q * nn + e] : 0.0);
-                    dots[q] += ev * hv;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < kBatchDiis; ++q) {
-                if (q < hn) {   // uniform across the workgroup
-                    const double v = wg_sum(dots[q], s_red);
-                    if (threadIdx.x == 0) {
-                        s_B[head * MD + q] = v;
-                        s_B[q * MD + head] = v;
+                for (int q = 0; q < EL; ++q) {
+                    const int e = t + q * TH, i = e % NP, j = e / NP;
+                    f[q] = 0.0;
+                    if (i < n && j < n) {
+                        const double h = Hg[i + n * j], d = Dt[j + ld * i];
+                        f[q] = h + T[packed(max(i, j), min(i, j))];
+                        ed += d * (f[q] + h);
+                        if (it > 1) dd = fmax(dd, fabs(d - Dn[i + n * j]));
                     }
                 }
             }
+            ed = wave_total(ed);
+            dd = wave_largest(dd);
+            if (lane == 0) {
+                s.sum[2 * w] = ed;
+                s.sum[2 * w + 1] = dd;
+            }
+            __syncthreads();   // (and D, T and the rows are free)
+            ed = dd = 0.0;
+            for (int q = 0; q < WV; ++q) {
+                ed += s.sum[2 * q];
+                dd = fmax(dd, s.sum[2 * q + 1]);
+            }
+            E = 0.5 * ed + mol.e_nuc;
+            // the previous iteration's convergence
+            if (it > 2 && dE_prev < a.e_tol && dd < a.d_tol && err_prev < 100.0 * a.d_tol) {
+                conv = 1;
+                break;
+            }
+            if (it > maxit) break;
+#pragma unroll
+            for (int q = 0; q < EL; ++q) {
+                const int e = t + q * TH;
+                if (e < NP * NP) sB[e % NP + LD * (e / NP)] = f[q];
+            }
+            // F' = X F X into the history; error F' Do - Do F'
+            orthonormal();
+            double *fs = hF + head * nn, *es = hE + head * nn;
+            each<C>(acc, [&](int i, int j, double v) {
+                if (i < n && j < n) fs[i + n * j] = v;
+            });
+            load<C>(sB, Do, n);
+            __syncthreads();
+            product<C>(sA, sB, acc);
+            __syncthreads();
+            to_lds<C>(sB, acc);
+            __syncthreads();
+            const int hn = min(hist + 1, MD);
+            double dots[MD];
+#pragma unroll
+            for (int q = 0; q < MD; ++q) dots[q] = 0.0;
+            for (int e = t; e < nn; e += TH) {
+                const int i = e % n, j = e / n;
+                const double ev = sB[i + LD * j] - sB[j + LD * i];
+                es[e] = ev;
+#pragma unroll
+                for (int q = 0; q < MD; ++q)
+                    if (q < hn) dots[q] += ev * (q == head ? ev : hE[q * nn + e]);
+            }
+#pragma unroll
+            for (int q = 0; q < MD; ++q) {
+                const double v = wave_total(dots[q]);
+                if (lane == 0) s.sum[w * MD + q] = v;
+            }
+            __syncthreads();
+            if (t < hn) {
+                double v = 0.0;
+                for (int q = 0; q < WV; ++q) v += s.sum[q * MD + t];
+                s.B[head * MD + t] = v;
+                s.B[t * MD + head] = v;
+            }
             __syncthreads();
             hist = hn;
-            // DIIS extrapolation of F' into L0
-            if (threadIdx.x == 0) {
-                const bool ok = hist >= 2 && diis_solve(s_B, MD, hist, s_M, s_c);
-                if (!ok) {
-                    for (int q = 0; q < MD; ++q) s_c[q] = 0.0;
-                    s_c[head] = 1.0;
-                }
-                s_misc[0] = ok ? 1.0 : 0.0;
-            }
+            // DIIS extrapolation of F' into sA
+            if (w == 0) diis_wave(s.B, hist, head, s.c);
             __syncthreads();
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) {
+            for (int e = t; e < NP * NP; e += TH) {
+                const int i = e % NP, j = e / NP;
                 double v = 0.0;
-                for (int q = 0; q < hist; ++q) v += s_c[q] * hF[q * nn + e];
-                L0[e] = v;
+                if (i < n && j < n) {
+                    const int x = i + n * j;
+#pragma unroll
+                    for (int q = 0; q < MD; ++q)
+                        if (q < hist) v += s.c[q] * hF[q * nn + x];
+                    Fx[x] = v;
+                }
+                sA[i + LD * j] = v;
             }
-            err_prev = sqrt(fabs(s_B[head * MD + head]));
+            err_prev = sqrt(fabs(s.B[head * MD + head]));
             dE_prev = fabs(E - E_old);
             E_old = E;
             head = (head + 1) % MD;
@@ -693,38 +750,86 @@ __global__ __launch_bounds__(512, 4) void k_batch_scf(BScfArgs a, int nmax) {
                 abandoned = true;
                 break;
             }
-            // new orthonormal density: the projector onto the nocc lowest
-            // levels of F' by purification, or by diagonalisation when the
-            // frontier levels are too close for it
-            if (purify_lds(L0, L2, L3, n, nocc, s_red)) {
-                for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) Dp[e] = L2[e];
-            } else {
-                jacobi(L0, L2, n, s_rot, s_red);
-                select_occ(L0, n, nocc, s_occ, s_tmp);
-                occ_projector(Dp, L2, s_occ, n, nocc);
-            }
-            __syncthreads();
-            // keep D_k in L3 for the change; D_{k+1} = 2 X Dp X into L1
-            for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) L3[e] = L1[e];
-            mm(W, Dp, X, n, false, 1.0);
-            __syncthreads();
-            mm(L1, X, W, n, false, 2.0);
-            __syncthreads();
+            new_density(Dn);
+            D = Dn;
         }
         it_total += abandoned ? it : min(it - 1, maxit);
         if (conv || !from_guess || !a.restart) {
             if (threadIdx.x == 0 && a.fallback) a.fallback[m] = from_guess ? 0 : (a.guess ? 1 : 0);
             break;
         }
-        }   // attempts
-        for (int e = threadIdx.x; e < (int)nn; e += blockDim.x) a.Dout[mol.mat0 + e] = L1[e];
-        if (threadIdx.x == 0) {
-            a.energy[m] = E;
-            a.iters[m] = it_total;
-            a.conv[m] = conv;
-        }
-        __syncthreads();
     }
+    const int t = thread_index();
+    if (D != D0)
+        for (int e = t; e < nn; e += TH) D0[e] = D[e];
+    if (t == 0) {
+        a.energy[m] = E;
+        a.iters[m] = it_total;
+        a.conv[m] = conv;
+    }
+}
+
+// Registers bound the residency (256 VGPRs: two wavefronts per SIMD; at 128 the
+// Fock rows spill and a build takes twice as long).  1024 clusters of 2 to 5
+// waters: 16 ms -> 5.0 ms; of an iteration's 218 us at 35 functions (eight
+// wavefronts) 123 are the Fock build, 51 the 30 purification steps, 10 X F X, 21
+// the DIIS error, its dots and the extrapolation.  The two Jacobi
+// diagonalisations of a molecule's start, 870 us, are 81 us of Newton-Schulz and
+// a purification.
+// arena_doubles: the largest of the batch's molecules (scf_lds_bytes)
+template <int WV>
+__global__ __launch_bounds__(64 * WV, 2) void k_batch_scf(BScfArgs a, int arena_doubles) {
+    extern __shared__ __attribute__((aligned(16))) double smem[];
+    BScfLds s;
+    s.arena = smem;
+    s.red = s.arena + arena_doubles;
+    s.part = s.red + WV;
+    s.sum = s.part + 16 * WV;
+    s.c = s.sum + 10 * WV;
+    s.B = s.c + kBatchDiis;
+    s.rot = s.B + kBatchDiis * kBatchDiis;
+    s.occ = reinterpret_cast<int *>(s.rot + 2 * (kBatchMaxN + 2));
+    s.tmp = s.occ + kBatchMaxN;
+    int *s_job = s.tmp + kBatchMaxN;
+    while (true) {
+        __syncthreads();
+        if (threadIdx.x == 0) *s_job = atomicAdd(a.counter, 1);
+        __syncthreads();
+        const int job = __builtin_amdgcn_readfirstlane(*s_job);
+        if (job >= a.nmol) break;
+        const int m = __builtin_amdgcn_readfirstlane(a.order[job]);
+        // (in scalar registers, which the compiler cannot tell by itself)
+        union {
+            BMol mol;
+            int word[sizeof(BMol) / 4];
+        } x;
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(BMol) / 4); ++k)
+            x.word[k] = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int *>(a.mols + m)[k]);
+        const BMol mol = x.mol;
+        if (mol.n <= 16) batch_solve<DenseLds<16, WV>>(a, mol, m, s);
+        else if (mol.n <= 32) batch_solve<DenseLds<32, WV>>(a, mol, m, s);
+        else batch_solve<DenseLds<48, WV>>(a, mol, m, s);
+    }
+}
+
+template <int WV>
+static size_t scf_lds_doubles(const std::vector<BMol> &mols, int *arena) {
+    int x = 0;
+    for (const BMol &m : mols)
+        x = std::max(x, m.n <= 16 ? scf_arena_doubles<DenseLds<16, WV>>(m.n)
+                                  : m.n <= 32 ? scf_arena_doubles<DenseLds<32, WV>>(m.n)
+                                              : scf_arena_doubles<DenseLds<48, WV>>(m.n));
+    *arena = x;
+    return x + scf_tail_doubles<WV>();
+}
+// bytes of LDS and the arena's doubles at `threads` per workgroup
+static size_t scf_lds_bytes(const std::vector<BMol> &mols, int threads, int *arena) {
+    const size_t d = threads == 64    ? scf_lds_doubles<1>(mols, arena)
+                     : threads == 128 ? scf_lds_doubles<2>(mols, arena)
+                     : threads == 256 ? scf_lds_doubles<4>(mols, arena)
+                                      : scf_lds_doubles<8>(mols, arena);
+    return sizeof(double) * d;
 }
 
 __global__ void k_zero_int(int *p, int cnt) {
@@ -735,6 +840,8 @@ __global__ void k_zero_int(int *p, int cnt) {
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+constexpr int kScfThreads = 256;   // of a batch that is not tuned; its LDS fits for every n
+
 struct BatchState {
     int nmol = 0, nmax = 0, npairs = 0, natom = 0;
     long long total_eri = 0, total_mat = 0, nq[6] = {0, 0, 0, 0, 0, 0};
@@ -762,7 +869,7 @@ struct BatchState {
     int gl_maxit = 0, gl_gen = -1;
     // launch shapes (autotuned) and the captured graph
     int eri_threads[6] = {256, 256, 256, 256, 256, 256};
-    int scf_threads = 256;
+    int scf_threads = kScfThreads;
     bool tuned = false;
     hipGraphExec_t graph = nullptr;
     bool graph_guess = false;
@@ -824,10 +931,11 @@ static void launch_batch_eri(myqc_ctx *ctx, BatchState &b, int c, int threads) {
     }
 }
 
-static int scf_grid(myqc_ctx *ctx, const BatchState &b) {
+// as many workgroups as the registers of the SCF kernel let a CU hold
+static int scf_grid(myqc_ctx *ctx, const BatchState &b, int threads) {
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
-    return std::max(1, std::min(b.nmol, 4 * cus));
+    return std::max(1, std::min(b.nmol, std::max(1024 / threads, 4) * cus));
 }
 
 // A start from the guess whose DIIS error is still above kCheckErr after
@@ -866,8 +974,15 @@ static void launch_batch_scf(myqc_ctx *ctx, BatchState &b, bool guess, double e_
     a.check_it = kCheckIt;
     a.check_err = kCheckErr;
     k_zero_int<<<1, 64, 0, ctx->stream>>>(b.d_counter, 1);
-    const int grid = std::max(1, std::min(scf_grid(ctx, b), a.nmol));
-    k_batch_scf<<<grid, threads, scf_lds_bytes(b.nmax, threads), ctx->stream>>>(a, b.nmax);
+    const int grid = std::max(1, std::min(scf_grid(ctx, b, threads), a.nmol));
+    int arena = 0;
+    const size_t lds = scf_lds_bytes(b.mols, threads, &arena);
+    switch (threads) {
+        case 64: k_batch_scf<1><<<grid, threads, lds, ctx->stream>>>(a, arena); break;
+        case 128: k_batch_scf<2><<<grid, threads, lds, ctx->stream>>>(a, arena); break;
+        case 256: k_batch_scf<4><<<grid, threads, lds, ctx->stream>>>(a, arena); break;
+        default: k_batch_scf<8><<<grid, threads, lds, ctx->stream>>>(a, arena); break;
+    }
 }
 
 // the whole pipeline: integrals, then the SCF
@@ -913,7 +1028,11 @@ static int batch_tune(myqc_ctx *ctx, BatchState &b, bool guess, double e_tol, do
     k_batch_one_e<<<(b.npairs + 127) / 128, 128, 0, ctx->stream>>>(b.d_pairs, b.d_prims, b.d_ftT, b.d_atoms,
                                                                    b.d_pair_mol, b.d_mols, b.npairs, b.d_S, b.d_H);
     float best = 1e30f;
+    int lds_limit = 65536;
+    (void)hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device);
     for (int th : {64, 128, 256, 512}) {
+        int arena = 0;
+        if (scf_lds_bytes(b.mols, th, &arena) > (size_t)lds_limit) continue;
         const float ms = timed([&] { launch_batch_scf(ctx, b, guess, e_tol, d_tol, max_iter, th); });
         if (ms < best) {
             best = ms;
@@ -1118,9 +1237,10 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     int lds_limit = 65536;
     (void)hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device);
-    if (scf_lds_bytes(b.nmax, 512) > (size_t)lds_limit)
+    int arena = 0;
+    if (scf_lds_bytes(b.mols, kScfThreads, &arena) > (size_t)lds_limit)
         return set_error(ctx, MYQC_E_ARG, "myqc_batch_set: n=%d needs %zu B of LDS per workgroup (limit %d)", b.nmax,
-                         scf_lds_bytes(b.nmax, 512), lds_limit);
+                         scf_lds_bytes(b.mols, kScfThreads, &arena), lds_limit);
     return 0;
 }
 

@@ -26,188 +26,19 @@
 #include <algorithm>
 
 #include "scf_small.h"
-#include "wave.h"
+#include "small_dense.h"
 
 namespace myqc {
 
-typedef double d4_t __attribute__((ext_vector_type(4)));
-
+// enough wavefronts for a tile or two each
 template <int NP>
-struct Sm {
-    static constexpr int LD = NP % 32 == 16 ? NP : NP == 96 ? NP + 1 : NP + 16;
-    static constexpr int NT = NP / 16, T2 = NT * NT, TU = NT * (NT + 1) / 2;
-    static constexpr int THREADS = NP <= 32 ? 256 : NP <= 48 ? 512 : 1024, WAVES = THREADS / 64;
-    static constexpr int MT = (T2 + WAVES - 1) / WAVES, MU = (TU + WAVES - 1) / WAVES;
-};
-
-__device__ __forceinline__ d4_t mfma64(double a, double b, d4_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// tile (ti, tj) of A B, B symmetric
-template <int NP>
-__device__ __forceinline__ d4_t tile_sym(const double *A, const double *B, int ti, int tj) {
-    constexpr int LD = Sm<NP>::LD;
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const double *pa = A + 16 * ti + c + LD * g, *pb = B + 16 * tj + c + LD * g;
-    d4_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < NP; k += 4) acc = mfma64(pa[LD * k], pb[LD * k], acc);
-    return acc;
-}
-
-// the wavefront's tiles w, w + WAVES, ... of A B (B symmetric)
-template <int NP>
-__device__ __forceinline__ void product(const double *A, const double *B, d4_t (&acc)[Sm<NP>::MT]) {
-    const int w = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < Sm<NP>::MT; ++q) {
-        const int tile = w + q * Sm<NP>::WAVES;
-        if (tile < Sm<NP>::T2) acc[q] = tile_sym<NP>(A, B, tile % Sm<NP>::NT, tile / Sm<NP>::NT);
-    }
-}
-
-// f(row, column, value) over the wavefront's tiles
-template <int NP, typename F>
-__device__ __forceinline__ void each(const d4_t (&acc)[Sm<NP>::MT], F f) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-#pragma unroll
-    for (int q = 0; q < Sm<NP>::MT; ++q) {
-        const int tile = w + q * Sm<NP>::WAVES;
-        if (tile >= Sm<NP>::T2) break;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            f(16 * (tile % Sm<NP>::NT) + g + 4 * v, 16 * (tile / Sm<NP>::NT) + c, acc[q][v]);
-    }
-}
-
-template <int NP>
-__device__ __forceinline__ void to_lds(double *M, const d4_t (&acc)[Sm<NP>::MT]) {
-    each<NP>(acc, [&](int i, int j, double v) { M[i + Sm<NP>::LD * j] = v; });
-}
-
-// M = scale times the n x n A, zero beyond
-template <int NP>
-__device__ __forceinline__ void load(double *M, const double *__restrict__ A, int n, double scale = 1.0) {
-    for (int e = threadIdx.x; e < NP * NP; e += Sm<NP>::THREADS) {
-        const int i = e % NP, j = e / NP;
-        M[i + Sm<NP>::LD * j] = (i < n && j < n) ? scale * A[i + n * j] : 0.0;
-    }
-}
-
-// sum (or maximum) over the workgroup of a value per thread; s: a double per wavefront
-template <int NP>
-__device__ __forceinline__ double wg_total(double v, double *s) {
-    v = wave_total(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return wave_total((threadIdx.x & 63) < Sm<NP>::WAVES ? s[threadIdx.x & 63] : 0.0);
-}
-// sum over each aligned 16 lanes
-__device__ __forceinline__ double row_total(double v) {
-    v = dpp_add<0xB1>(v);
-    v = dpp_add<0x4E>(v);
-    v = dpp_add<0x141>(v);
-    return dpp_add<0x140>(v);
-}
-__device__ __forceinline__ double wave_largest(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-template <int NP>
-__device__ __forceinline__ double wg_largest(double v, double *s) {
-    v = wave_largest(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return wave_largest(s[(threadIdx.x & 63) % Sm<NP>::WAVES]);
-}
-
-// Gershgorin bounds of the symmetric matrix in M
-template <int NP>
-__device__ __forceinline__ void bounds(const double *M, int n, double *s, double &lo, double &hi) {
-    // a wavefront per row
-    const int lane = threadIdx.x & 63;
-    double l = 1e300, h = -1e300;
-    for (int i = threadIdx.x >> 6; i < n; i += Sm<NP>::WAVES) {
-        double r = 0.0;
-        for (int j = lane; j < n; j += 64)
-            if (j != i) r += fabs(M[j + Sm<NP>::LD * i]);
-        r = wave_total(r);
-        const double c = M[i * (Sm<NP>::LD + 1)];
-        l = fmin(l, c - r);
-        h = fmax(h, c + r);
-    }
-    lo = -wg_largest<NP>(-l, s);
-    hi = wg_largest<NP>(h, s);
-}
-
-// DIIS coefficients c_0 .. c_{m-1} of the (m + 1) system, Gauss-Jordan with
-// column pivoting, by the first wavefront: lane r holds row r in registers.
-// Zeros with c[head] = 1 when the system is singular or m < 2.
-__device__ __forceinline__ bool diis_wave(const double *B, int m, int head, double *s_c) {
-    constexpr int MD = 8, W = MD + 2;
-    const int r = threadIdx.x & 63, N = m + 1;
-    double row[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) row[k] = 0.0;
-    if (r < m) {
-#pragma unroll
-        for (int k = 0; k < MD; ++k)
-            if (k < m) row[k] = B[r * MD + k];
-    }
-    // columns 0 .. m - 1 the B block, MD the border, MD + 1 the right side
-    if (r < m) row[MD] = -1.0;
-    if (r == m) {
-#pragma unroll
-        for (int k = 0; k < MD; ++k)
-            if (k < m) row[k] = -1.0;
-        row[MD + 1] = -1.0;
-    }
-    bool used = false, ok = m >= 2;
-    int mine = -1;   // the column this lane's row is the pivot of
-#pragma unroll
-    for (int col = 0; col <= MD; ++col) {
-        if (col < MD && col >= m) continue;   // (uniform)
-        const double v = (r < N && !used) ? fabs(row[col]) : -1.0;
-        double best = v;
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) best = fmax(best, __shfl_xor(best, off, 64));
-        best = lane_value(best, 0);   // (rows are lanes 0 .. 8 of the first 16)
-        if (!(best >= 1e-300)) ok = false;
-        const unsigned long long who = __ballot(r < 16 && v == best);
-        const int p = who ? __ffsll((long long)who) - 1 : 0;
-        double pr[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) pr[k] = lane_value(row[k], p);
-        if (r == p) {
-            used = true;
-            mine = col;
-        } else if (r < N) {
-            const double f = row[col] / pr[col];
-#pragma unroll
-            for (int k = 0; k < W; ++k) row[k] -= f * pr[k];
-            row[col] = 0.0;
-        }
-    }
-    ok = __ballot(!ok) == 0;
-    if (ok) {
-#pragma unroll
-        for (int k = 0; k < MD; ++k)
-            if (mine == k) s_c[k] = row[MD + 1] / row[k];
-    } else if (r < MD) {
-        s_c[r] = r == head ? 1.0 : 0.0;
-    }
-    return ok;
-}
+using Sm = DenseLds<NP, NP <= 32 ? 4 : NP <= 48 ? 8 : 16>;
 
 template <int NP>
 __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
     constexpr int LD = Sm<NP>::LD, MD = 8, MT = Sm<NP>::MT, MU = Sm<NP>::MU, TH = Sm<NP>::THREADS, WV = Sm<NP>::WAVES;
     __shared__ double sA[NP * LD], sB[NP * LD];
-    __shared__ double s_red[WV], s_part[2][8 * WV], s_sum[WV][MD + 2], s_c[MD], s_tot[MD + 2];
+    __shared__ double s_red[WV], s_part[16 * WV], s_sum[WV][MD + 2], s_c[MD], s_tot[MD + 2];
     const int n = a.n, nn = n * n, t = threadIdx.x, lane = t & 63, w = t >> 6;
     d4_t acc[MT];
     // F = H + G, with the energy sums and the density change
@@ -229,28 +60,28 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
         }
         sB[i + LD * j] = f;
     }
-    load<NP>(sA, a.X, n);
+    load<Sm<NP>>(sA, a.X, n);
     __syncthreads();
     // Fo = X F X: W = X F (F symmetric), then W X
-    product<NP>(sA, sB, acc);
+    product<Sm<NP>>(sA, sB, acc);
     __syncthreads();
-    to_lds<NP>(sB, acc);   // W
+    to_lds<Sm<NP>>(sB, acc);   // W
     __syncthreads();
-    product<NP>(sB, sA, acc);
+    product<Sm<NP>>(sB, sA, acc);
     __syncthreads();
-    to_lds<NP>(sA, acc);   // Fo
+    to_lds<Sm<NP>>(sA, acc);   // Fo
     double err = 0.0;
     if (!a.core) {
         double *fs = a.hF + (size_t)nn * a.head, *es = a.hE + (size_t)nn * a.head;
-        each<NP>(acc, [&](int i, int j, double v) {
+        each<Sm<NP>>(acc, [&](int i, int j, double v) {
             if (i < n && j < n) fs[i + n * j] = v;
         });
-        load<NP>(sB, a.Do, n);
+        load<Sm<NP>>(sB, a.Do, n);
         __syncthreads();
         // the error Fo Do - Do Fo, and its products with the history
-        product<NP>(sA, sB, acc);
+        product<Sm<NP>>(sA, sB, acc);
         __syncthreads();
-        to_lds<NP>(sB, acc);
+        to_lds<Sm<NP>>(sB, acc);
         __syncthreads();
         double dot[MD];
 #pragma unroll
@@ -315,7 +146,7 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
             sA[i + LD * j] = v;
         }
     } else {
-        each<NP>(acc, [&](int i, int j, double v) {
+        each<Sm<NP>>(acc, [&](int i, int j, double v) {
             if (i < n && j < n) a.Fx[i + n * j] = v;
         });
     }
@@ -329,85 +160,7 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
         }
         __syncthreads();
     } else {
-        double lo, hi;
-        bounds<NP>(sA, n, s_red, lo, hi);
-        const double sc = 1.0 / (hi - lo);
-        const int g = lane >> 4, c = lane & 15;
-        // the wavefront's upper tiles of P^2
-        int ti[MU], tj[MU];
-#pragma unroll
-        for (int q = 0; q < MU; ++q) {
-            int rem = w + q * WV, col = 0;
-            while (rem > col) rem -= ++col;
-            ti[q] = rem;
-            tj[q] = col;
-        }
-        // tr P and ||P||^2: each 16 lanes' sums go to LDS when P is written,
-        // and every wavefront adds the partial sums up for itself
-        double tr = 0.0, fr = 0.0;
-        __syncthreads();
-        for (int e = t; e < NP * NP; e += TH) {
-            const int i = e % NP, j = e / NP;
-            double v = 0.0;
-            if (i < n && j < n) {
-                v = ((i == j ? hi : 0.0) - sA[i + LD * j]) * sc;
-                fr += v * v;
-                if (i == j) tr += v;
-            }
-            sB[i + LD * j] = v;
-        }
-        const double nocc = a.nocc;
-        int cs = -1;
-        ok = 0;
-        // P_k and P_{k+1} take turns in the two arrays: one barrier per step
-        const double *P = sB;
-        double *Pn = sA;
-        for (int step = 0; step <= 120; ++step) {
-            double *part = s_part[step & 1];
-            tr = row_total(tr);
-            fr = row_total(fr);
-            if (c == 0) {
-                part[4 * w + g] = tr;
-                part[4 * WV + 4 * w + g] = fr;
-            }
-            __syncthreads();   // P and its sums are complete; P_{k-1} is free
-            const double pt = lane < 4 * WV ? part[lane] : 0.0, pf = lane < 4 * WV ? part[4 * WV + lane] : 0.0;
-            d4_t p2[MU];
-#pragma unroll
-            for (int q = 0; q < MU; ++q)
-                if (w + q * WV < Sm<NP>::TU) p2[q] = tile_sym<NP>(P, P, ti[q], tj[q]);
-            tr = wave_total(pt);
-            fr = wave_total(pf);
-            if (cs < 0 && step >= 8 && fabs(tr - fr) < 1e-8 && fabs(tr - nocc) < 1e-6) cs = step;
-            if (cs >= 0 && step >= cs + 2) {
-                ok = 1;
-                steps = step;
-                break;
-            }
-            if (step == 120) break;
-            const bool square = fabs(fr - nocc) < fabs(2.0 * tr - fr - nocc);
-            tr = fr = 0.0;
-#pragma unroll
-            for (int q = 0; q < MU; ++q) {
-                if (w + q * WV >= Sm<NP>::TU) break;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int i = 16 * ti[q] + g + 4 * v, j = 16 * tj[q] + c;
-                    const double nw = square ? p2[q][v] : 2.0 * P[i + LD * j] - p2[q][v];
-                    Pn[i + LD * j] = nw;
-                    if (ti[q] != tj[q]) Pn[j + LD * i] = nw;
-                    fr += (ti[q] != tj[q] ? 2.0 : 1.0) * nw * nw;
-                    if (i == j) tr += nw;
-                }
-            }
-            double *x = const_cast<double *>(P);
-            P = Pn;
-            Pn = x;
-        }
-        if (ok && P != sA) {   // (uniform) into sA, where the rest expects it
-            __syncthreads();
-            for (int e = t; e < NP * LD; e += TH) sA[e] = sB[e];
-        }
+        ok = purify<Sm<NP>>(sA, sB, n, a.nocc, 120, s_red, s_part, steps);
         __syncthreads();
     }
     if (t == 0) {
@@ -417,113 +170,25 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
     if (!ok) return;   // (uniform) the host takes the eigenvectors of Fx
     // the projector, and D = 2 X P X
     for (int e = t; e < nn; e += TH) a.Don[e] = sA[e % n + LD * (e / n)];
-    load<NP>(sB, a.X, n);
+    load<Sm<NP>>(sB, a.X, n);
     __syncthreads();
-    product<NP>(sB, sA, acc);   // X P
+    product<Sm<NP>>(sB, sA, acc);   // X P
     __syncthreads();
-    to_lds<NP>(sA, acc);
+    to_lds<Sm<NP>>(sA, acc);
     __syncthreads();
-    product<NP>(sA, sB, acc);
-    each<NP>(acc, [&](int i, int j, double v) {
+    product<Sm<NP>>(sA, sB, acc);
+    each<Sm<NP>>(acc, [&](int i, int j, double v) {
         if (i < n && j < n) a.Dnext[i + n * j] = 2.0 * v;
     });
 }
 
-// X = S^-1/2 and Xi = S^1/2 by the coupled Newton-Schulz iteration of
-// inv_sqrt_ns (scf.hip): A = S / c, T = (3 I - Z Y) / 2, Y <- Y T, Z <- T Z; Y and Z
-// in memory, T and one of them in LDS.  The iteration is stable only with
-// the products as they stand: although Y, Z and T are symmetric up to
-// rounding, reading a right operand by rows (its transpose), or mirroring a
-// product's upper half, diverges from condition numbers of 1e3 on.  The
-// right operand is read down its columns, and the leading dimension is odd,
-// which leaves a two-way bank conflict.
+// X = S^-1/2 and Xi = S^1/2 (small_dense.h); out[0] = 1, or 0 if they were not reached
 template <int NP>
 __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_inv_sqrt(int n, const double *__restrict__ S, double *X,
                                                                     double *Xi, double *Y, double *Z, double *out) {
-    constexpr int LD = NP + 1, MT = Sm<NP>::MT, TH = Sm<NP>::THREADS;
-    __shared__ double sA[NP * LD], sB[NP * LD], s_red[Sm<NP>::WAVES];
-    const int t = threadIdx.x, nn = n * n, w = t >> 6, lane = t & 63, g = lane >> 4, cc = lane & 15;
-    auto fill = [&](double *M, const double *A) {
-        for (int e = t; e < NP * NP; e += TH) {
-            const int i = e % NP, j = e / NP;
-            M[i + LD * j] = (i < n && j < n) ? A[i + n * j] : 0.0;
-        }
-    };
-    d4_t acc[MT];
-    auto mul = [&](const double *A, const double *B) {
-#pragma unroll
-        for (int q = 0; q < MT; ++q) {
-            const int tile = w + q * Sm<NP>::WAVES;
-            if (tile >= Sm<NP>::T2) break;
-            const double *pa = A + 16 * (tile % Sm<NP>::NT) + cc + LD * g;
-            const double *pb = B + LD * (16 * (tile / Sm<NP>::NT) + cc) + g;
-            acc[q] = (d4_t){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int k = 0; k < NP; k += 4) acc[q] = mfma64(pa[LD * k], pb[k], acc[q]);
-        }
-    };
-    // Gershgorin's upper bound
-    double c = -1e300;
-    for (int i = t; i < n; i += TH) {
-        double r = S[i * (n + 1)];
-        for (int j = 0; j < n; ++j)
-            if (j != i) r += fabs(S[j + n * i]);
-        c = fmax(c, r);
-    }
-    c = wg_largest<NP>(c, s_red);
-    if (!(c > 0.0)) {
-        if (t == 0) out[0] = 0.0;
-        return;
-    }
-    for (int e = t; e < nn; e += TH) {
-        Y[e] = S[e] / c;
-        Z[e] = e % n == e / n ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    int extra = -1, done = 0;
-    for (int k = 0; k < 40; ++k) {
-        fill(sA, Z);
-        fill(sB, Y);
-        __syncthreads();
-        mul(sA, sB);   // Z Y
-        double far = 0.0;
-        each<NP>(acc, [&](int i, int j, double v) {
-            if (i >= n || j >= n) return;
-            const double d = fabs(v - (i == j ? 1.0 : 0.0));
-            far = fmax(far, d < 1e300 ? d : 1e300);   // (not a number counts as far)
-        });
-        far = wg_largest<NP>(far, s_red);   // (its barriers also end the reads of sA)
-        if (extra == 0) {
-            done = 1;
-            break;
-        }
-        // quadratic convergence: one more step takes 1e-9 below round-off
-        if (extra < 0 && far < 1e-9) extra = 1;
-        each<NP>(acc, [&](int i, int j, double v) {
-            sA[i + LD * j] = (i < n && j < n) ? (i == j ? 1.5 : 0.0) - 0.5 * v : 0.0;
-        });
-        __syncthreads();
-        mul(sB, sA);   // Y T
-        __syncthreads();
-        each<NP>(acc, [&](int i, int j, double v) {
-            if (i < n && j < n) Y[i + n * j] = v;
-        });
-        fill(sB, Z);
-        __syncthreads();
-        mul(sA, sB);   // T Z
-        __syncthreads();
-        each<NP>(acc, [&](int i, int j, double v) {
-            if (i < n && j < n) Z[i + n * j] = v;
-        });
-        __syncthreads();
-        if (extra > 0) --extra;
-    }
-    const double rc = sqrt(c);
-    for (int e = t; e < nn; e += TH) {
-        X[e] = Z[e] / rc;
-        Xi[e] = Y[e] * rc;
-    }
-    if (t == 0) out[0] = done;
+    __shared__ double sM[2 * NP * (NP + 1)], s_red[Sm<NP>::WAVES];
+    const bool ok = inv_sqrt_ns<Sm<NP>>(n, S, X, Xi, Y, Z, sM, s_red, 40);
+    if (threadIdx.x == 0) out[0] = ok ? 1.0 : 0.0;
 }
 
 // Eigenvalues (ascending) and C = X U by cyclic Jacobi, round-robin pairs: the
@@ -538,7 +203,7 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_orbitals(int n, const
     __shared__ int s_p[NP / 2], s_q[NP / 2], s_at[NP];
     const int t = threadIdx.x;
     const int npad = n + (n & 1), half = npad >> 1;
-    load<NP>(sA, Fo, n);
+    load<Sm<NP>>(sA, Fo, n);
     for (int e = t; e < NP * NP; e += TH) sU[e % NP + LD * (e / NP)] = e % NP == e / NP ? 1.0 : 0.0;
     __syncthreads();
     for (int sweep = 0; sweep < 40; ++sweep) {
@@ -548,8 +213,8 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_orbitals(int n, const
             if (e % NP == e / NP) dia += v * v;
             else off += v * v;
         }
-        off = wg_total<NP>(off, s_red);
-        dia = wg_total<NP>(dia, s_red);
+        off = wg_total<Sm<NP>>(off, s_red);
+        dia = wg_total<Sm<NP>>(dia, s_red);
         if (!(off > 1e-30 * dia)) break;
         for (int r = 0; r < npad - 1; ++r) {
             for (int k = t; k < half; k += TH) {
@@ -612,7 +277,7 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_orbitals(int n, const
     }
     __syncthreads();
     // C = X U, columns to their places
-    load<NP>(sA, X, n);
+    load<Sm<NP>>(sA, X, n);
     __syncthreads();
     const int w = t >> 6, lane = t & 63, g = lane >> 4, c = lane & 15;
     for (int tile = w; tile < Sm<NP>::T2; tile += WV) {
