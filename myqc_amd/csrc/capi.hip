@@ -68,7 +68,6 @@ extern "C" int myqc_finalize(myqc_ctx *ctx) {
                      (void **)&ctx->d_A32,   (void **)&ctx->d_iajb, (void **)&ctx->d_planes, (void **)&ctx->d_dmax,
                      (void **)&ctx->d_q12,   (void **)&ctx->d_q3,   (void **)&ctx->d_xwork, &ctx->d_dtab};
     for (auto p : ptrs) dfree(p);
-    for (int c = 0; c < 3; ++c) dfree((void **)&ctx->d_sorted[c]);
     for (int c = 0; c < 3; ++c) dfree((void **)&ctx->d_ksoa[c]);
     for (int c = 0; c < 3; ++c) dfree((void **)&ctx->d_uhf[c]);
     for (int c = 0; c < 2; ++c) dfree((void **)&ctx->d_vvoo[c]);

@@ -65,14 +65,13 @@ struct myqc_ctx {
     std::vector<double> xyz;              // [atom][3]
     std::vector<myqc::Shell> shells;
     std::vector<myqc::ShellPair> pairs;
-    std::vector<myqc::PrimPair> prims;
     std::vector<int> pair_ids[3];         // per pair class, sorted by Schwarz value (descending)
     std::vector<double> schwarz;          // per pair
     std::vector<double> ftT;              // the Boys tables' inputs (boys_inputs)
     myqc::ShellPair *d_pairs = nullptr;
     myqc::PrimPair *d_prims = nullptr;
     double *d_ftT = nullptr;
-    int *d_sorted[3] = {nullptr, nullptr, nullptr};
+    int *d_sorted[3] = {nullptr, nullptr, nullptr};   // the sorted pairs of each class (in d_schwarz's allocation)
     // per class, the primitive pairs of the sorted pairs as structure of
     // arrays: field f of primitive j of rank r at [(j * kKetFields + f) * np + r]
     double *d_ksoa[3] = {nullptr, nullptr, nullptr};
@@ -248,7 +247,7 @@ int blas_reserve(myqc_ctx *ctx, F calls) {
 }
 
 // slots of ctx->d_tmp
-enum TmpSlot { TMP_S = 0, TMP_H, TMP_ATOMS, TMP_GPAIRS, TMP_GATOMS, TMP_GDENS, TMP_GMOL, TMP_CA, TMP_CB, TMP_NSLOT };
+enum TmpSlot { TMP_S = 0, TMP_H, TMP_ATOMS, TMP_GPAIRS, TMP_GATOMS, TMP_GDENS, TMP_GMOL, TMP_CA, TMP_CB, TMP_SHELLS, TMP_FOCK, TMP_NSLOT };
 static_assert(TMP_NSLOT <= 16, "d_tmp slots");
 // a temporary of at least `bytes` in slot `slot`, kept by the context
 template <typename T>

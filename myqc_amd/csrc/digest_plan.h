@@ -72,6 +72,7 @@ struct DigestPlan {
     int n = 0, ns = 0, np = 0;
     int max_rows = 0;                    // LDS rows of one workgroup at most
     std::vector<int> rank, pcls;         // per pair: rank within its class, class
+    std::vector<std::vector<int>> of_a;  // per row shell, its pairs (pairs_by_row_shell)
     std::vector<int> lo, hi;             // [p*3+ck] ket ranks of which p is the bra
     std::vector<long long> off;          // [p*3+ck] element e of ket rank r at off + r + e*(hi - lo)
     long long n_values = 0;              // stored (pre-weighted) values
@@ -96,8 +97,9 @@ inline std::vector<std::vector<int>> pairs_by_row_shell(int ns, const std::vecto
                                                          const std::vector<ShellPair> &pairs) {
     std::vector<std::vector<int>> of_a(ns);
     for (int p = 0; p < (int)pairs.size(); ++p) of_a[pairs[p].sa].push_back(p);
-    for (auto &v : of_a)
-        std::sort(v.begin(), v.end(), [&](int x, int y) { return shells_ao[pairs[x].sb] < shells_ao[pairs[y].sb]; });
+    auto before = [&](int x, int y) { return shells_ao[pairs[x].sb] < shells_ao[pairs[y].sb]; };
+    for (auto &v : of_a)   // (build_pairs makes them in this order)
+        if (!std::is_sorted(v.begin(), v.end(), before)) std::sort(v.begin(), v.end(), before);
     return of_a;
 }
 
@@ -150,7 +152,8 @@ inline std::string build_digest_layout(DigestPlan &pl, int n, const std::vector<
             }
         }
     // value offsets, pairs grouped by row shell
-    const auto of_a = pairs_by_row_shell(ns, shells_ao, pairs);
+    pl.of_a = pairs_by_row_shell(ns, shells_ao, pairs);
+    const auto &of_a = pl.of_a;
     pl.off.assign((size_t)np * 3, 0);
     long long off = 0;
     for (int A = 0; A < ns; ++A)
@@ -178,7 +181,7 @@ inline std::string build_digest_schedule(DigestPlan &pl, const std::vector<int> 
     const int ns = pl.ns, np = pl.np, n = pl.n;
     pl.max_rows = max_rows;
     if (max_rows < 6) return "digestion: too few LDS rows for one p-shell row pair";
-    const auto of_a = pairs_by_row_shell(ns, shells_ao, pairs);
+    const auto &of_a = pl.of_a;
     // J-ket layout and the pair -> J-ket block map
     pl.jk_base.assign(4, 0);
     for (int c = 0; c < 3; ++c) pl.jk_base[c + 1] = pl.jk_base[c] + (int)pair_ids[c].size() * dig_ncd(c);

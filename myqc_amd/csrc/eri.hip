@@ -250,7 +250,8 @@ constexpr int kSchwarzLanes = 8, kSchwarzPairs = 256 / kSchwarzLanes;
 
 template <int C>
 __device__ __forceinline__ void schwarz_pair(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
-                                             const double *__restrict__ ftT, double *s_ft, int p, bool on, int sub, double *__restrict__ q) {
+                                             const double *__restrict__ ftT, double *s_ft, int p, bool on, int sub, double *__restrict__ q,
+                                             int *__restrict__ rank) {
     constexpr int LA = PairL<C>::a, LB = PairL<C>::b;
     constexpr int na = ncart(LA), nb = ncart(LB);
     const BoysTab ft = stage_boys<2 * C>(ftT, s_ft);
@@ -270,7 +271,10 @@ __device__ __forceinline__ void schwarz_pair(const ShellPair *__restrict__ pairs
     for (int ia = 0; ia < na; ++ia)
 #pragma unroll
         for (int ib = 0; ib < nb; ++ib) m = fmax(m, fabs(out[((ia * nb + ib) * na + ia) * nb + ib]));
-    if (on && sub == 0) q[p] = sqrt(m);
+    if (on && sub == 0) {
+        q[p] = sqrt(m);
+        rank[p] = 0;
+    }
 }
 
 struct SchwarzArgs {
@@ -280,16 +284,83 @@ struct SchwarzArgs {
 };
 
 __global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
-                                                 const double *__restrict__ ftT, SchwarzArgs a, double *__restrict__ q) {
+                                                 const double *__restrict__ ftT, SchwarzArgs a, double *__restrict__ q,
+                                                 int *__restrict__ rank) {
     __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(4)];
     const int b = blockIdx.x, c = b >= a.blk[0] ? 0 : b >= a.blk[1] ? 1 : 2;
     // lanes past the last pair repeat it (the group sums need every lane)
     const int t = (b - a.blk[c]) * kSchwarzPairs + threadIdx.x / kSchwarzLanes, sub = threadIdx.x % kSchwarzLanes;
     const bool on = t < a.np[c];
     const int p = a.ids[c][on ? t : a.np[c] - 1];
-    if (c == 0) schwarz_pair<0>(pairs, prims, ftT, s_ft, p, on, sub, q);
-    else if (c == 1) schwarz_pair<1>(pairs, prims, ftT, s_ft, p, on, sub, q);
-    else schwarz_pair<2>(pairs, prims, ftT, s_ft, p, on, sub, q);
+    if (c == 0) schwarz_pair<0>(pairs, prims, ftT, s_ft, p, on, sub, q, rank);
+    else if (c == 1) schwarz_pair<1>(pairs, prims, ftT, s_ft, p, on, sub, q, rank);
+    else schwarz_pair<2>(pairs, prims, ftT, s_ft, p, on, sub, q, rank);
+}
+
+// The order of each class by Schwarz factor, largest first (ties by position,
+// which is by pair id): a pair's rank is the number of pairs before it.  Every
+// comparison of a class is made, n^2 of them, a tile of keys in LDS at a time:
+// for 12880 pairs that is less than a radix sort's launches take, and the host
+// sort it replaces took 0.5 ms with the GPU idle.  The keys are the factors'
+// bits (non-negative, so ordered like them; not-a-number has its place too).
+constexpr int kRankTile = 1024;
+__global__ __launch_bounds__(256) void k_rank(SchwarzArgs a, const double *__restrict__ q, int *__restrict__ rank) {
+    __shared__ unsigned long long s_key[kRankTile];
+    const int b = blockIdx.x, c = b >= a.blk[0] ? 0 : b >= a.blk[1] ? 1 : 2;
+    const int np = a.np[c], i = (b - a.blk[c]) * 256 + threadIdx.x, j0 = blockIdx.y * kRankTile;
+    if (j0 >= np) return;
+    const int nj = min(kRankTile, np - j0);
+    for (int j = threadIdx.x; j < nj; j += 256) s_key[j] = __double_as_longlong(q[a.ids[c][j0 + j]]);
+    __syncthreads();
+    if (i >= np) return;
+    const int p = a.ids[c][i];
+    const unsigned long long key = __double_as_longlong(q[p]);
+    int before = 0;
+    for (int j = 0; j < nj; ++j) before += s_key[j] > key || (s_key[j] == key && j0 + j < i) ? 1 : 0;
+    if (before) atomicAdd(&rank[p], before);
+}
+// sorted (the three classes one after another, as ids)
+__global__ __launch_bounds__(256) void k_by_rank(const int *__restrict__ ids, const int *__restrict__ rank, int np0,
+                                                 int np1, int np, int *__restrict__ sorted) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= np) return;
+    const int first = i < np0 ? 0 : i < np0 + np1 ? np0 : np0 + np1, p = ids[i];
+    sorted[first + rank[p]] = p;
+}
+
+// The shells as k_prim_pairs reads them: kShellDoubles each
+constexpr int kShellPrims = 6, kShellDoubles = 16;   // exponents, coefficients, centre, primitives
+
+// The primitive pairs of every shell pair (fill_prims, system.h), a thread
+// each: its place is the number of the pair's primitives with a larger screen
+// factor (or an equal one and before it).  The host took 18 ms of core time for
+// the 181k of 40 waters and sent 17 MB.
+__global__ __launch_bounds__(256) void k_prim_pairs(const ShellPair *__restrict__ pairs, int npairs, int most,
+                                                    const double *__restrict__ shells, PrimPair *__restrict__ prims) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= (long long)npairs * most) return;
+    const ShellPair sp = pairs[t / most];
+    const int x = (int)(t % most);
+    if (x >= sp.npp) return;
+    const double *A = shells + kShellDoubles * sp.sa, *B = shells + kShellDoubles * sp.sb;
+    const int nb = (int)B[kShellDoubles - 1];
+    const double ab2 = sp.AB[0] * sp.AB[0] + sp.AB[1] * sp.AB[1] + sp.AB[2] * sp.AB[2];
+    auto screen = [&](int y) {
+        const double aa = A[y / nb], bb = B[y % nb];
+        return exp(-aa * bb * ab2 / (aa + bb));
+    };
+    // (not a number: before every number, so that each still has its own place)
+    auto key = [](double e) { return e == e ? e : 2.0; };
+    const double e = screen(x);
+    int place = 0;
+    for (int y = 0; y < sp.npp; ++y) {
+        const double f = key(screen(y));
+        place += f > key(e) || (f == key(e) && y < x) ? 1 : 0;
+    }
+    PrimPair pp;
+    prim_pair(pp, A[x / nb], B[x % nb], A[kShellPrims + x / nb], B[kShellPrims + x % nb], A + 2 * kShellPrims,
+              B + 2 * kShellPrims, e);
+    prims[sp.pp0 + place] = pp;
 }
 
 // ---------------------------------------------------------------------------
@@ -328,59 +399,52 @@ void free_eri(myqc_ctx *ctx, bool keep_memory) {
 int eri_schwarz(myqc_ctx *ctx) {
     if (ctx->have_schwarz) return 0;
     const int np = (int)ctx->pairs.size();
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_schwarz, sizeof(double) * np));
-    SchwarzArgs sa{};
-    int nblk = 0;
-    for (int c = 2; c >= 0; --c) {
-        const auto &ids = ctx->pair_ids[c];
-        sa.blk[c] = nblk;
-        sa.np[c] = (int)ids.size();
-        if (ids.empty()) continue;
-        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_sorted[c], sizeof(int) * ids.size()));
-        MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_sorted[c], ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice,
-                                     ctx->stream));
-        sa.ids[c] = ctx->d_sorted[c];
-        nblk += ((int)ids.size() + kSchwarzPairs - 1) / kSchwarzPairs;
-    }
-    k_schwarz<<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, sa, ctx->d_schwarz);
-    MYQC_HIP(ctx, hipGetLastError());
-    ctx->schwarz.resize(np);
-    MYQC_HIP(ctx, hipMemcpyAsync(ctx->schwarz.data(), ctx->d_schwarz, sizeof(double) * np, hipMemcpyDeviceToHost,
-                                 ctx->stream));
-    MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     for (const ShellPair &sp : ctx->pairs)
         if (sp.npp > kKetPrims)
             return set_error(ctx, MYQC_E_ARG, "a shell pair has %d primitive pairs (at most %d: STO-3G shells)",
                              sp.npp, kKetPrims);
-    // sort each class by Schwarz factor, largest first (ties by pair id); one
-    // host thread per class
-    {
-        auto sort_class = [ctx](int c) {
-            auto &ids = ctx->pair_ids[c];
-            std::vector<std::pair<double, int>> key(ids.size());
-            for (size_t r = 0; r < ids.size(); ++r) key[r] = {-ctx->schwarz[ids[r]], ids[r]};
-            std::sort(key.begin(), key.end());   // descending factor, ties by pair id
-            for (size_t r = 0; r < ids.size(); ++r) ids[r] = key[r].second;
-        };
-        std::thread t1(sort_class, 1), t2(sort_class, 2);
-        sort_class(0);
-        t1.join();
-        t2.join();
-    }
+    // one allocation: the factors and the sorted pairs (which the host takes
+    // together), then ranks and the pairs by class
+    const size_t back = (sizeof(double) + sizeof(int)) * (size_t)np;
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_schwarz, back + 2 * sizeof(int) * (size_t)np));
+    int *sorted = reinterpret_cast<int *>(ctx->d_schwarz + np), *rank = sorted + np, *ids = rank + np;
+    std::vector<int> all;
+    all.reserve(np);
+    SchwarzArgs sa{}, ra{};
+    int nblk = 0, nrank = 0, most = 0;
     for (int c = 0; c < 3; ++c) {
-        auto &ids = ctx->pair_ids[c];
-        if (!ids.empty()) {
-            MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_sorted[c], ids.data(), sizeof(int) * ids.size(),
-                                         hipMemcpyHostToDevice, ctx->stream));
-            const int np = (int)ids.size();
-            MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_ksoa[c], sizeof(double) * kKetPrims * kKetFields * (size_t)np));
-            k_ket_soa<<<dim3((np + 255) / 256, kKetPrims), 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims,
-                                                                                  ctx->d_sorted[c], np,
-                                                                                  ctx->d_ksoa[c]);
-            MYQC_HIP(ctx, hipGetLastError());
-        }
+        ctx->d_sorted[c] = sorted + all.size();
+        sa.ids[c] = ra.ids[c] = ids + all.size();
+        sa.np[c] = ra.np[c] = (int)ctx->pair_ids[c].size();
+        most = std::max(most, sa.np[c]);
+        all.insert(all.end(), ctx->pair_ids[c].begin(), ctx->pair_ids[c].end());
     }
+    for (int c = 2; c >= 0; --c) {
+        sa.blk[c] = nblk;
+        ra.blk[c] = nrank;
+        nblk += (sa.np[c] + kSchwarzPairs - 1) / kSchwarzPairs;
+        nrank += (sa.np[c] + 255) / 256;
+    }
+    MYQC_HIP(ctx, hipMemcpyAsync(ids, all.data(), sizeof(int) * np, hipMemcpyHostToDevice, ctx->stream));
+    k_schwarz<<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, sa, ctx->d_schwarz, rank);
+    k_rank<<<dim3(nrank, (most + kRankTile - 1) / kRankTile), 256, 0, ctx->stream>>>(ra, ctx->d_schwarz, rank);
+    k_by_rank<<<(np + 255) / 256, 256, 0, ctx->stream>>>(ids, rank, sa.np[0], sa.np[1], np, sorted);
+    for (int c = 0; c < 3; ++c) {
+        if (sa.np[c] == 0) continue;
+        MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_ksoa[c], sizeof(double) * kKetPrims * kKetFields * (size_t)sa.np[c]));
+        k_ket_soa<<<dim3((sa.np[c] + 255) / 256, kKetPrims), 256, 0, ctx->stream>>>(
+            ctx->d_pairs, ctx->d_prims, ctx->d_sorted[c], sa.np[c], ctx->d_ksoa[c]);
+    }
+    MYQC_HIP(ctx, hipGetLastError());
+    std::vector<double> host((back + sizeof(double) - 1) / sizeof(double));
+    MYQC_HIP(ctx, hipMemcpyAsync(host.data(), ctx->d_schwarz, back, hipMemcpyDeviceToHost, ctx->stream));
     MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->schwarz.assign(host.begin(), host.begin() + np);
+    const int *order = reinterpret_cast<const int *>(host.data() + np);
+    for (int c = 0; c < 3; ++c) {
+        ctx->pair_ids[c].assign(order, order + sa.np[c]);
+        order += sa.np[c];
+    }
     ctx->have_schwarz = true;
     return 0;
 }
@@ -792,19 +856,35 @@ extern "C" int myqc_set_system(myqc_ctx *ctx, int nnuc, const int *Z, const doub
     ctx->xyz.resize(3 * nnuc);
     for (int a = 0; a < nnuc; ++a)
         for (int c = 0; c < 3; ++c) ctx->xyz[3 * a + c] = xyz_bohr[a + nnuc * c];
-    const std::string why = build_system(nnuc, ctx->xyz.data(), nset, set_alpha, setinfo, bas, norb, basinfo,
-                                         ctx->shells, ctx->pairs, ctx->prims, ctx->pair_ids);
+    size_t nprims = 0;
+    const std::string why = build_pairs(nnuc, nset, set_alpha, setinfo, bas, norb, basinfo, ctx->xyz.data(),
+                                        ctx->shells, ctx->pairs, nprims, ctx->pair_ids);
     if (!why.empty()) return set_error(ctx, MYQC_E_ARG, "myqc_set_system: %s", why.c_str());
     hc.mark("set_system: shells and pairs");
+    const int np = (int)ctx->pairs.size();
+    int most = 0;
+    std::vector<double> sh(kShellDoubles * ctx->shells.size(), 0.0);
+    for (size_t k = 0; k < ctx->shells.size(); ++k) {
+        const Shell &x = ctx->shells[k];
+        double *d = sh.data() + kShellDoubles * k;
+        std::copy(x.alpha.begin(), x.alpha.end(), d);
+        std::copy(x.coef.begin(), x.coef.end(), d + kShellPrims);
+        std::copy(&ctx->xyz[3 * x.center], &ctx->xyz[3 * x.center] + 3, d + 2 * kShellPrims);
+        d[kShellDoubles - 1] = (double)x.alpha.size();
+        most = std::max(most, (int)(x.alpha.size() * x.alpha.size()));
+    }
     ctx->ftT.resize(FT_TOTAL - FT_EG);
     boys_inputs(Ftab, ctx->ftT.data());
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_pairs, sizeof(ShellPair) * ctx->pairs.size()));
-    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_prims, sizeof(PrimPair) * ctx->prims.size()));
+    double *d_sh = nullptr;
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_pairs, sizeof(ShellPair) * np));
+    MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_prims, sizeof(PrimPair) * nprims));
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_ftT, sizeof(double) * FT_TOTAL));
-    MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_pairs, ctx->pairs.data(), sizeof(ShellPair) * ctx->pairs.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
-    MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_prims, ctx->prims.data(), sizeof(PrimPair) * ctx->prims.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
+    MYQC_CHECK(dtmp(ctx, TMP_SHELLS, &d_sh, sizeof(double) * sh.size()));
+    MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_pairs, ctx->pairs.data(), sizeof(ShellPair) * np, hipMemcpyHostToDevice,
+                                 ctx->stream));
+    MYQC_HIP(ctx, hipMemcpyAsync(d_sh, sh.data(), sizeof(double) * sh.size(), hipMemcpyHostToDevice, ctx->stream));
+    k_prim_pairs<<<(unsigned)(((long long)np * most + 255) / 256), 256, 0, ctx->stream>>>(ctx->d_pairs, np, most, d_sh,
+                                                                                         ctx->d_prims);
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_ftT + FT_EG, ctx->ftT.data(), sizeof(double) * ctx->ftT.size(),
                                  hipMemcpyHostToDevice, ctx->stream));
     k_boys_rows<<<kBoysRowBlocks, 64, 0, ctx->stream>>>(ctx->d_ftT);

@@ -15,7 +15,6 @@
 #include <algorithm>
 #include <cmath>
 #include <map>
-#include <thread>
 #include <string>
 #include <vector>
 
@@ -34,11 +33,30 @@ inline double gto_norm(int l, double a) {
     return pow(128.0 * pow(a, 5.0) / pow(PI_SP, 3.0), 1.0 / 4.0);
 }
 
+// One primitive pair: exponents, coefficients and centres of the two
+// primitives, and their screen factor e = exp(-aa bb |RA - RB|^2 / (aa + bb))
+// (int2e.f90:223)
+MYQC_HD void prim_pair(PrimPair &pp, double aa, double bb, double ca, double cb, const double *RA, const double *RB,
+                       double e) {
+    const double p = aa + bb;
+    pp.p = p;
+    for (int d = 0; d < 3; ++d) {
+        pp.P[d] = (aa * RA[d] + bb * RB[d]) / p;
+        pp.PA[d] = pp.P[d] - RA[d];
+    }
+    pp.EIJ = e;
+    pp.K = e * ca * cb;
+    pp.beta = bb;
+    pp.ip = 1.0 / p;
+    pp.KI = pp.K * pp.ip;
+}
+
+// Shells and shell pairs; nprims: the primitive pairs of all of them.
 // Returns an empty string on success, else the reason.
-inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int nset, const double *set_alpha,
-                                const int *setinfo, const double *bas, int norb, const int *basinfo,
-                                std::vector<Shell> &shells, std::vector<ShellPair> &pairs,
-                                std::vector<PrimPair> &prims, std::vector<int> pair_ids[3]) {
+inline std::string build_pairs(int nnuc, int nset, const double *set_alpha, const int *setinfo, const double *bas,
+                               int norb, const int *basinfo, const double *xyz /*[atom][3]*/,
+                               std::vector<Shell> &shells, std::vector<ShellPair> &pairs, size_t &nprims,
+                               std::vector<int> pair_ids[3]) {
     char buf[256];
     if (setinfo[0] != nset || basinfo[1] != norb) return "setinfo/basinfo headers disagree with nset/norb";
     const int setl = setinfo[1], OpS = basinfo[0];
@@ -94,21 +112,10 @@ inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int n
             return buf;
         }
     pairs.clear();
-    prims.clear();
     for (int c = 0; c < 3; ++c) pair_ids[c].clear();
     const int ns = (int)shells.size();
-    // pairs first (cheap), then their primitive pairs in parallel: each pair
-    // owns the slice [pp0, pp0 + npp) of prims, which is sized once
-    {
-        size_t npairs = 0, nprims = 0;
-        for (int A = 0; A < ns; ++A)
-            for (int B = A; B < ns; ++B) {
-                ++npairs;
-                nprims += shells[A].alpha.size() * shells[B].alpha.size();
-            }
-        pairs.reserve(npairs);
-        prims.resize(nprims);
-    }
+    pairs.reserve((size_t)ns * (ns + 1) / 2);
+    // each pair owns the slice [pp0, pp0 + npp) of the primitive pairs
     size_t pnext = 0;
     for (int A = 0; A < ns; ++A)
         for (int B = A; B < ns; ++B) {
@@ -132,53 +139,51 @@ inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int n
             pair_ids[sa.L + sb.L].push_back((int)pairs.size());
             pairs.push_back(sp);
         }
-    auto fill = [&](size_t p0, size_t p1) {
-        for (size_t q = p0; q < p1; ++q) {
-            const ShellPair &sp = pairs[q];
-            const Shell &sa = shells[sp.sa], &sb = shells[sp.sb];
-            const double *RA = xyz + 3 * sa.center, *RB = xyz + 3 * sb.center;
-            const double ab2 = sp.AB[0] * sp.AB[0] + sp.AB[1] * sp.AB[1] + sp.AB[2] * sp.AB[2];
-            PrimPair *out = prims.data() + sp.pp0;
-            // largest screen factor first: the primitive quartets of a shell
-            // quartet that pass the screen are then a prefix of each row
-            const int na = (int)sa.alpha.size(), nb = (int)sb.alpha.size();
-            double eij[36];
-            int order[36];
-            for (int x = 0; x < na * nb; ++x) {
-                const double aa = sa.alpha[x / nb], bb = sb.alpha[x % nb];
-                const double e = exp(-aa * bb * ab2 / (aa + bb));       // int2e.f90:223
-                int y = x;
-                for (; y > 0 && eij[y - 1] < e; --y) {
-                    eij[y] = eij[y - 1];
-                    order[y] = order[y - 1];
-                }
-                eij[y] = e;
-                order[y] = x;
+    nprims = pnext;
+    return "";
+}
+
+// The pairs' primitive pairs, each pair's largest screen factor first: the
+// primitive quartets of a shell quartet that pass the screen are then a
+// prefix of each row.  (On the device: k_prim_pairs, eri.hip.)
+inline void fill_prims(const std::vector<Shell> &shells, const std::vector<ShellPair> &pairs, const double *xyz,
+                       PrimPair *prims) {
+    for (const ShellPair &sp : pairs) {
+        const Shell &sa = shells[sp.sa], &sb = shells[sp.sb];
+        const double ab2 = sp.AB[0] * sp.AB[0] + sp.AB[1] * sp.AB[1] + sp.AB[2] * sp.AB[2];
+        const int na = (int)sa.alpha.size(), nb = (int)sb.alpha.size();
+        double eij[36];
+        int order[36];
+        for (int x = 0; x < na * nb; ++x) {
+            const double aa = sa.alpha[x / nb], bb = sb.alpha[x % nb];
+            const double e = exp(-aa * bb * ab2 / (aa + bb));
+            int y = x;
+            for (; y > 0 && eij[y - 1] < e; --y) {
+                eij[y] = eij[y - 1];
+                order[y] = order[y - 1];
             }
-            for (int x = 0; x < na * nb; ++x) {
-                const int i = order[x] / nb, j = order[x] % nb;
-                const double aa = sa.alpha[i], bb = sb.alpha[j], p = aa + bb;
-                PrimPair &pp = *out++;
-                pp.p = p;
-                for (int d = 0; d < 3; ++d) {
-                    pp.P[d] = (aa * RA[d] + bb * RB[d]) / p;
-                    pp.PA[d] = pp.P[d] - RA[d];
-                }
-                pp.EIJ = eij[x];
-                pp.K = pp.EIJ * sa.coef[i] * sb.coef[j];
-                pp.beta = bb;
-                pp.ip = 1.0 / p;
-                pp.KI = pp.K * pp.ip;
-            }
+            eij[y] = e;
+            order[y] = x;
         }
-    };
-    const size_t np = pairs.size();
-    const unsigned nt = (unsigned)std::max<size_t>(1, std::min<size_t>({16, std::thread::hardware_concurrency(),
-                                                                         np / 2048 + 1}));
-    std::vector<std::thread> pool;
-    for (unsigned t = 1; t < nt; ++t) pool.emplace_back(fill, np * t / nt, np * (t + 1) / nt);
-    fill(0, np / nt);
-    for (auto &th : pool) th.join();
+        for (int x = 0; x < na * nb; ++x) {
+            const int i = order[x] / nb, j = order[x] % nb;
+            prim_pair(prims[sp.pp0 + x], sa.alpha[i], sb.alpha[j], sa.coef[i], sb.coef[j], xyz + 3 * sa.center,
+                      xyz + 3 * sb.center, eij[x]);
+        }
+    }
+}
+
+inline std::string build_system(int nnuc, const double *xyz /*[atom][3]*/, int nset, const double *set_alpha,
+                                const int *setinfo, const double *bas, int norb, const int *basinfo,
+                                std::vector<Shell> &shells, std::vector<ShellPair> &pairs,
+                                std::vector<PrimPair> &prims, std::vector<int> pair_ids[3]) {
+    size_t nprims = 0;
+    prims.clear();
+    const std::string why =
+        build_pairs(nnuc, nset, set_alpha, setinfo, bas, norb, basinfo, xyz, shells, pairs, nprims, pair_ids);
+    if (!why.empty()) return why;
+    prims.resize(nprims);
+    fill_prims(shells, pairs, xyz, prims.data());
     return "";
 }
 
