@@ -257,6 +257,9 @@ int dtmp(myqc_ctx *ctx, int slot, T **p, size_t bytes) {
     return 0;
 }
 
+// ends a call's use of a slot: what is too large to keep is freed
+void dtmp_end(myqc_ctx *ctx, int slot);
+
 // timing helpers: bracket a launch sequence on ctx->stream
 int timer_begin(myqc_ctx *ctx, int cat, hipEvent_t *ev);
 int timer_end(myqc_ctx *ctx, int cat, hipEvent_t ev, double work);

@@ -103,6 +103,10 @@ void dfree(void **p) {
     *p = nullptr;
 }
 
+void dtmp_end(myqc_ctx *ctx, int slot) {
+    if (dcapacity(ctx->d_tmp[slot]) > kKeepWork) dfree(&ctx->d_tmp[slot]);
+}
+
 int timer_begin(myqc_ctx *ctx, int cat, hipEvent_t *ev) {
     *ev = nullptr;
     if (!ctx->timing) return 0;

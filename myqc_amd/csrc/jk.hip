@@ -683,7 +683,7 @@ extern "C" int myqc_fock_G_uhf(myqc_ctx *ctx, const double *Da, const double *Db
     if (!ctx->have_eri) return set_error(ctx, MYQC_E_STATE, "myqc_fock_G_uhf: call myqc_eri_build first");
     const size_t nn = (size_t)ctx->n * ctx->n;
     double *buf = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&buf, sizeof(double) * 4 * nn));
+    MYQC_CHECK(dtmp(ctx, TMP_FOCK, &buf, sizeof(double) * 4 * nn));
     double *dA = buf, *dB = buf + nn, *gA = buf + 2 * nn, *gB = buf + 3 * nn;
     int rc = 0;
     if (hipMemcpyAsync(dA, Da, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
@@ -693,7 +693,7 @@ extern "C" int myqc_fock_G_uhf(myqc_ctx *ctx, const double *Da, const double *Db
     if (rc == 0 && (d2h(ctx, Ga, gA, sizeof(double) * nn) != hipSuccess ||
                     d2h(ctx, Gb, gB, sizeof(double) * nn) != hipSuccess))
         rc = set_error(ctx, MYQC_E_HIP, "myqc_fock_G_uhf: download failed");
-    dfree((void **)&buf);
+    dtmp_end(ctx, TMP_FOCK);
     return rc;
 }
 
@@ -706,13 +706,13 @@ extern "C" int myqc_fock_G(myqc_ctx *ctx, const double *D, double *G, int precis
     const size_t nn = (size_t)ctx->n * ctx->n;
     MYQC_HIP(ctx, hipMemcpyAsync(ctx->d_G, D, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream));
     double *d_out = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&d_out, sizeof(double) * nn));
+    MYQC_CHECK(dtmp(ctx, TMP_FOCK, &d_out, sizeof(double) * nn));
     int rc = 0;
     if (precision == MYQC_FP32 && hipMemsetAsync(d_out, 0, sizeof(double) * nn, ctx->stream) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "memset failed");
     if (rc == 0) rc = digest_G(ctx, ctx->d_G, d_out, precision);
     if (rc == 0 && d2h(ctx, G, d_out, sizeof(double) * nn) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "myqc_fock_G: copy failed");
-    dfree((void **)&d_out);
+    dtmp_end(ctx, TMP_FOCK);
     return rc;
 }

@@ -1444,16 +1444,16 @@ extern "C" int myqc_density_rhf(myqc_ctx *ctx, const double *C, int nocc, double
     const int n = ctx->n;
     if (nocc < 0 || nocc > n) return set_error(ctx, MYQC_E_ARG, "myqc_density_rhf: nocc=%d", nocc);
     const size_t nn = (size_t)n * n;
-    double *dC = nullptr, *dD = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&dC, sizeof(double) * nn));
-    int rc = dalloc(ctx, (void **)&dD, sizeof(double) * nn);
-    if (rc == 0 && hipMemcpyAsync(dC, C, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+    double *dC = nullptr;
+    MYQC_CHECK(dtmp(ctx, TMP_FOCK, &dC, sizeof(double) * 2 * nn));
+    double *dD = dC + nn;
+    int rc = 0;
+    if (hipMemcpyAsync(dC, C, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "upload failed");
     if (rc == 0) rc = density(ctx, dC, nocc, dD, n);
     if (rc == 0 && d2h(ctx, D, dD, sizeof(double) * nn) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "download failed");
-    dfree((void **)&dC);
-    dfree((void **)&dD);
+    dtmp_end(ctx, TMP_FOCK);
     return rc;
 }
 
@@ -1505,7 +1505,7 @@ extern "C" int myqc_density_uhf(myqc_ctx *ctx, const double *Ca, const double *C
         return set_error(ctx, MYQC_E_ARG, "myqc_density_uhf: nalpha=%d nbeta=%d", nalpha, nbeta);
     const size_t nn = (size_t)n * n;
     double *buf = nullptr;
-    MYQC_CHECK(dalloc(ctx, (void **)&buf, sizeof(double) * 2 * nn));
+    MYQC_CHECK(dtmp(ctx, TMP_FOCK, &buf, sizeof(double) * 2 * nn));
     const double *Cs[2] = {Ca, Cb};
     double *Ds[2] = {Da, Db};
     const int occ[2] = {nalpha, nbeta};
@@ -1517,7 +1517,7 @@ extern "C" int myqc_density_uhf(myqc_ctx *ctx, const double *Ca, const double *C
         if (rc == 0 && d2h(ctx, Ds[s], buf + nn, sizeof(double) * nn) != hipSuccess)
             rc = set_error(ctx, MYQC_E_HIP, "download failed");
     }
-    dfree((void **)&buf);
+    dtmp_end(ctx, TMP_FOCK);
     return rc;
 }
 
