@@ -307,21 +307,35 @@ __global__ __launch_bounds__(256) void k_schwarz(const ShellPair *__restrict__ p
 // for 12880 pairs that is less than a radix sort's launches take, and the host
 // sort it replaces took 0.5 ms with the GPU idle.  The keys are the factors'
 // bits (non-negative, so ordered like them; not-a-number has its place too).
-constexpr int kRankTile = 1024;
-__global__ __launch_bounds__(256) void k_rank(SchwarzArgs a, const double *__restrict__ q, int *__restrict__ rank) {
+// A workgroup takes 256 pairs and every kRankSplit-th tile: more splits spend
+// their time in the atomics (50 us with one tile each at 40 waters), fewer leave
+// the chip idle (78 us with four times larger tiles).
+constexpr int kRankTile = 256, kRankSplit = 16;
+__global__ __launch_bounds__(kRankTile) void k_rank(SchwarzArgs a, const double *__restrict__ q,
+                                                    int *__restrict__ rank) {
     __shared__ unsigned long long s_key[kRankTile];
     const int b = blockIdx.x, c = b >= a.blk[0] ? 0 : b >= a.blk[1] ? 1 : 2;
-    const int np = a.np[c], i = (b - a.blk[c]) * 256 + threadIdx.x, j0 = blockIdx.y * kRankTile;
-    if (j0 >= np) return;
-    const int nj = min(kRankTile, np - j0);
-    for (int j = threadIdx.x; j < nj; j += 256) s_key[j] = __double_as_longlong(q[a.ids[c][j0 + j]]);
-    __syncthreads();
-    if (i >= np) return;
-    const int p = a.ids[c][i];
+    const int np = a.np[c], i0 = (b - a.blk[c]) * kRankTile, i = i0 + threadIdx.x;
+    const int p = a.ids[c][min(i, np - 1)];
     const unsigned long long key = __double_as_longlong(q[p]);
     int before = 0;
-    for (int j = 0; j < nj; ++j) before += s_key[j] > key || (s_key[j] == key && j0 + j < i) ? 1 : 0;
-    if (before) atomicAdd(&rank[p], before);
+    for (int j0 = blockIdx.y * kRankTile; j0 < np; j0 += kRankSplit * kRankTile) {
+        const int nj = min(kRankTile, np - j0);
+        __syncthreads();
+        // (past the class: 0, which is before nothing by the strict comparison of a last tile)
+        s_key[threadIdx.x] = (int)threadIdx.x < nj ? __double_as_longlong(q[a.ids[c][j0 + threadIdx.x]]) : 0;
+        __syncthreads();
+        if (j0 < i0) {   // every position of the tile is before the thread's: equal keys are too
+#pragma unroll 16
+            for (int j = 0; j < kRankTile; ++j) before += s_key[j] >= key ? 1 : 0;
+        } else if (j0 > i0) {
+#pragma unroll 16
+            for (int j = 0; j < kRankTile; ++j) before += s_key[j] > key ? 1 : 0;
+        } else {
+            for (int j = 0; j < nj; ++j) before += s_key[j] > key || (s_key[j] == key && j0 + j < i) ? 1 : 0;
+        }
+    }
+    if (i < np && before) atomicAdd(&rank[p], before);
 }
 // sorted (the three classes one after another, as ids)
 __global__ __launch_bounds__(256) void k_by_rank(const int *__restrict__ ids, const int *__restrict__ rank, int np0,
@@ -427,11 +441,11 @@ int eri_schwarz(myqc_ctx *ctx) {
         sa.blk[c] = nblk;
         ra.blk[c] = nrank;
         nblk += (sa.np[c] + kSchwarzPairs - 1) / kSchwarzPairs;
-        nrank += (sa.np[c] + 255) / 256;
+        nrank += (sa.np[c] + kRankTile - 1) / kRankTile;
     }
     MYQC_HIP(ctx, hipMemcpyAsync(ids, all.data(), sizeof(int) * np, hipMemcpyHostToDevice, ctx->stream));
     k_schwarz<<<nblk, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, sa, ctx->d_schwarz, rank);
-    k_rank<<<dim3(nrank, (most + kRankTile - 1) / kRankTile), 256, 0, ctx->stream>>>(ra, ctx->d_schwarz, rank);
+    k_rank<<<dim3(nrank, std::min(kRankSplit, (most + kRankTile - 1) / kRankTile)), kRankTile, 0, ctx->stream>>>(ra, ctx->d_schwarz, rank);
     k_by_rank<<<(np + 255) / 256, 256, 0, ctx->stream>>>(ids, rank, sa.np[0], sa.np[1], np, sorted);
     for (int c = 0; c < 3; ++c) {
         if (sa.np[c] == 0) continue;

@@ -388,8 +388,9 @@ __global__ __launch_bounds__(256, sizeof(TV) == 4 ? 4 : 3) void k_digest(DigArgs
 // The ket-side J of every pair: jk[base(c) + r ncd(c) + e] = sum of the
 // partial slots of the chunks that cover rank r of class c.  One workgroup
 // per group of at most kJkGroup slots of one block of W(c) ranks (positions
-// of the block across the threads, coalesced; four independent sums), added
-// into jk (zeroed before the pass) with one atomic per position.
+// of the block across the threads, coalesced; sixteen loads in flight), added
+// into jk (zeroed before the pass) with one atomic per position.  Bounded by
+// the latency of its loads: with four at a time 40 waters took 18 us, now 14.
 template <typename PT>
 __global__ __launch_bounds__(256) void k_gather_jk(const PT *__restrict__ jk_part, const int *__restrict__ list,
                                                    const int *__restrict__ group, int3 base, int3 block0, int4 nps,
@@ -403,20 +404,24 @@ __global__ __launch_bounds__(256) void k_gather_jk(const PT *__restrict__ jk_par
     const int b0 = c == 0 ? base.x : c == 1 ? base.y : base.z;
     for (int pos = threadIdx.x; pos < npos; pos += blockDim.x) {
         if (r0 + pos / ncd >= np) break;
-        double s4[4] = {0.0, 0.0, 0.0, 0.0};
-        int k = k0;
-        for (; k + 4 <= k1; k += 4)
+        double s8[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        for (int k = k0; k < k1; k += 16) {
+            PT v[16];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) s4[q] += jk_part[(size_t)list[k + q] * kJkSlot + pos];
-        for (; k < k1; ++k) s4[0] += jk_part[(size_t)list[k] * kJkSlot + pos];
-        atomicAdd(&jk[b0 + (size_t)r0 * ncd + pos], (s4[0] + s4[1]) + (s4[2] + s4[3]));
+            for (int q = 0; q < 16; ++q) v[q] = jk_part[(size_t)list[min(k + q, k1 - 1)] * kJkSlot + pos];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) s8[q % 8] += k + q < k1 ? (double)v[q] : 0.0;
+        }
+        atomicAdd(&jk[b0 + (size_t)r0 * ncd + pos],
+                  ((s8[0] + s8[1]) + (s8[2] + s8[3])) + ((s8[4] + s8[5]) + (s8[6] + s8[7])));
     }
 }
 
 // A(i, j) = the sum of the partial rows holding AO i, plus the ket-side J of
 // the pair (shell(i), shell(j)) when it is stored in that orientation.  One
 // workgroup per (AO, 64 columns); its four thread rows take every fourth
-// partial row (two independent sums each) and meet in LDS in a fixed order.
+// partial row (twelve loads in flight each, as many as 40 waters' AOs have) and
+// meet in LDS in a fixed order.  Two at a time took 18 us at 40 waters, now 13.4.
 template <typename PT>
 __global__ __launch_bounds__(256) void k_gather_rows(const PT *__restrict__ partial,
                                                      const int *__restrict__ list_off, const int *__restrict__ list,
@@ -428,14 +433,15 @@ __global__ __launch_bounds__(256) void k_gather_rows(const PT *__restrict__ part
     double s = 0.0;
     if (j < n) {
         const int k0 = list_off[i], k1 = list_off[i + 1];
-        double s2[2] = {0.0, 0.0};
-        int k = k0 + q;
-        for (; k + 4 < k1; k += 8) {
-            s2[0] += partial[(size_t)list[k] * n + j];
-            s2[1] += partial[(size_t)list[k + 4] * n + j];
+        double s4[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int k = k0 + q; k < k1; k += 4 * 12) {
+            PT v[12];
+#pragma unroll
+            for (int u = 0; u < 12; ++u) v[u] = partial[(size_t)list[min(k + 4 * u, k1 - 1)] * n + j];
+#pragma unroll
+            for (int u = 0; u < 12; ++u) s4[u % 4] += k + 4 * u < k1 ? (double)v[u] : 0.0;
         }
-        if (k < k1) s2[0] += partial[(size_t)list[k] * n + j];
-        s = s2[0] + s2[1];
+        s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     }
     s_sum[q][threadIdx.x] = s;
     __syncthreads();
@@ -457,82 +463,102 @@ __global__ void k_zero(double *__restrict__ p, size_t cnt) {
 // dk_c at dk + {0, np0, np0 + 3 np1}; and the zeroing of jk (njk values), in
 // one launch
 template <typename TV>
-__global__ void k_pack_kets_all(const ShellPair *__restrict__ pairs, const int *__restrict__ s0,
-                                const int *__restrict__ s1, const int *__restrict__ s2, int np0, int np1, int np2,
+__global__ void k_pack_kets_all(const int *__restrict__ m0, const int *__restrict__ m1, const int *__restrict__ m2,
+                                int np0, int np1, int np2,
                                 const TV *__restrict__ D, int n, TV *__restrict__ dk, double *__restrict__ jk,
                                 size_t njk) {
     const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (id < njk) jk[id] = 0.0;
     if (id >= (size_t)np0 + np1 + np2) return;
     int r = (int)id, nc = 1, nd = 1;
-    const int *sorted = s0;
+    const int *meta = m0;
     TV *out = dk;
     if (r >= np0 + np1) {
         r -= np0 + np1;
-        sorted = s2;
+        meta = m2;
         nc = nd = 3;
         out = dk + np0 + 3 * (size_t)np1;
     } else if (r >= np0) {
         r -= np0;
-        sorted = s1;
+        meta = m1;
         nc = 3;
         out = dk + np0;
     }
-    const ShellPair sp = pairs[sorted[r]];
+    const int ao_a = meta[r] & 0x7fff, ao_b = meta[r] >> 15;
     for (int c = 0; c < nc; ++c)
-        for (int d = 0; d < nd; ++d) out[(size_t)r * nc * nd + c * nd + d] = D[(sp.ao_a + c) + (size_t)n * (sp.ao_b + d)];
+        for (int d = 0; d < nd; ++d) out[(size_t)r * nc * nd + c * nd + d] = D[(ao_a + c) + (size_t)n * (ao_b + d)];
 }
 
 // --- small elementwise kernels ------------------------------------------------
 
 
+// The kernels below work on 16 x 16 tiles, a thread per element; the mirrored tile
+// goes through LDS, since read in place (one column per element) it was most
+// of their time with several systems at once (280 functions, 32 systems: 15 us
+// a launch, 4.3 alone; 12 and 4.2 so).
+constexpr int kTile = 16;
+static dim3 tiles(int n) { return dim3((n + kTile - 1) / kTile, (n + kTile - 1) / kTile); }
+
+// f(q, own, mirrored) for the elements q of the workgroup's tile, value(q)
+// being element q of the matrix
+template <typename V, typename F>
+__device__ __forceinline__ void with_mirror(int n, double (&s)[kTile][kTile + 1], V value, F f) {
+    const int x = threadIdx.x % kTile, y = threadIdx.x / kTile;
+    const int i0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile;
+    const bool in = i0 + x < n && j0 + y < n;
+    const size_t q = i0 + x + (size_t)n * (j0 + y);
+    // element (j0 + x, i0 + y) of the mirrored tile, (i0 + x, j0 + y) of the own
+    s[y][x] = (j0 + x < n && i0 + y < n) ? value(j0 + x + (size_t)n * (i0 + y)) : 0.0;
+    const double own = in ? value(q) : 0.0;
+    __syncthreads();
+    if (in) f(q, own, s[x][y]);
+}
+
 // Ds = scale (E + E^T), E = D - Dm (Dm may be NULL: E = D); with amax, also
 // max |Ds32| into *amax as the bit pattern of a non-negative float (ordered
 // like the value; *amax starts at 0)
-__global__ __launch_bounds__(128) void k_symmetrize(const double *__restrict__ D, double *__restrict__ Ds, float *__restrict__ Ds32, int n,
-                             double scale, unsigned *__restrict__ amax = nullptr,
-                             const double *__restrict__ Dm = nullptr) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+__global__ __launch_bounds__(256) void k_symmetrize(const double *__restrict__ D, double *__restrict__ Ds,
+                                                    float *__restrict__ Ds32, int n, double scale,
+                                                    unsigned *__restrict__ amax = nullptr,
+                                                    const double *__restrict__ Dm = nullptr) {
+    __shared__ double s_t[kTile][kTile + 1];
     float m = 0.0f;
-    if (i < n) {
-        const size_t ij = i + (size_t)n * j, ji = j + (size_t)n * i;
-        const double v = Dm ? scale * ((D[ij] - Dm[ij]) + (D[ji] - Dm[ji])) : scale * (D[ij] + D[ji]);
-        if (Ds) Ds[ij] = v;
-        if (Ds32) {
-            Ds32[ij] = (float)v;
-            m = fabsf((float)v);
-        }
-    }
+    with_mirror(
+        n, s_t, [&](size_t q) { return Dm ? D[q] - Dm[q] : D[q]; },
+        [&](size_t q, double own, double mirrored) {
+            const double v = scale * (own + mirrored);
+            if (Ds) Ds[q] = v;
+            if (Ds32) {
+                Ds32[q] = (float)v;
+                m = fmaxf(m, fabsf((float)v));
+            }
+        });
     if (amax) {
         // one atomic per workgroup at most, and none once the stored maximum
         // is already as large (the stored value only grows, so a stale read
         // can only cost an unneeded atomic)
-        __shared__ float s_m[2];
+        __shared__ float s_m[4];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
         if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
         __syncthreads();
         if (threadIdx.x == 0) {
-            const unsigned b = __float_as_uint(fmaxf(s_m[0], s_m[1]));
+            const unsigned b = __float_as_uint(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])));
             if (b > __atomic_load_n(amax, __ATOMIC_RELAXED)) atomicMax(amax, b);
         }
     }
 }
 
-
-
-
-
 // G += A + A^T (the incremental passes); the pass's max |dD| word is
 // cleared for the next pass (the digestion has read it)
-__global__ __launch_bounds__(128) void k_sym_add(const double *__restrict__ A, double *__restrict__ G, int n,
+__global__ __launch_bounds__(256) void k_sym_add(const double *__restrict__ A, double *__restrict__ G, int n,
                                                  unsigned *__restrict__ amax) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    if (i < n) G[i + (size_t)n * j] += A[i + (size_t)n * j] + A[j + (size_t)n * i];
-    if (i == 0 && j == 0) *amax = 0u;
+    __shared__ double s_t[kTile][kTile + 1];
+    with_mirror(
+        n, s_t, [&](size_t q) { return A[q]; },
+        [&](size_t q, double own, double mirrored) { G[q] += own + mirrored; });
+    if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0) *amax = 0u;
 }
-
-static dim3 grid2(int n) { return dim3((n + 127) / 128, n); }
 
 int ensure_work(myqc_ctx *ctx) {
     if (ctx->work_n == ctx->n) return 0;
@@ -562,7 +588,7 @@ static int launch_digest(myqc_ctx *ctx, const TV *D, const TV *x, TV *dk, double
     const size_t njk = (size_t)std::max(pl.jk_base[3], 1);
     const size_t npack = std::max(njk, (size_t)np0 + np1 + np2);
     k_pack_kets_all<TV><<<(unsigned)((npack + 255) / 256), 256, 0, ctx->stream>>>(
-        ctx->d_pairs, ctx->d_sorted[0], ctx->d_sorted[1], ctx->d_sorted[2], np0, np1, np2, D, n, dk, ctx->d_jk, njk);
+        ctx->d_meta[0], ctx->d_meta[1], ctx->d_meta[2], np0, np1, np2, D, n, dk, ctx->d_jk, njk);
     if (ctx->n_wg > 0) {
         DigArgs<TV> a;
         a.meta0 = ctx->d_meta[0];
@@ -628,19 +654,19 @@ int digest_G(myqc_ctx *ctx, const double *d_Din, double *d_Gout, int precision, 
     const int n = ctx->n;
     const size_t nn = (size_t)n * n;
     if (precision == MYQC_FP64) {
-        k_symmetrize<<<grid2(n), 128, 0, ctx->stream>>>(d_Din, ctx->d_D, nullptr, n, 0.5);
+        k_symmetrize<<<tiles(n), 256, 0, ctx->stream>>>(d_Din, ctx->d_D, nullptr, n, 0.5);
         MYQC_CHECK(launch_digest<double>(ctx, ctx->d_D, ctx->d_x64, ctx->d_Dpair, ctx->d_partial, ctx->d_A));
-        k_symmetrize<<<grid2(n), 128, 0, ctx->stream>>>(ctx->d_A, d_Gout, nullptr, n, 1.0);
+        k_symmetrize<<<tiles(n), 256, 0, ctx->stream>>>(ctx->d_A, d_Gout, nullptr, n, 1.0);
     } else {
         if (!ctx->have_eri32) return set_error(ctx, MYQC_E_STATE, "no FP32 integrals stored");
         // the density change (Din - Dprev when Dprev is given) symmetrised
         // into FP32, with the pass's max |dD| for the screen folded in; the
         // word is 0 here (k_sym_add clears it at the end of each pass)
         unsigned *amax = reinterpret_cast<unsigned *>(ctx->d_dmax);
-        k_symmetrize<<<grid2(n), 128, 0, ctx->stream>>>(d_Din, nullptr, ctx->d_D32, n, 0.5, amax, d_Dprev);
+        k_symmetrize<<<tiles(n), 256, 0, ctx->stream>>>(d_Din, nullptr, ctx->d_D32, n, 0.5, amax, d_Dprev);
         MYQC_CHECK(launch_digest<float>(ctx, ctx->d_D32, ctx->d_x32, ctx->d_Dpair32, ctx->d_partial, ctx->d_A, 1.0,
                                         kIncrementalScreen));
-        k_sym_add<<<grid2(n), 128, 0, ctx->stream>>>(ctx->d_A, d_Gout, n, amax);
+        k_sym_add<<<tiles(n), 256, 0, ctx->stream>>>(ctx->d_A, d_Gout, n, amax);
         (void)nn;
     }
     MYQC_HIP(ctx, hipGetLastError());
@@ -664,9 +690,9 @@ int digest_G_uhf(myqc_ctx *ctx, const double *d_Da, const double *d_Db, double *
     // total density into Ga, spin difference into Gb (both overwritten below)
     k_axpby<<<256, 256, 0, ctx->stream>>>(d_Da, d_Db, d_Ga, 1.0, 1.0, nn);
     k_axpby<<<256, 256, 0, ctx->stream>>>(d_Da, d_Db, d_Gb, 1.0, -1.0, nn);
-    k_symmetrize<<<grid2(n), 128, 0, ctx->stream>>>(d_Gb, ctx->d_D, nullptr, n, 0.5);
+    k_symmetrize<<<tiles(n), 256, 0, ctx->stream>>>(d_Gb, ctx->d_D, nullptr, n, 0.5);
     MYQC_CHECK(launch_digest<double>(ctx, ctx->d_D, ctx->d_x64, ctx->d_Dpair, ctx->d_partial, ctx->d_A, 0.0));
-    k_symmetrize<<<grid2(n), 128, 0, ctx->stream>>>(ctx->d_A, ctx->d_G, nullptr, n, 1.0);   // Gk(Da - Db)
+    k_symmetrize<<<tiles(n), 256, 0, ctx->stream>>>(ctx->d_A, ctx->d_G, nullptr, n, 1.0);   // Gk(Da - Db)
     MYQC_CHECK(digest_G(ctx, d_Ga, d_Gb, MYQC_FP64));                                           // G(Da + Db)
     k_axpby<<<256, 256, 0, ctx->stream>>>(d_Gb, ctx->d_G, d_Ga, 1.0, 1.0, nn);
     k_axpby<<<256, 256, 0, ctx->stream>>>(d_Gb, ctx->d_G, d_Gb, 1.0, -1.0, nn);
