@@ -3,51 +3,48 @@
 // src/integrals/int1e.f90:132-280; the per-pair math is in one_e_math.h),
 // the dipole integrals of int1p (src/integrals/int1p.f90:140-355) and the
 // SCF dipole moment of cphf_dipole_rhf (src/props/cphf.f90:106-121).
+#include <algorithm>
 #include <cmath>
 
 #include "boys_dev.h"
 #include "context.h"
 #include "one_e_math.h"
+#include "wave.h"
 
 namespace myqc {
 
+constexpr int kOneEBlocks = 1024;   // four workgroups per CU (the staged tables' LDS)
 __global__ __launch_bounds__(256) void k_one_e(const ShellPair *__restrict__ pairs, const PrimPair *__restrict__ prims,
                                                const double *__restrict__ ftT, const double *__restrict__ atoms,
                                                int nnuc, int npairs, int n, double *__restrict__ S, double *__restrict__ H) {
     __shared__ __attribute__((aligned(16))) double s_ft[ft_staged(2)];
     const BoysTab ft = stage_boys<2>(ftT, s_ft);
-    // one wavefront per shell pair: lane l takes the nuclei l, l + 64, ... of
-    // the attraction integrals and the primitive pairs l, l + 64, ... of S and
-    // T, then the lanes' sums are added across the wavefront
-    const int lane = threadIdx.x & 63;
-    const int t = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-    if (t >= npairs) return;   // whole wavefronts
-    const ShellPair sp = pairs[t];
-    double s[3][3], h[3][3];
-    one_e_pair(sp, prims, ft, atoms, nnuc, s, h, lane, 64);
+    // one wavefront per shell pair at a time: lane l takes the nuclei l, l + 64,
+    // ... of the attraction integrals and the primitive pairs l, l + 64, ... of S
+    // and T, then the lanes' sums are added across the wavefront.  A workgroup
+    // goes on to further pairs: staging the tables (40 KB) for four pairs alone
+    // was half of the time.
+    const int lane = threadIdx.x & 63, step = gridDim.x * (blockDim.x / 64);
+    for (int t = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); t < npairs; t += step) {   // whole wavefronts
+        const ShellPair sp = pairs[t];
+        double s[3][3], h[3][3];
+        one_e_pair(sp, prims, ft, atoms, nnuc, s, h, lane, 64);
+        const int na = sp.la ? 3 : 1, nb = sp.lb ? 3 : 1;
+        // constant indices into s and h (registers), the sizes as guards
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+        for (int a = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                h[a][b] += __shfl_xor(h[a][b], off, 64);
-                s[a][b] += __shfl_xor(s[a][b], off, 64);
+            for (int b = 0; b < 3; ++b) {
+                if (a >= na || b >= nb) continue;
+                const double hs = wave_total(h[a][b]), ss = wave_total(s[a][b]);
+                if (lane != 0) continue;
+                const size_t i = sp.ao_a + a, j = sp.ao_b + b;
+                S[i + n * j] = ss;
+                S[j + n * i] = ss;
+                H[i + n * j] = hs;
+                H[j + n * i] = hs;
             }
-    if (lane != 0) return;
-    const int na = sp.la ? 3 : 1, nb = sp.lb ? 3 : 1;
-    // constant indices into s and h (registers), the sizes as guards
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            if (a >= na || b >= nb) continue;
-            const size_t i = sp.ao_a + a, j = sp.ao_b + b;
-            S[i + n * j] = s[a][b];
-            S[j + n * i] = s[a][b];
-            H[i + n * j] = h[a][b];
-            H[j + n * i] = h[a][b];
-        }
+    }
 }
 
 // P_c (c = x, y, z) at P + c n^2, both triangles
@@ -157,7 +154,7 @@ extern "C" int myqc_int1e(myqc_ctx *ctx, double *S, double *H) {
                                   ctx->stream) != hipSuccess)
         rc = set_error(ctx, MYQC_E_HIP, "upload failed");
     if (rc == 0) {
-        k_one_e<<<(np + 3) / 4, 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, dA, ctx->nnuc, np, n,
+        k_one_e<<<std::min((np + 3) / 4, kOneEBlocks), 256, 0, ctx->stream>>>(ctx->d_pairs, ctx->d_prims, ctx->d_ftT, dA, ctx->nnuc, np, n,
                                                       dS, dH);
         if (hipGetLastError() != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "one-electron kernel launch failed");
     }

@@ -80,36 +80,38 @@ MYQC_HD void one_e_pair_t(const ShellPair &sp, const PrimPair *__restrict__ prim
     for (int a = 0; a < 3; ++a)
         for (int b = 0; b < 3; ++b) s[a][b] = kin[a][b] = v[a][b] = 0.0;
     const int Q = 3 * sp.bl;
-    for (int ip = 0; ip < sp.npp; ++ip) {
+    // the primitive pairs stand with the largest screen factor first
+    for (int ip = c0; ip < sp.npp; ip += cstep) {
         const PrimPair pr = prims[sp.pp0 + ip];
-        if (pr.EIJ < 1.0e-14) continue;                  // int1e.f90:238-241
-        const double p = pr.p;
+        if (pr.EIJ < 1.0e-14) break;                     // int1e.f90:238-241
+        const double p = pr.p, beta = pr.beta;
         double PB[3];
         for (int d = 0; d < 3; ++d) PB[d] = pr.PA[d] + sp.AB[d];   // P - B = (P - A) + (A - B)
-        const double beta = pr.beta;
-        const bool st = ip % cstep == c0;
-        const double pref = st ? pow(PI_SP / p, 1.5) * pr.K : 0.0;
-        if (st) {
+        const double pref = pow(PI_SP / p, 1.5) * pr.K;
 #pragma unroll
-            for (int a = 0; a < na; ++a)
+        for (int a = 0; a < na; ++a)
 #pragma unroll
-                for (int b = 0; b < nb; ++b) {
-                    int la[3] = {0, 0, 0}, lb[3] = {0, 0, 0};
-                    if (LA) la[a] = 1;
-                    if (LB) lb[b] = 1;
-                    double Ex[3], kx[3];
+            for (int b = 0; b < nb; ++b) {
+                int la[3] = {0, 0, 0}, lb[3] = {0, 0, 0};
+                if (LA) la[a] = 1;
+                if (LB) lb[b] = 1;
+                double Ex[3], kx[3];
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        const int i = la[d], j = lb[d];
-                        Ex[d] = e1d(i, j, pr.PA[d], PB[d], p);
-                        // int1e.f90:442-462
-                        kx[d] = j * (j - 1) * e1d(i, j - 2, pr.PA[d], PB[d], p) - 2.0 * beta * j * Ex[d] -
-                                2.0 * beta * (j + 1) * Ex[d] + 4.0 * beta * beta * e1d(i, j + 2, pr.PA[d], PB[d], p);
-                    }
-                    s[a][b] += pref * Ex[0] * Ex[1] * Ex[2];
-                    kin[a][b] += -0.5 * pref * (kx[0] * Ex[1] * Ex[2] + Ex[0] * kx[1] * Ex[2] + Ex[0] * Ex[1] * kx[2]);
+                for (int d = 0; d < 3; ++d) {
+                    const int i = la[d], j = lb[d];
+                    Ex[d] = e1d(i, j, pr.PA[d], PB[d], p);
+                    // int1e.f90:442-462
+                    kx[d] = j * (j - 1) * e1d(i, j - 2, pr.PA[d], PB[d], p) - 2.0 * beta * j * Ex[d] -
+                            2.0 * beta * (j + 1) * Ex[d] + 4.0 * beta * beta * e1d(i, j + 2, pr.PA[d], PB[d], p);
                 }
-        }
+                s[a][b] += pref * Ex[0] * Ex[1] * Ex[2];
+                kin[a][b] += -0.5 * pref * (kx[0] * Ex[1] * Ex[2] + Ex[0] * kx[1] * Ex[2] + Ex[0] * Ex[1] * kx[2]);
+            }
+    }
+    for (int ip = 0; ip < sp.npp; ++ip) {
+        const PrimPair pr = prims[sp.pp0 + ip];
+        if (pr.EIJ < 1.0e-14) break;
+        const double p = pr.p;
         // nuclear attraction: [a|V|s]^(m) for a up to level la+lb, then HRR
         for (int c = c0; c < nnuc; c += cstep) {
             const double Zc = atoms[4 * c];
