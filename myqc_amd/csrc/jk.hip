@@ -673,6 +673,14 @@ int digest_G(myqc_ctx *ctx, const double *d_Din, double *d_Gout, int precision, 
     return 0;
 }
 
+// The A of G(D) = A + A^T for a D that is symmetric (to rounding), for a caller
+// that adds the transpose itself: two launches fewer than digest_G
+int digest_A(myqc_ctx *ctx, const double *d_D, double *d_A) {
+    if (!ctx->have_eri) return set_error(ctx, MYQC_E_STATE, "no stored integrals (call myqc_eri_build)");
+    MYQC_CHECK(ensure_work(ctx));
+    return launch_digest<double>(ctx, d_D, ctx->d_x64, ctx->d_Dpair, ctx->d_partial, d_A);
+}
+
 // Z = a X + b Y
 __global__ void k_axpby(const double *__restrict__ X, const double *__restrict__ Y, double *__restrict__ Z, double a,
                         double b, size_t cnt) {

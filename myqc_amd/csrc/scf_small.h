@@ -17,6 +17,7 @@ struct SmallStep {
     int core;               // 1: the density of H alone (no error, no DIIS)
     int head, hn;           // DIIS slot of this iteration, history length with it
     int with_dd;            // 1: max |D - Dprev| is wanted
+    int g_half;             // 1: G holds A of G(D) = A + A^T (digest_A)
     double shift, shift_err;   // level shift while the DIIS error is above shift_err (shift 0: none)
     const double *H, *G, *X, *D, *Dprev, *Do;
     double *hF, *hE;        // histories, n^2 per slot

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_step(SmallStep a) {
             const double h = a.H[q];
             f = h;
             if (!a.core) {
-                f += a.G[q];
+                f += a.g_half ? a.G[q] + a.G[j + n * i] : a.G[q];
                 const double d = a.D[q];
                 e0 += d * f;
                 e1 += d * h;
