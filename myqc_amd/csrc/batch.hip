@@ -110,7 +110,7 @@ struct BEriArgs {
     const double *ksoa;      // primitive pairs of the ket class list (ket_soa.h)
     long long nket;          // entries of the ket class list
     const long long *qcum;   // nmol + 1 prefix counts of this class combination
-    int nmol;
+    const int *qfirst;       // the molecule of quartets 0, 64, 128, ...
     long long nq;
     double *eri;
 };
@@ -122,12 +122,11 @@ __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
     const BoysTab ft = stage_boys<M>(a.ftT, s_ft);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.nq) return;
-    int lo = 0, hi = a.nmol;   // last m with qcum[m] <= t
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (a.qcum[mid] <= t) lo = mid;
-        else hi = mid;
-    }
+    // last m with qcum[m] <= t: from the wavefront's first quartet on (a search
+    // over the molecules is ten dependent loads; the six classes of
+    // 1024 clusters 6.0 -> 5.7 ms)
+    int lo = a.qfirst[t >> 6];
+    while (a.qcum[lo + 1] <= t) ++lo;
     const BMol mol = a.mols[lo];
     const long long q = t - a.qcum[lo];
     long long p, r;
@@ -869,6 +868,7 @@ struct BatchState {
     PrimPair *d_prims = nullptr;
     double *d_atoms = nullptr, *d_ftT = nullptr;
     long long *d_qcum[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    int *d_qfirst[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     double *d_eri = nullptr, *d_S = nullptr, *d_H = nullptr, *d_D = nullptr, *d_guess = nullptr, *d_scratch = nullptr,
            *d_hist = nullptr, *d_energy = nullptr;
     int *d_iters = nullptr, *d_conv = nullptr, *d_counter = nullptr;
@@ -901,6 +901,7 @@ struct BatchState {
         if (graph_learned) (void)hipGraphExecDestroy(graph_learned);
         graph_learned = nullptr;
         for (auto &q : d_qcum) dfree((void **)&q);
+        for (auto &q : d_qfirst) dfree((void **)&q);
         for (auto &q : d_ksoa) dfree((void **)&q);
         if (graph) (void)hipGraphExecDestroy(graph);
         graph = nullptr;
@@ -931,7 +932,7 @@ static void launch_batch_eri(myqc_ctx *ctx, BatchState &b, int c, int threads) {
     a.ksoa = b.d_ksoa[kCK[c]];
     a.nket = b.ncls[kCK[c]];
     a.qcum = b.d_qcum[c];
-    a.nmol = b.nmol;
+    a.qfirst = b.d_qfirst[c];
     a.nq = b.nq[c];
     a.eri = b.d_eri;
     const unsigned grid = (unsigned)((b.nq[c] + threads - 1) / threads);
@@ -1214,7 +1215,15 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
             qc[m + 1] = qc[m] + (kCB[c] == kCK[c] ? tri(nb) : nb * nk);
         }
         b.nq[c] = qc[nmol];
+        std::vector<int> first((size_t)((qc[nmol] + 63) / 64));
+        int m = 0;
+        for (size_t k = 0; k < first.size(); ++k) {
+            while (qc[m + 1] <= (long long)(64 * k)) ++m;
+            first[k] = m;
+        }
         MYQC_CHECK(upload(ctx, &b.d_qcum[c], qc));
+        MYQC_CHECK(upload(ctx, &b.d_qfirst[c], first));
+        MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));   // (the vectors end here)
     }
     std::vector<double> ftT(FT_TOTAL);
     boys_inputs(Ftab, ftT.data() + FT_EG);
