@@ -286,7 +286,7 @@ struct HostClock {
 // internals shared between translation units
 int eri_schwarz(myqc_ctx *ctx);
 int eri_store(myqc_ctx *ctx, double tol, bool want32);
-int eri_values(myqc_ctx *ctx, double tol, bool want32);
+int eri_values(myqc_ctx *ctx, double tol, bool want32, bool given_shapes);
 // G(D) into d_G (precision FP64), or d_G += G32(D - Dprev) (precision FP32;
 // Dprev may be NULL for D itself)
 int digest_G(myqc_ctx *ctx, const double *d_D, double *d_G, int precision, const double *d_Dprev = nullptr);

@@ -189,7 +189,7 @@ int DenseSource::open(double tol) {
         swapped = true;
     }
     opened = true;
-    return eri_values(ctx, tol, false);
+    return eri_values(ctx, tol, false, false);
 }
 
 void DenseSource::close() {

@@ -520,9 +520,9 @@ static int rule_split(int c, long long nq) {
     return s;
 }
 
-static EriShape class_shape(int c, long long nq) {
+static EriShape class_shape(int c, long long nq, bool given) {
     EriShape sh;
-    {
+    if (given) {
         std::lock_guard<std::mutex> g(g_shape_mu);
         sh = g_shape[c];
     }
@@ -725,8 +725,10 @@ static int ensure_side_streams(myqc_ctx *ctx) {
 
 // The values of every screened quartet at threshold tol, and their layout:
 // all of the stored build but the digestion schedule.  Leaves the kernels
-// in flight on the context stream.
-int eri_values(myqc_ctx *ctx, double tol, bool want32) {
+// in flight on the context stream.  given_shapes: the shapes tuned or set for
+// stored builds; without, the rule's alone, so that dense results do not
+// depend on what the process has tuned.
+int eri_values(myqc_ctx *ctx, double tol, bool want32, bool given_shapes) {
     HostClock hc(ctx);
     MYQC_CHECK(eri_schwarz(ctx));
     hc.mark("eri_store: Schwarz factors");
@@ -751,7 +753,7 @@ int eri_values(myqc_ctx *ctx, double tol, bool want32) {
     for (int c : kOrder) {
         if (ctx->cls[c].nq == 0) continue;
         launch_class(ctx, c, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream,
-                     class_shape(c, ctx->cls[c].nq));
+                     class_shape(c, ctx->cls[c].nq, given_shapes));
         MYQC_HIP(ctx, hipGetLastError());
     }
     for (int k = 0; k < 2; ++k) {
@@ -766,7 +768,7 @@ int eri_values(myqc_ctx *ctx, double tol, bool want32) {
 int eri_store(myqc_ctx *ctx, double tol, bool want32) {
     HostClock hc(ctx);
     free_eri(ctx, true);
-    MYQC_CHECK(eri_values(ctx, tol, want32));
+    MYQC_CHECK(eri_values(ctx, tol, want32, true));
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair, sizeof(double) * 9 * ctx->pairs.size()));
     MYQC_CHECK(dalloc(ctx, (void **)&ctx->d_Dpair32, sizeof(float) * 9 * ctx->pairs.size()));
     hc.mark("eri_store: values");
@@ -798,7 +800,7 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
     EriShape best[6];
     double best_ms[6];
     for (int c = 0; c < 6 && rc == 0; ++c) {
-        best[c] = class_shape(c, ctx->cls[c].nq);
+        best[c] = class_shape(c, ctx->cls[c].nq, true);
         best_ms[c] = 0.0;
         if (ctx->cls[c].nq == 0) continue;
         best_ms[c] = 1e300;
