@@ -1089,7 +1089,7 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
     BatchState &b = *ctx->batch;
     std::vector<ShellPair> pairs;
     std::vector<PrimPair> prims;
-    std::vector<int> cls[3], pair_mol;
+    std::vector<int> cls[3], pair_mol, weight;
     std::vector<double> atoms;
     b.mols.resize(nmol);
     int atom0 = 0;
@@ -1118,11 +1118,12 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
         // 0.28 survive; 1024 clusters 2.98 -> 2.21 ms): by the primitive pairs
         // that pass alone halfway to it, then at it
         {
-            std::vector<int> weight(mp.size());
+            weight.assign(mp.size(), 0);
             for (size_t q = 0; q < mp.size(); ++q)
                 for (int i = 0; i < mp[q].npp; ++i) {
                     const double e = mpr[mp[q].pp0 + i].EIJ;
-                    weight[q] += e >= 1e-7 ? 101 : e >= 1e-14 ? 1 : 0;
+                    if (e < 1e-14) break;   // (largest first)
+                    weight[q] += e >= 1e-7 ? 101 : 1;
                 }
             for (auto &v : ids)
                 std::stable_sort(v.begin(), v.end(), [&](int x, int y) { return weight[x] > weight[y]; });
@@ -1208,22 +1209,21 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
     b.order.resize(nmol);
     std::iota(b.order.begin(), b.order.end(), 0);
     std::stable_sort(b.order.begin(), b.order.end(), [&](int x, int y) { return b.mols[x].n > b.mols[y].n; });
+    std::vector<long long> qcum[6];
+    std::vector<int> qfirst[6];
     for (int c = 0; c < 6; ++c) {
-        std::vector<long long> qc(nmol + 1, 0);
+        std::vector<long long> &qc = qcum[c];
+        qc.assign(nmol + 1, 0);
         for (int m = 0; m < nmol; ++m) {
             const long long nb = b.mols[m].ncls[kCB[c]], nk = b.mols[m].ncls[kCK[c]];
             qc[m + 1] = qc[m] + (kCB[c] == kCK[c] ? tri(nb) : nb * nk);
         }
         b.nq[c] = qc[nmol];
-        std::vector<int> first((size_t)((qc[nmol] + 63) / 64));
-        int m = 0;
-        for (size_t k = 0; k < first.size(); ++k) {
-            while (qc[m + 1] <= (long long)(64 * k)) ++m;
-            first[k] = m;
-        }
+        qfirst[c].resize((size_t)((qc[nmol] + 63) / 64));
+        for (int m = 0; m < nmol; ++m)   // the quartets 64 k of molecule m
+            for (long long k = (qc[m] + 63) / 64; 64 * k < qc[m + 1]; ++k) qfirst[c][k] = m;
         MYQC_CHECK(upload(ctx, &b.d_qcum[c], qc));
-        MYQC_CHECK(upload(ctx, &b.d_qfirst[c], first));
-        MYQC_HIP(ctx, hipStreamSynchronize(ctx->stream));   // (the vectors end here)
+        MYQC_CHECK(upload(ctx, &b.d_qfirst[c], qfirst[c]));
     }
     std::vector<double> ftT(FT_TOTAL);
     boys_inputs(Ftab, ftT.data() + FT_EG);
