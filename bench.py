@@ -402,7 +402,7 @@ def main():
     from myqc_amd import guess as G
     have_net = G.load(ctx)
     # the ERI launch shapes, searched once on the headline cluster (untimed;
-    # kept for the process, so every later build uses them)
+    # kept for the process's builds of about that size)
     ctx.set_system(Z, xyz, basis, ftab)
     ctx.eri_build(1e-12)
     eri_shapes, eri_shape_ms = ctx.eri_tune(reps=2)

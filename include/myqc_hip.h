@@ -72,14 +72,17 @@ int myqc_eri_build(myqc_ctx *ctx, double schwarz_tol, long long *n_stored);
  * quartet classes (ss|ss, ps|ss, ps|ps, pp|ss, pp|ps, pp|pp) present in the
  * system of the last myqc_eri_build, every candidate of lanes per shell
  * quartet (1, 2, 4, 8) x threads per workgroup (64, 128, 256) is timed (best
- * of `reps`), and the fastest is kept for all later builds in the process.
+ * of `reps`), and the fastest is kept for the process's later builds in which
+ * the class has half to twice as many quartets (by default, and for other
+ * sizes, the lanes follow the number of quartets).
  * shapes (may be NULL): 12 ints, {lanes, threads} per class; ms (may be
  * NULL): 6 doubles, the chosen shape's time.  No counterpart in the
  * reference (whose int2e loop, src/integrals/int2e.f90:192-284, has one
  * fixed order); for callers that build many systems of one kind. */
 int myqc_eri_tune(myqc_ctx *ctx, int reps, int *shapes, double *ms);
-/* Sets the shapes myqc_eri_tune would choose (12 ints as above; a class
- * with 0 lanes keeps its shape). */
+/* Sets the shapes of later builds, whatever their size (12 ints as above; a
+ * class with 0 lanes keeps its shape, one with -1 lanes goes back to the
+ * default, lanes by its number of quartets). */
 int myqc_eri_set_shapes(myqc_ctx *ctx, const int *shapes);
 
 /* RHFI2G drop-in: G(i,j) = sum_kl D(k,l)[(ij|kl) - 1/4 (ik|jl) - 1/4 (il|jk)]

@@ -493,12 +493,15 @@ static void class_counts(myqc_ctx *ctx, int cb, int ck, double tol, std::vector<
 }
 
 // Launch shape of each quartet class in the stored build: lanes per shell
-// quartet (1, 2, 4, 8) and threads per workgroup (64, 128, 256).  Until
-// myqc_eri_tune measures the candidates on a system and keeps the fastest of
-// each class for the process (or myqc_eri_set_shapes gives one), the lanes
-// follow the class's size.
+// quartet (1, 2, 4, 8) and threads per workgroup (64, 128, 256).  The lanes
+// follow the class's size, unless myqc_eri_set_shapes gives a shape or
+// myqc_eri_tune has measured the candidates: what it kept holds for classes of
+// half to twice the quartets it was measured at, the step of lanes of the
+// rule.  (Kept for every size, the shapes tuned at 40 waters took 0.31 ms for
+// a build of one water and 0.39 for 8, against 0.25 and 0.30 by the rule.)
 struct EriShape {
     int split = 0, tpb = 256;   // split 0: by the rule
+    long long nq = 0;           // quartets it was tuned at; 0: for every size
 };
 static std::mutex g_shape_mu;
 static EriShape g_shape[6];
@@ -526,6 +529,7 @@ static EriShape class_shape(int c, long long nq, bool given) {
         std::lock_guard<std::mutex> g(g_shape_mu);
         sh = g_shape[c];
     }
+    if (sh.nq > 0 && (nq > 2 * sh.nq || 2 * nq < sh.nq)) sh = EriShape{};
     if (sh.split == 0) sh.split = rule_split(c, nq);
     return sh;
 }
@@ -787,7 +791,7 @@ int eri_store(myqc_ctx *ctx, double tol, bool want32) {
 // threads per workgroup) candidate of every class with quartets in the
 // current system is timed on the context stream (the fastest of `reps`
 // launches; each launch rewrites the same values into the store), and the
-// fastest shape of each class is kept for the process.
+// fastest shape of each class is kept for the process's builds of that size.
 static const int kSplits[4] = {1, 2, 4, 8}, kTpbs[3] = {64, 128, 256};
 
 int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
@@ -806,7 +810,7 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
         best_ms[c] = 1e300;
         for (int sp : kSplits)
             for (int tpb : kTpbs) {
-                const EriShape sh{sp, tpb};
+                const EriShape sh{sp, tpb, ctx->cls[c].nq};
                 double t = 1e300;
                 for (int r = 0; r < reps && rc == 0; ++r) {
                     float ms = 0.0f;
@@ -841,17 +845,19 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
     return 0;
 }
 
-// sets the launch shapes directly (a shape of 0 lanes keeps that class's)
+// sets the launch shapes directly, for every size of a class (a shape of 0
+// lanes keeps that class's, one of -1 goes back to the rule)
 int eri_set_shapes(myqc_ctx *ctx, const int *shape) {
     for (int c = 0; c < 6; ++c) {
         const int sp = shape[2 * c], tpb = shape[2 * c + 1];
-        if (sp == 0) continue;
+        if (sp == 0 || sp == -1) continue;
         if ((sp != 1 && sp != 2 && sp != 4 && sp != 8) || (tpb != 64 && tpb != 128 && tpb != 256))
             return set_error(ctx, MYQC_E_ARG, "myqc_eri_set_shapes: class %d: %d lanes, %d threads", c, sp, tpb);
     }
     std::lock_guard<std::mutex> g(g_shape_mu);
     for (int c = 0; c < 6; ++c)
-        if (shape[2 * c] != 0) g_shape[c] = EriShape{shape[2 * c], shape[2 * c + 1]};
+        if (shape[2 * c] == -1) g_shape[c] = EriShape{};
+        else if (shape[2 * c] != 0) g_shape[c] = EriShape{shape[2 * c], shape[2 * c + 1]};
     return 0;
 }
 

@@ -184,7 +184,7 @@ class Context:
 
     def eri_tune(self, reps: int = 2):
         """Times the ERI launch shapes on the current system and keeps the
-        fastest per class for the process; returns ({class: (lanes,
+        fastest per class for the process's builds of about that size; returns ({class: (lanes,
         threads)}, {class: ms})."""
         sh = np.zeros(12, dtype=np.int32)
         ms = np.zeros(6)
@@ -192,7 +192,8 @@ class Context:
         return {c: (int(sh[2 * c]), int(sh[2 * c + 1])) for c in range(6)}, {c: float(ms[c]) for c in range(6)}
 
     def eri_set_shapes(self, shapes):
-        """shapes: {class: (lanes, threads)} (classes left out keep theirs)."""
+        """shapes: {class: (lanes, threads)} (classes left out keep theirs;
+        -1 lanes: back to the default, lanes by the class's size)."""
         sh = np.zeros(12, dtype=np.int32)
         for c, (sp, tpb) in shapes.items():
             sh[2 * c], sh[2 * c + 1] = sp, tpb

@@ -31,3 +31,14 @@ def ctx():
     c = Context(0)
     yield c
     c.close()
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _default_shapes(request):
+    """The ERI launch shapes are the process's: a module that sets or tunes them
+    leaves the next ones the default again."""
+    gpu = any(i.get_closest_marker("gpu") for i in request.session.items if i.module is request.module)
+    c = request.getfixturevalue("ctx") if gpu else None
+    yield
+    if gpu:
+        c.eri_set_shapes({k: (-1, 256) for k in range(6)})
