@@ -82,6 +82,7 @@ struct myqc_ctx {
     // under its bra pair (the layout and schedule of digest_plan.h)
     bool have_eri = false;
     bool have_eri32 = false;
+    bool eri_by_rule = false;             // the store's values are of the launch shapes by the rule
     double eri_tol = 0.0;
     myqc::QuartetClass cls[6];
     long long n_stored = 0;               // stored values (one per unique integral slot)

@@ -20,9 +20,9 @@ struct ExpandChunk {
 
 // The values of the quartets above the Schwarz threshold `tol`, opened for
 // expansion: the context's stored integrals when they were built at that
-// threshold, else a build of its own, which leaves the context's stored
-// integrals as they are.  close() (or the destructor) gives back what the
-// open made.
+// threshold and in the rule's launch shapes (others sum in another order),
+// else a build of its own, which leaves the context's stored integrals as
+// they are.  close() (or the destructor) gives back what the open made.
 class DenseSource {
   public:
     explicit DenseSource(myqc_ctx *c) : ctx(c) {}
@@ -57,6 +57,7 @@ class DenseSource {
         long long n_stored, n_quartets;
         double eri_flops;
         int ns;
+        bool by_rule;
     } saved;
     // device tables (ctx->d_dtab)
     const long long *d_off = nullptr;

@@ -163,7 +163,7 @@ constexpr size_t kChunkBytes = kKeepWork;
 constexpr size_t kKeepStore = (size_t)2 << 30;
 
 int DenseSource::open(double tol) {
-    if (ctx->have_eri && ctx->eri_tol == tol) {
+    if (ctx->have_eri && ctx->eri_tol == tol && ctx->eri_by_rule) {
         opened = true;
         return 0;
     }
@@ -186,6 +186,7 @@ int DenseSource::open(double tol) {
         saved.n_quartets = ctx->n_quartets;
         saved.eri_flops = ctx->eri_flops;
         saved.ns = ctx->ns;
+        saved.by_rule = ctx->eri_by_rule;
         swapped = true;
     }
     opened = true;
@@ -213,6 +214,7 @@ void DenseSource::close() {
         ctx->n_quartets = saved.n_quartets;
         ctx->eri_flops = saved.eri_flops;
         ctx->ns = saved.ns;
+        ctx->eri_by_rule = saved.by_rule;
         swapped = false;
     } else if (!ctx->have_eri && dcapacity(ctx->d_x64) > kKeepStore) {
         dfree((void **)&ctx->d_x64);

@@ -551,7 +551,7 @@ static void launch_eri(myqc_ctx *ctx, const QuartetClass &qc, hipStream_t s, Eri
     a.segoff = ctx->d_segoff;
     a.x64 = ctx->d_x64;
     a.x32 = ctx->d_x32;
-        const long long nblk = (qc.nq * sh.split + sh.tpb - 1) / sh.tpb;
+    const long long nblk = (qc.nq * sh.split + sh.tpb - 1) / sh.tpb;
     switch (sh.split) {
         case 2: k_eri<CB, CK, 2><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
         case 4: k_eri<CB, CK, 4><<<(unsigned)nblk, sh.tpb, 0, s>>>(a); break;
@@ -731,7 +731,8 @@ static int ensure_side_streams(myqc_ctx *ctx) {
 // all of the stored build but the digestion schedule.  Leaves the kernels
 // in flight on the context stream.  given_shapes: the shapes tuned or set for
 // stored builds; without, the rule's alone, so that dense results do not
-// depend on what the process has tuned.
+// depend on what the process has tuned (a stored build serves them only if its
+// shapes were the rule's, DenseSource::open).
 int eri_values(myqc_ctx *ctx, double tol, bool want32, bool given_shapes) {
     HostClock hc(ctx);
     MYQC_CHECK(eri_schwarz(ctx));
@@ -754,10 +755,12 @@ int eri_values(myqc_ctx *ctx, double tol, bool want32, bool given_shapes) {
     MYQC_HIP(ctx, hipEventRecord(ctx->fork_ev, ctx->stream));
     for (int k = 0; k < 2; ++k) MYQC_HIP(ctx, hipStreamWaitEvent(ctx->side[k], ctx->fork_ev, 0));
     static const int kOrder[6] = {5, 4, 3, 2, 0, 1};
+    ctx->eri_by_rule = true;
     for (int c : kOrder) {
         if (ctx->cls[c].nq == 0) continue;
-        launch_class(ctx, c, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream,
-                     class_shape(c, ctx->cls[c].nq, given_shapes));
+        const EriShape sh = class_shape(c, ctx->cls[c].nq, given_shapes), rule = class_shape(c, ctx->cls[c].nq, false);
+        if (sh.split != rule.split || sh.tpb != rule.tpb) ctx->eri_by_rule = false;
+        launch_class(ctx, c, c >= 3 ? ctx->side[0] : c == 2 ? ctx->side[1] : ctx->stream, sh);
         MYQC_HIP(ctx, hipGetLastError());
     }
     for (int k = 0; k < 2; ++k) {
@@ -801,6 +804,7 @@ int eri_tune(myqc_ctx *ctx, int reps, int *shape_out, double *ms_out) {
     MYQC_HIP(ctx, hipEventCreate(&e0));
     MYQC_HIP(ctx, hipEventCreate(&e1));
     int rc = 0;
+    ctx->eri_by_rule = false;   // the store ends with the last candidates' values
     EriShape best[6];
     double best_ms[6];
     for (int c = 0; c < 6 && rc == 0; ++c) {
