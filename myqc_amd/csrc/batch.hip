@@ -28,6 +28,7 @@
 #include <string>
 #include <vector>
 
+#include "batch_find.h"
 #include "boys_dev.h"
 #include "context.h"
 #include "guess.h"
@@ -110,7 +111,7 @@ struct BEriArgs {
     const double *ksoa;      // primitive pairs of the ket class list (ket_soa.h)
     long long nket;          // entries of the ket class list
     const long long *qcum;   // nmol + 1 prefix counts of this class combination
-    const int *qfirst;       // the molecule of quartets 0, 64, 128, ...
+    const int *qfirst;       // the molecules of quartets 0, 64, 128, ... and of the last (quartet_marks)
     long long nq;
     double *eri;
 };
@@ -122,11 +123,9 @@ __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
     const BoysTab ft = stage_boys<M>(a.ftT, s_ft);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.nq) return;
-    // last m with qcum[m] <= t: from the wavefront's first quartet on (a search
-    // over the molecules is ten dependent loads; the six classes of
+    // (a search over all molecules is ten dependent loads; the six classes of
     // 1024 clusters 6.0 -> 5.7 ms)
-    int lo = a.qfirst[t >> 6];
-    while (a.qcum[lo + 1] <= t) ++lo;
+    const int lo = quartet_molecule(a.qcum, a.qfirst, t);
     const BMol mol = a.mols[lo];
     const long long q = t - a.qcum[lo];
     long long p, r;
@@ -1219,9 +1218,7 @@ extern "C" int myqc_batch_set(myqc_ctx *ctx, int nmol, const int *mol_nnuc, cons
             qc[m + 1] = qc[m] + (kCB[c] == kCK[c] ? tri(nb) : nb * nk);
         }
         b.nq[c] = qc[nmol];
-        qfirst[c].resize((size_t)((qc[nmol] + 63) / 64));
-        for (int m = 0; m < nmol; ++m)   // the quartets 64 k of molecule m
-            for (long long k = (qc[m] + 63) / 64; 64 * k < qc[m + 1]; ++k) qfirst[c][k] = m;
+        qfirst[c] = quartet_marks(qc);
         MYQC_CHECK(upload(ctx, &b.d_qcum[c], qc));
         MYQC_CHECK(upload(ctx, &b.d_qfirst[c], qfirst[c]));
     }

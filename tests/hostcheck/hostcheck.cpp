@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 
+#include "../../myqc_amd/csrc/batch_find.h"
 #include "../../myqc_amd/csrc/eri_math.h"
 #include "../../myqc_amd/csrc/one_e_math.h"
 #include "../../myqc_amd/csrc/system.h"
@@ -151,6 +152,29 @@ extern "C" int hc_boys(int M, int Q, double T, const double *Ftab, double *F) {
         default: return -1;
     }
     return 0;
+}
+
+// the molecule of every quartet of a batch class (batch.hip), counts[m] of them
+// in molecule m; returns the most prefix counts read for one of them
+extern "C" int hc_quartet_molecules(int nmol, const long long *counts, int *out) {
+    std::vector<long long> qcum(nmol + 1, 0);
+    for (int m = 0; m < nmol; ++m) qcum[m + 1] = qcum[m] + counts[m];
+    const std::vector<int> first = quartet_marks(qcum);
+    struct Counted {
+        const long long *p;
+        int *reads;
+        long long operator[](int m) const {
+            ++*reads;
+            return p[m];
+        }
+    };
+    int most = 0;
+    for (long long t = 0; t < qcum[nmol]; ++t) {
+        int reads = 0;
+        out[t] = quartet_molecule(Counted{qcum.data(), &reads}, first.data(), t);
+        most = reads > most ? reads : most;
+    }
+    return most;
 }
 
 // the row-owned digestion of jk.hip: for every ordered bra shell pair (A,B)
