@@ -6,8 +6,9 @@
 
 namespace myqc {
 
-// functions at most: two padded matrices in 160 KiB of LDS
-constexpr int kSmallScfN = 96;
+// functions at most: above, the general loop's launches over the whole chip are
+// no slower than one CU's matrix cores and its Jacobi (figures in scf_small.hip)
+constexpr int kSmallScfN = 84;
 
 // results of one small_step, in this order
 enum SmallOut { SO_DF = 0, SO_DH, SO_DD, SO_B, SO_OK = SO_B + 8, SO_STEPS, SO_COUNT };

@@ -19,10 +19,15 @@
 // half-wavefront's read in distinct banks.  Rows and columns beyond n are
 // zero.
 //
-// Why up to 96: above, two matrices no longer fit, and from there on a
-// purification step spread over the chip (5 to 7 us) is no slower than one
-// CU's matrix cores.  Measured, one whole solve: 1 water (n = 7) 4.04 -> 1.37 ms, 8
-// waters (n = 56) 9.1 -> 4.4 ms (112 us for a step of about 36 purifications).
+// Why up to 84: from there on a purification step spread over the chip (5 to 7
+// us) is no slower than one CU's matrix cores, and the library's eigenvectors
+// no slower than one CU's Jacobi (n = 56: 112 us for a step of about 36
+// purifications, 656 for the orbitals).  Whole solves of water clusters with
+// helium, here / by the general loop, ms, in FP64 from the core guess and mixed
+// from the learned one: n = 56 4.0 / 7.0 and 4.1 / 6.8; 70 7.6 / 10.1 and 5.6 / 6.9;
+// 80 7.5 / 8.5 and 6.3 / 7.1; 84 9.5 / 9.8 and 7.1 / 7.2 (never the slower of
+// three clusters); 86 9.3 / 9.5 and 7.3 / 7.3; 88 10.0 / 9.8 and 7.5 / 7.2; 96
+// 11.6 / 11.2 and 8.3 / 7.6.  One water (n = 7) 4.04 -> 1.37.
 #include <algorithm>
 
 #include "scf_small.h"
