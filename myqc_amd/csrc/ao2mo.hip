@@ -455,9 +455,7 @@ extern "C" int myqc_ao2mo_ovov(myqc_ctx *ctx, const double *C, int nocc, double 
     if (nocc < 1 || nocc >= ctx->n) return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov: nocc=%d", nocc);
     if (precision != MYQC_FP64 && precision != MYQC_BF16X3)
         return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov: precision %d", precision);
-    const size_t n = ctx->n;
-    if (n * n * n * n * 8 > (size_t)200 << 30)
-        return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov: n=%zu needs more than 200 GB of dense AO integrals", n);
+    MYQC_CHECK(transform_fits(ctx, "myqc_ao2mo_ovov"));
     MYQC_CHECK(ao2mo(ctx, C, nocc, precision));
     if (iajb) {
         const int d[4] = {nocc, ctx->n - nocc, nocc, ctx->n - nocc};
@@ -529,9 +527,7 @@ extern "C" int myqc_ao2mo_ovov_uhf(myqc_ctx *ctx, const double *Ca, const double
         return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov_uhf: nalpha=%d nbeta=%d", nalpha, nbeta);
     if (precision != MYQC_FP64 && precision != MYQC_BF16X3)
         return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov_uhf: precision %d", precision);
-    const size_t n = ctx->n;
-    if (n * n * n * n * 8 > (size_t)200 << 30)
-        return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_ovov_uhf: n=%zu needs more than 200 GB of dense AO integrals", n);
+    MYQC_CHECK(transform_fits(ctx, "myqc_ao2mo_ovov_uhf"));
     MYQC_CHECK(ao2mo_uhf(ctx, Ca, Cb, nalpha, nbeta, precision, false));
     if (ijab_aa) MYQC_CHECK(download_records(ctx, ctx->d_uhf[0], ctx->uhf_dims[0], 1, ijab_aa));
     if (ijab_bb) MYQC_CHECK(download_records(ctx, ctx->d_uhf[1], ctx->uhf_dims[1], 1, ijab_bb));

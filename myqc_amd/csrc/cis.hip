@@ -18,7 +18,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "context.h"
+#include "dense.h"
 
 namespace myqc {
 
@@ -145,9 +145,7 @@ extern "C" int myqc_ao2mo_cis_uhf(myqc_ctx *ctx, const double *Ca, const double 
     if (!ctx->have_system) return set_error(ctx, MYQC_E_STATE, "myqc_ao2mo_cis_uhf: no system set");
     if (nalpha < 0 || nalpha > ctx->n || nbeta < 0 || nbeta > ctx->n)
         return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_cis_uhf: nalpha=%d nbeta=%d", nalpha, nbeta);
-    const size_t n = ctx->n;
-    if (n * n * n * n * 8 > (size_t)200 << 30)
-        return set_error(ctx, MYQC_E_ARG, "myqc_ao2mo_cis_uhf: n=%zu needs more than 200 GB of dense AO integrals", n);
+    MYQC_CHECK(transform_fits(ctx, "myqc_ao2mo_cis_uhf"));
     MYQC_CHECK(ao2mo_uhf(ctx, Ca, Cb, nalpha, nbeta, MYQC_FP64, true));
     double *outs[5] = {ajib_aa, ajbi_aa, ajib_ab, ajib_bb, ajbi_bb};
     const CisDims d{nalpha, ctx->n - nalpha, nbeta, ctx->n - nbeta};

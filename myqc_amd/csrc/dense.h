@@ -66,6 +66,15 @@ class DenseSource {
     int nrec = 0, pos[4] = {0, 0, 0, 0}, inv0[3] = {0, 0, 0};
 };
 
+// The transforms' limit: what quarter steps 1 and 2 leave is at most 8 n^3 nvirt
+// bytes (both spins' virtual pairs, l >= d), here 200 GB beside the store's n^4.
+inline int transform_fits(myqc_ctx *ctx, const char *who) {
+    const size_t n = ctx->n;
+    if (n * n * n * n * 8 > (size_t)200 << 30)
+        return set_error(ctx, MYQC_E_ARG, "%s: n=%zu: the transforms take up to 404 functions", who, n);
+    return 0;
+}
+
 // One product of quarter steps 1 and 2: M(p, q, l d) from the orbital blocks
 // Cp (n x np) and Cq (n x nq), both with leading dimension n.
 struct TransformJob {
