@@ -38,12 +38,13 @@ class DenseSource {
     const int *d_tri = nullptr;
     int expand(const ExpandChunk &c, double *X);
     size_t chunk_bytes() const;
-    // all blocks at their places in the dense n^4 array
-    int expand_full(double *XX);
+    // the blocks of second index d0 .. d1 - 1 of the dense n^4 array, in their
+    // order, to XX (n^3 (d1 - d0) values)
+    int expand_full(double *XX, int d0, int d1);
 
   private:
-    int tables(bool full);
-    int launch(const ExpandChunk &c, double *X, int full);
+    int tables(int d0, int d1);
+    int launch(const ExpandChunk &c, double *X, int d0, int d1);
     myqc_ctx *ctx;
     bool opened = false, swapped = false;
     // the context's own store, put aside while another is open

@@ -25,7 +25,8 @@ struct ExpandArgs {
     int n, nrec;
     int pos[4];                // first position of each class, and the end
     int inv0[3];               // first entry of inv of each class
-    int full;                  // blocks at l + n d and d + n l
+    int d0, d1;                // blocks (l, d) and (d, l) at l + n (d - d0) and d + n (l - d0) as far as the second
+                               // index is within [d0, d1); d1 = 0: the record's block alone, at rec.blk
     int m[kExpParts + 1];      // the ranges of u (blockIdx.y)
 };
 
@@ -141,13 +142,18 @@ __global__ __launch_bounds__(THREADS) void k_expand(ExpandArgs a) {
     }
     __syncthreads();
     // the square: a wavefront per column v, rows u with max(u, v) in [m0, m1)
-    double *X = a.X + (size_t)n * n * rec->blk;
-    double *X2 = a.full && l != d ? a.X + (size_t)n * n * ((size_t)d + (size_t)n * l) : nullptr;
+    const size_t nn = (size_t)n * n;
+    double *X = nullptr, *X2 = nullptr;
+    if (a.d1 == 0) X = a.X + nn * rec->blk;
+    else {
+        if (d >= a.d0 && d < a.d1) X = a.X + nn * (l + (size_t)n * (d - a.d0));
+        if (l != d && l >= a.d0 && l < a.d1) X2 = a.X + nn * (d + (size_t)n * (l - a.d0));
+    }
     for (int v = t >> 6; v < m1; v += THREADS / 64)
         for (int u = (v < m0 ? m0 : 0) + (t & 63); u < m1; u += 64) {
             const int hi = max(u, v), lo = min(u, v);
             const double x = s_b[hi * (hi + 1) / 2 + lo - t0];
-            X[u + (size_t)n * v] = x;
+            if (X) X[u + (size_t)n * v] = x;
             if (X2) X2[u + (size_t)n * v] = x;
         }
 }
@@ -221,8 +227,9 @@ void DenseSource::close() {
     }
 }
 
-// The tables and records, in one upload to ctx->d_dtab.
-int DenseSource::tables(bool full) {
+// The tables and records, in one upload to ctx->d_dtab: chunks of all blocks
+// (d1 = 0), or the records of the blocks with an index within [d0, d1).
+int DenseSource::tables(int d0, int d1) {
     const DigestPlan &pl = ctx->plan;
     const int n = ctx->n, np = (int)ctx->pairs.size();
     pos[0] = inv0[0] = 0;
@@ -260,7 +267,7 @@ int DenseSource::tables(bool full) {
                 const int l = std::max(i, j), d = std::min(i, j), at = l * (l + 1) / 2 + d;
                 const bool kept = !(sp.same && x > y);
                 inv[inv0[c] + r * nf + e] = kept ? 2 * at + (l == d) : -1;
-                if (!kept) continue;
+                if (!kept || (d1 > 0 && (d < d0 || d >= d1) && (l < d0 || l >= d1))) continue;
                 recs.push_back(ExpandRec{pos[c] + (int)r, e, l, d, 0});
                 tri.push_back(at);
             }
@@ -268,11 +275,11 @@ int DenseSource::tables(bool full) {
     nrec = (int)recs.size();
     // chunks of whole rounds of a workgroup per CU
     const size_t nn8 = sizeof(double) * (size_t)n * n;
-    int most = full ? nrec : (int)std::min<size_t>(nrec, std::max<size_t>(1, kChunkBytes / nn8));
+    int most = d1 > 0 ? nrec : (int)std::min<size_t>(nrec, std::max<size_t>(1, kChunkBytes / nn8));
     if (most > 256 && most < nrec) most -= most % 256;
     chunks.clear();
     for (int r = 0; r < nrec; r += most) chunks.push_back(ExpandChunk{r, std::min(most, nrec - r)});
-    for (int r = 0; r < nrec; ++r) recs[r].blk = full ? recs[r].l + n * recs[r].d : r % most;
+    for (int r = 0; r < nrec; ++r) recs[r].blk = r % most;
     const size_t b_off = sizeof(long long) * off.size(), b_range = sizeof(int) * range.size(),
                  b_rec = sizeof(ExpandRec) * recs.size(), b_inv = sizeof(int) * inv.size(),
                  b_tri = sizeof(int) * tri.size();
@@ -299,16 +306,16 @@ int DenseSource::tables(bool full) {
     return 0;
 }
 
-int DenseSource::plan_chunks() { return tables(false); }
+int DenseSource::plan_chunks() { return tables(0, 0); }
 
 size_t DenseSource::chunk_bytes() const {
     return chunks.empty() ? 0 : sizeof(double) * (size_t)ctx->n * ctx->n * chunks[0].nblk;
 }
 
-int DenseSource::launch(const ExpandChunk &c, double *X, int full) {
+int DenseSource::launch(const ExpandChunk &c, double *X, int d0, int d1) {
     const int n = ctx->n;
     ExpandArgs a{ctx->d_x64, d_inv, d_off, d_range, d_rec + c.blk0, X, n, c.nblk, {pos[0], pos[1], pos[2], pos[3]},
-                 {inv0[0], inv0[1], inv0[2]}, full, {}};
+                 {inv0[0], inv0[1], inv0[2]}, d0, d1, {}};
     const unsigned grid = (unsigned)((c.nblk + 255) / 256 * 256);
     constexpr int kSmall = 2048, kLarge = 16384, kLT = 1024;
     const int tri = n * (n + 1) / 2;
@@ -333,11 +340,11 @@ int DenseSource::launch(const ExpandChunk &c, double *X, int full) {
     return 0;
 }
 
-int DenseSource::expand(const ExpandChunk &c, double *X) { return launch(c, X, 0); }
+int DenseSource::expand(const ExpandChunk &c, double *X) { return launch(c, X, 0, 0); }
 
-int DenseSource::expand_full(double *XX) {
-    MYQC_CHECK(tables(true));
-    return launch(ExpandChunk{0, nrec}, XX, 1);
+int DenseSource::expand_full(double *XX, int d0, int d1) {
+    MYQC_CHECK(tables(d0, d1));
+    return launch(ExpandChunk{0, nrec}, XX, d0, d1);
 }
 
 }  // namespace myqc

@@ -929,23 +929,23 @@ extern "C" int myqc_set_system(myqc_ctx *ctx, int nnuc, const int *Z, const doub
 extern "C" int myqc_eri_full(myqc_ctx *ctx, double schwarz_tol, double *XX) {
     if (!ctx || !XX) return MYQC_E_ARG;
     if (!ctx->have_system) return set_error(ctx, MYQC_E_STATE, "myqc_eri_full: no system set");
-    const size_t n = ctx->n, n4 = n * n * n * n, bytes = sizeof(double) * n4;
-    // the context's work buffer, unless the array is too large to keep
-    double *own = nullptr, *&d_XX = bytes <= kKeepWork ? ctx->d_xwork : own;
-    MYQC_CHECK(dalloc(ctx, (void **)&d_XX, bytes));
-    int rc = 0;
-    {
-        DenseSource src(ctx);
-        rc = src.open(schwarz_tol);
-        if (rc == 0) rc = src.expand_full(d_XX);
-        if (rc == 0) {
-            hipError_t e = d2h(ctx, XX, d_XX, bytes);
-            if (e != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "myqc_eri_full: copy failed: %s", hipGetErrorString(e));
-        } else {
-            (void)hipStreamSynchronize(ctx->stream);   // nothing in flight when the store is given back
-        }
+    // through the context's work buffer, a slab of the last index at a time where
+    // the array is too large to keep: beside the stored integrals (an eighth of
+    // it) the device need not hold the array
+    const size_t n = ctx->n, n3 = n * n * n, col = sizeof(double) * n3;
+    const int per = (int)std::min(n, std::max<size_t>(1, kKeepWork / col));
+    DenseSource src(ctx);
+    int rc = dalloc(ctx, (void **)&ctx->d_xwork, col * per);
+    if (rc == 0) rc = src.open(schwarz_tol);
+    for (int d0 = 0; d0 < ctx->n && rc == 0; d0 += per) {
+        const int d1 = std::min(ctx->n, d0 + per);
+        rc = src.expand_full(ctx->d_xwork, d0, d1);
+        if (rc) break;
+        const hipError_t e = d2h(ctx, XX + n3 * d0, ctx->d_xwork, col * (d1 - d0));
+        if (e != hipSuccess) rc = set_error(ctx, MYQC_E_HIP, "myqc_eri_full: copy failed: %s", hipGetErrorString(e));
     }
-    dfree((void **)&own);
+    if (rc) (void)hipStreamSynchronize(ctx->stream);   // nothing in flight when the store is given back
+    if (dcapacity(ctx->d_xwork) > kKeepWork) dfree((void **)&ctx->d_xwork);
     return rc;
 }
 
