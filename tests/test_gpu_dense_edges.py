@@ -1,5 +1,6 @@
 """Dense integrals at the sizes where their expansion changes form
-(csrc/dense.hip): the dense array in one piece (n <= 80) or in slabs.
+(csrc/dense.hip): a block in 16 KiB of LDS (n <= 63), in 128 KiB (n <= 180), in
+several ranges of u above; the dense array in one piece (n <= 80) or in slabs.
 
 An integral depends on its own shells alone, so those of a few of the atoms are
 compared with the CPU oracle's for these atoms.  Tolerance: the parity bound of
@@ -35,7 +36,7 @@ def _some_atoms(Z, xyz, first, atoms):
     return f, O.eri_full(O.System(z, x, build_basis(z), FT))
 
 
-@pytest.mark.parametrize("n", [80, 81, 98])
+@pytest.mark.parametrize("n", [62, 63, 64, 80, 81, 98])
 def test_dense_array_at_size_edges(ctx, n):
     Z, xyz, first = _system(ctx, n)
     print(f"[dense] n = {n}", flush=True)
@@ -46,3 +47,17 @@ def test_dense_array_at_size_edges(ctx, n):
     for atoms in ([0, 1, last], [0, 3, last - 1], [last - 2, 12, 5]):
         f, want = _some_atoms(Z, xyz, first, atoms)
         assert np.max(np.abs(XX[np.ix_(f, f, f, f)] - want)) <= 1e-10
+
+
+@pytest.mark.parametrize("n", [62, 63, 64, 180, 181])
+def test_transform_blocks_at_size_edges(ctx, n):
+    """(ia|jb) over orbitals that are single functions"""
+    Z, xyz, first = _system(ctx, n)
+    print(f"[blocks] n = {n}", flush=True)
+    atoms = [0, 1, 36 if n > 100 else 12, len(Z) - 1]
+    f, want = _some_atoms(Z, xyz, first, atoms)
+    o = 5                                     # occupied: the functions of the first atom
+    perm = np.concatenate([f, np.setdiff1d(np.arange(n), f)])
+    t = ctx.ao2mo(np.eye(n)[:, perm], o)      # no build stored: unscreened integrals
+    m = len(f)
+    assert np.max(np.abs(t[:, :m - o, :, :m - o] - want[:o, o:m, :o, o:m])) <= 1e-10
