@@ -166,9 +166,12 @@ __device__ __forceinline__ void find_quartet(const long long *__restrict__ cum, 
 
 // SPLIT lanes per shell quartet: they share its primitive quartets, add their
 // sums (group_sum), and each stores every SPLIT-th element of the block.
-// Waves per SIMD asked of the register allocator per class (the staged
-// tables' 39 to 41 KB of LDS allow four 256-thread workgroups per CU): ss|ss 6,
-// ps|ss 5, ps|ps and pp|ss 4, the rest unconstrained.
+// Waves per SIMD asked of the register allocator per class: the staged tables'
+// 39 to 41 KB of LDS allow four 256-thread workgroups per CU, so four at most
+// (the compiler drops a request that LDS cannot meet): ps|ps and pp|ss 4, the
+// rest unconstrained.  ss|ss then has 92 registers and four waves, ps|ss 137 and
+// three; ps|ss held to four spills (52 B of scratch): the class in 0.55 instead
+// of 0.62 ms at 40 waters, but 54 instead of 51 us at 13.
 //
 // Bounded by FP64 VALU issue (70 to 80 % of it): about 90 instructions per
 // primitive quartet of ss|ss, 30 of the 81 surviving the screen.  40 waters,
@@ -177,7 +180,7 @@ __device__ __forceinline__ void find_quartet(const long long *__restrict__ cum, 
 // (eri_math.h), 1.90 with F_M tabulated, 1.78 with one transcendental less, K/p
 // and fewer conversions.  512 threads (eight waves per SIMD on the same
 // staged tables): 1.79, and small systems 30 % slower.
-constexpr int eri_waves(int cb, int ck) { return cb + ck == 0 ? 6 : cb + ck == 1 ? 5 : cb + ck == 2 ? 4 : 1; }
+constexpr int eri_waves(int cb, int ck) { return cb + ck == 2 ? 4 : 1; }
 template <int CB, int CK, int SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(eri_waves(CB, CK)))) void k_eri(EriArgs a) {
     constexpr int M = CB + CK;
