@@ -123,8 +123,8 @@ __global__ __launch_bounds__(256) void k_batch_eri(BEriArgs a) {
     const BoysTab ft = stage_boys<M>(a.ftT, s_ft);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.nq) return;
-    // (a search over all molecules is ten dependent loads; the six classes of
-    // 1024 clusters 6.0 -> 5.7 ms)
+    // (a search over all molecules is ten dependent loads: 5 % of the six
+    // classes' time for 1024 clusters)
     const int lo = quartet_molecule(a.qcum, a.qfirst, t);
     const BMol mol = a.mols[lo];
     const long long q = t - a.qcum[lo];
@@ -175,7 +175,7 @@ struct BScfArgs {
     int nmol;
     int *counter;              // work queue head (zeroed before the launch)
     const double *eri, *S, *H, *guess;   // guess: NULL or n^2 blocks
-    double *scratch;           // 4 n^2 blocks per molecule: X, F', Dp, W
+    double *scratch;           // 4 n^2 blocks per molecule: X, the projector, F', a density
     double *hist;              // 2 kBatchDiis n^2 blocks per molecule
     double *Dout;
     double *energy;
@@ -783,7 +783,7 @@ __device__ __forceinline__ void batch_solve(const BScfArgs &a, const BMol &mol, 
 
 // Registers bound the residency (256 VGPRs: two wavefronts per SIMD; at 128 the
 // Fock rows spill and a build takes twice as long).  1024 clusters of 2 to 5
-// waters: 16 ms -> 5.0 ms; of an iteration's 218 us at 35 functions (eight
+// waters: 17 ms -> 6.3 ms; of an iteration's 218 us at 35 functions (eight
 // wavefronts) 123 are the Fock build, 51 the 30 purification steps, 10 X F X, 21
 // the DIIS error, its dots and the extrapolation.  The two Jacobi
 // diagonalisations of a molecule's start, 870 us, are 81 us of Newton-Schulz and

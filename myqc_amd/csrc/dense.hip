@@ -14,7 +14,9 @@
 
 namespace myqc {
 
-constexpr int kExpParts = 64;   // ranges of u at most (n <= 1500)
+// values of a block in LDS: small blocks, and a range of u of large ones
+constexpr int kExpSmall = 2048, kExpLarge = 16384;
+constexpr int kExpParts = 64;   // ranges of u at most (n <= 1425: a range ends with a whole row)
 struct ExpandArgs {
     const double *x;
     const int *inv;            // per class-sorted pair and element: 2 (u (u + 1) / 2 + v) + (u == v), -1: not kept
@@ -317,24 +319,24 @@ int DenseSource::launch(const ExpandChunk &c, double *X, int d0, int d1) {
     ExpandArgs a{ctx->d_x64, d_inv, d_off, d_range, d_rec + c.blk0, X, n, c.nblk, {pos[0], pos[1], pos[2], pos[3]},
                  {inv0[0], inv0[1], inv0[2]}, d0, d1, {}};
     const unsigned grid = (unsigned)((c.nblk + 255) / 256 * 256);
-    constexpr int kSmall = 2048, kLarge = 16384, kLT = 1024;
+    constexpr int kLT = 1024;
     const int tri = n * (n + 1) / 2;
-    if (tri <= kSmall) {
+    if (tri <= kExpSmall) {
         a.m[1] = n;
-        k_expand<kSmall, 256><<<grid, 256, 0, ctx->stream>>>(a);
+        k_expand<kExpSmall, 256><<<grid, 256, 0, ctx->stream>>>(a);
     } else {
         // ranges of u of about equal size
         int parts = 0, m = 0;
-        const int want = (tri + kLarge - 1) / kLarge;
+        const int want = (tri + kExpLarge - 1) / kExpLarge;
         for (; m < n && parts < kExpParts; ++parts) {
             const int t0 = m * (m + 1) / 2;
-            const long long goal = std::min<long long>((long long)tri * (parts + 1) / want, (long long)t0 + kLarge);
+            const long long goal = std::min<long long>((long long)tri * (parts + 1) / want, (long long)t0 + kExpLarge);
             while (m < n && (long long)(m + 1) * (m + 2) / 2 <= goal) ++m;
             a.m[parts + 1] = m;
             if (m * (m + 1) / 2 == t0) return set_error(ctx, MYQC_E_ARG, "dense integrals: n=%d too large", n);
         }
         if (m < n) return set_error(ctx, MYQC_E_ARG, "dense integrals: n=%d too large", n);
-        k_expand<kLarge, kLT><<<dim3(grid, (unsigned)parts), kLT, 0, ctx->stream>>>(a);
+        k_expand<kExpLarge, kLT><<<dim3(grid, (unsigned)parts), kLT, 0, ctx->stream>>>(a);
     }
     MYQC_HIP(ctx, hipGetLastError());
     return 0;

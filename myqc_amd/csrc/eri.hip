@@ -173,7 +173,7 @@ __device__ __forceinline__ void find_quartet(const long long *__restrict__ cum, 
 // three; ps|ss held to four spills (52 B of scratch): the class in 0.55 instead
 // of 0.62 ms at 40 waters, but 54 instead of 51 us at 13.
 //
-// Bounded by FP64 VALU issue (70 to 80 % of it): about 90 instructions per
+// Bounded by FP64 VALU issue (70 % of it in ss|ss, 64 in ps|ss): about 90 instructions per
 // primitive quartet of ss|ss, 30 of the 81 surviving the screen.  40 waters,
 // the six classes together: 2.33 ms with every primitive pair tested and the
 // reference's downward recursion from F_Q, 2.00 with rows cut at the screen
@@ -583,7 +583,7 @@ static void launch_class(myqc_ctx *ctx, int c, hipStream_t s, EriShape sh) {
 // count.  They include lanes that sit idle while a neighbour computes a
 // primitive quartet that its own pair screen drops, and both sides of a
 // divergent Boys branch, so they count issued rather than strictly useful work.
-static const double kQuartetFlops[6] = {2319.9, 2920.7, 4588.6, 4724.8, 9633.6, 31778.1};
+static const double kQuartetFlops[6] = {2297.3, 2893.7, 4533.7, 4648.9, 9444.8, 30695.8};
 
 static int build_classes(myqc_ctx *ctx, double tol) {
     std::vector<long long> cum;

@@ -40,8 +40,10 @@ constexpr int FT_NM = 19;    // m  = 0..18 of the record's 23: the largest order
 // polynomial in x = Tk/10 - T times known functions, so its value F_M is
 // tabulated instead, per (M, Q / 3, Tk), as a polynomial of degree 6 (7 for
 // M >= 2, the last coefficient in a float) in x, |x| <= 0.05: the series to
-// degree 9, telescoped.  Against the procedure in 80 bits its largest error is
-// 0.6 to 1.1e-15 relative, the recursion's in doubles 1.0 to 1.5e-15.
+// degree 9, telescoped.  Against the procedure in 80 bits (400,000 T below 12 for
+// each M and Q, all orders) the largest relative error grows with Q: 1.1e-16 for
+// Q = 0, at most 1.4, 1.4, 1.8 and 2.2e-15 for 3, 6, 9 and 12; the recursion in
+// doubles had 1.4e-16, 1.4, 2.0, 2.6 and 3.1e-15, and was in no row better.
 //
 // One block of FT_BLOCK per M = 0..4: FT_POLY coefficients ([Q / 3][Tk][power];
 // seven, an odd stride, spread a wavefront's rows over the LDS banks), then the
@@ -75,8 +77,9 @@ __host__ __device__ __forceinline__ BoysTab boys_tab(const BoysTab &t) {
     return t;
 }
 // staged for a kernel: polynomials, e and g, and the degree-7 floats for M >= 2
-// (with these 40752 B, four workgroups per CU)
+// (four workgroups per CU)
 constexpr int ft_staged(int M) { return FT_POLY + FT_EGN + (M >= 2 ? FT_TOP : 0); }
+static_assert(4 * sizeof(double) * ft_staged(4) <= 160 * 1024, "LDS of four workgroups");
 
 // Cartesian components up to l = 2: 0 s | 1 x 2 y 3 z | 4 xx 5 xy 6 xz 7 yy 8 yz 9 zz
 MYQC_HD constexpr int cexp(int idx, int d) {

@@ -420,8 +420,8 @@ __global__ __launch_bounds__(256) void k_gather_jk(const PT *__restrict__ jk_par
 // A(i, j) = the sum of the partial rows holding AO i, plus the ket-side J of
 // the pair (shell(i), shell(j)) when it is stored in that orientation.  One
 // workgroup per (AO, 64 columns); its four thread rows take every fourth
-// partial row (twelve loads in flight each, as many as 40 waters' AOs have) and
-// meet in LDS in a fixed order.  Two at a time took 18 us at 40 waters, now 13.4.
+// partial row (twelve loads in flight each, a choice: one round for most AOs of 40
+// waters) and meet in LDS in a fixed order.  Two at a time took 18 us at 40 waters, now 13.4.
 template <typename PT>
 __global__ __launch_bounds__(256) void k_gather_rows(const PT *__restrict__ partial,
                                                      const int *__restrict__ list_off, const int *__restrict__ list,
