@@ -144,18 +144,19 @@ __global__ __launch_bounds__(THREADS) void k_expand(ExpandArgs a) {
     }
     __syncthreads();
     // the square: a wavefront per column v, rows u with max(u, v) in [m0, m1)
-    const size_t nn = (size_t)n * n;
-    double *X = nullptr, *X2 = nullptr;
-    if (a.d1 == 0) X = a.X + nn * rec->blk;
-    else {
-        if (d >= a.d0 && d < a.d1) X = a.X + nn * (l + (size_t)n * (d - a.d0));
-        if (l != d && l >= a.d0 && l < a.d1) X2 = a.X + nn * (d + (size_t)n * (l - a.d0));
+    double *X = a.X + (size_t)n * n * rec->blk, *X2 = nullptr;
+    if (a.d1 > 0) {
+        // (one of them at least is within the slab)
+        const bool in = d >= a.d0 && d < a.d1, in2 = l >= a.d0 && l < a.d1;
+        double *Y = a.X + (size_t)n * n * (d + (size_t)n * (l - a.d0));
+        X = in ? a.X + (size_t)n * n * (l + (size_t)n * (d - a.d0)) : Y;
+        if (in && in2 && l != d) X2 = Y;
     }
     for (int v = t >> 6; v < m1; v += THREADS / 64)
         for (int u = (v < m0 ? m0 : 0) + (t & 63); u < m1; u += 64) {
             const int hi = max(u, v), lo = min(u, v);
             const double x = s_b[hi * (hi + 1) / 2 + lo - t0];
-            if (X) X[u + (size_t)n * v] = x;
+            X[u + (size_t)n * v] = x;
             if (X2) X2[u + (size_t)n * v] = x;
         }
 }
