@@ -273,9 +273,11 @@ __global__ __launch_bounds__(Sm<NP>::THREADS) void k_small_orbitals(int n, const
     if (t < n) {
         const double v = sA[t * (LD + 1)];
         int at = 0;
+        // (not a number: after every number, so that each still has its own place)
+        auto before = [](double x, double y) { return x < y || (x == x && y != y); };
         for (int j = 0; j < n; ++j) {
             const double u = sA[j * (LD + 1)];
-            at += u < v || (u == v && j < t);
+            at += before(u, v) || (!before(v, u) && j < t);
         }
         s_at[t] = at;
         eig[at] = v;
